@@ -73,8 +73,8 @@ int wotk_abi_version(void);
  * compute ||x - m||^2 + ||y - m||^2 - 2 (x - m).(y - m) (m = mean of both
  * days) with the cross term as a 3- or 6-term split-BF16 MFMA GEMM
  * accumulated in FP32 (x = hi + mid + lo in BF16; 3 terms hi.hi + hi.mid +
- * mid.hi, 6 terms add hi.lo + lo.hi + mid.mid).  The median is exact (radix select over the FP64
- * bit patterns; even count -> mean of the two middle values, numpy.median).
+ * mid.hi, 6 terms add hi.lo + lo.hi + mid.mid).  The median is exact (an order
+ * statistic of the FP64 bit patterns; even count -> mean of the two middle values, numpy.median).
  * Layout every sweep over C / CT assumes: ldc and ldct multiples of 4, and
  * columns J .. round_up(J, 4) - 1 of every row of C (I .. round_up(I, 4) - 1
  * of CT) holding finite values -- the sweeps read whole 16-byte groups.  This

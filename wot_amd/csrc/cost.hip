@@ -1,71 +1,12 @@
 // Cost matrix for wot's OT path: C = sqeuclid(X, Y) / median(C)
-// (wot/ot/ot_model.py:242-253).  FP64 direct-difference tiles, an exact
-// radix-select median over the FP64 bit patterns, and a normalise+transpose
-// pass that writes the FP32 pair (C, C^T) the Sinkhorn sweeps stream.
+// (wot/ot/ot_model.py:242-253).  The distances and their median are
+// regenerated tile by tile (distance.hip) and written once as the FP32 pair
+// (C, C^T) the Sinkhorn sweeps stream.  Here: the entry points, the radix-select
+// median of stored values, and the normalise+transpose pass of a given cost.
 #include "common.h"
+#include "distance.h"
 
 namespace wotk {
-
-// ---------------------------------------------------------------------------
-// FP64 direct difference: C_ij = sum_k (x_ik - y_jk)^2, 64x64 output tile per
-// 256-thread block, 4x4 outputs per thread, coordinates staged through LDS in
-// 32-wide k chunks (transposed so a thread's 4 rows are contiguous).
-// ---------------------------------------------------------------------------
-constexpr int kCostTile = 64;
-constexpr int kCostKc = 32;
-
-__global__ __launch_bounds__(256) void sqeuclid_f64_kernel(const double *__restrict__ X,
-                                                           const double *__restrict__ Y, int n_i,
-                                                           int n_j, int d, double *__restrict__ C,
-                                                           int64_t ldc) {
-    __shared__ double xs[kCostKc][kCostTile];
-    __shared__ double ys[kCostKc][kCostTile];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const int i0 = blockIdx.y * kCostTile, j0 = blockIdx.x * kCostTile;
-    double acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-
-    for (int k0 = 0; k0 < d; k0 += kCostKc) {
-        for (int e = tid; e < kCostTile * kCostKc; e += 256) {
-            const int r = e / kCostKc, kk = e % kCostKc;
-            const bool kin = (k0 + kk) < d;
-            xs[kk][r] = (kin && i0 + r < n_i) ? X[(int64_t)(i0 + r) * d + k0 + kk] : 0.0;
-            ys[kk][r] = (kin && j0 + r < n_j) ? Y[(int64_t)(j0 + r) * d + k0 + kk] : 0.0;
-        }
-        __syncthreads();
-        const int kmax = min(kCostKc, d - k0);
-        for (int kk = 0; kk < kmax; ++kk) {
-            double xv[4], yv[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                xv[q] = xs[kk][ty * 4 + q];
-                yv[q] = ys[kk][tx * 4 + q];
-            }
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const double t = xv[a] - yv[b];
-                    acc[a][b] = fma(t, t, acc[a][b]);
-                }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int i = i0 + ty * 4 + a;
-        if (i >= n_i) continue;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int j = j0 + tx * 4 + b;
-            if (j < n_j) C[(int64_t)i * ldc + j] = acc[a][b];
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Exact order statistics by MSB-first radix select on the bit patterns of
@@ -245,25 +186,21 @@ static int median_run(const double *values, int64_t n, double *out, int64_t *ind
 }
 
 // ---------------------------------------------------------------------------
-// FP64 (I x J) -> FP32 C (I x J) and C^T (J x I), each entry value/divisor
-// (divisor read from the device, e.g. the median) or value*scale.  Padding
+// FP64 (I x J) -> FP32 C (I x J) and C^T (J x I), each entry value*scale.  Padding
 // columns up to the next multiple of 4 are written as 0 so the float4 sweeps
 // read finite values there.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void normalise_transpose_kernel(
-    const double *__restrict__ C64, int64_t ld64, int n_i, int n_j, const double *__restrict__ divisor,
-    double scale, float *__restrict__ C, int64_t ldc, float *__restrict__ CT, int64_t ldct) {
+    const double *__restrict__ C64, int64_t ld64, int n_i, int n_j, double scale, float *__restrict__ C, int64_t ldc, float *__restrict__ CT, int64_t ldct) {
     __shared__ float tile[64][65];
     const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
-    const double dv = divisor ? *divisor : 0.0;
     const int pad_j = (n_j + 3) & ~3, pad_i = (n_i + 3) & ~3;
     for (int r = ty; r < 64; r += 4) {
         const int i = i0 + r, j = j0 + tx;
         float v = 0.f;
         if (i < n_i && j < n_j) {
-            const double c = C64[(int64_t)i * ld64 + j];
-            v = (float)(divisor ? c / dv : c * scale);
+            v = (float)(C64[(int64_t)i * ld64 + j] * scale);
         }
         tile[r][tx] = v;
         if (i < n_i && j < pad_j) C[(int64_t)i * ldc + j] = v;
@@ -275,27 +212,13 @@ __global__ __launch_bounds__(256) void normalise_transpose_kernel(
     }
 }
 
-int launch_normalise_transpose(const double *C64, int64_t ld64, int64_t I, int64_t J,
-                               const double *divisor, double scale, float *C, int64_t ldc,
-                               float *CT, int64_t ldct, hipStream_t s) {
+static int launch_normalise_transpose(const double *C64, int64_t ld64, int64_t I, int64_t J, double scale, float *C,
+                                      int64_t ldc, float *CT, int64_t ldct, hipStream_t s) {
     dim3 grid((unsigned)((round_up(J, 4) + 63) / 64), (unsigned)((round_up(I, 4) + 63) / 64));
-    normalise_transpose_kernel<<<grid, 256, 0, s>>>(C64, ld64, (int)I, (int)J, divisor, scale, C,
-                                                    ldc, CT, ldct);
+    normalise_transpose_kernel<<<grid, 256, 0, s>>>(C64, ld64, (int)I, (int)J, scale, C, ldc, CT, ldct);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
 }
-
-int launch_sqeuclid_f64(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
-                        double *C64, int64_t ld, hipStream_t s) {
-    dim3 grid((unsigned)((J + kCostTile - 1) / kCostTile), (unsigned)((I + kCostTile - 1) / kCostTile));
-    sqeuclid_f64_kernel<<<grid, 256, 0, s>>>(X, Y, (int)I, (int)J, (int)d, C64, ld);
-    WOTK_LAUNCH_CHECK();
-    return WOTK_OK;
-}
-
-int launch_cost_bf16(const double *X, const double *Y, int64_t I, int64_t J, int64_t d, int terms,
-                     double *C64, int64_t ld, void *scratch, hipStream_t s);
-size_t cost_bf16_scratch(int64_t I, int64_t J, int64_t d);
 
 static int check_cost_layout(int64_t I, int64_t J, int64_t d, const float *C, int64_t ldc,
                              const float *CT, int64_t ldct) {
@@ -332,10 +255,7 @@ extern "C" int wotk_median_f64(const double *values, int64_t n, double *median_o
 
 extern "C" size_t wotk_cost_workspace_size(int64_t I, int64_t J, int64_t d, int32_t mode) {
     Arena ar(nullptr, 0);
-    ar.take<double>((size_t)I * J);
-    SelectState *st;
-    unsigned long long *h;
-    median_ws(ar, I * J, &st, &h);
+    ar.take<char>(distance_median_bytes(I, J, false));
     if (mode == WOTK_COST_BF16X3 || mode == WOTK_COST_BF16X6) ar.take<char>(cost_bf16_scratch(I, J, d));
     return ar.off;
 }
@@ -357,22 +277,20 @@ extern "C" int wotk_cost_sqeuclid(const double *X, const double *Y, int64_t I, i
                  "unknown cost mode %d", mode);
     hipStream_t s = (hipStream_t)stream;
     Arena ar(workspace, workspace_bytes);
-    double *C64 = ar.take<double>((size_t)I * J);
-    SelectState *st;
-    unsigned long long *h;
-    median_ws(ar, I * J, &st, &h);
+    void *med_ws = ar.take<char>(distance_median_bytes(I, J, false));
     void *scratch = nullptr;
     if (mode != WOTK_COST_F64) scratch = ar.take<char>(cost_bf16_scratch(I, J, d));
     if (!ar.ok || !workspace) return fail(WOTK_EWORKSPACE, "cost workspace too small");
-    rc = (mode == WOTK_COST_F64) ? launch_sqeuclid_f64(X, Y, I, J, d, C64, J, s)
-                                 : launch_cost_bf16(X, Y, I, J, d, mode == WOTK_COST_BF16X3 ? 3 : 6, C64, J,
-                                                    scratch, s);
+    DistanceProblem pb{X, Y, (int)I, (int)J, (int)d,
+                       mode == WOTK_COST_F64 ? 0 : mode == WOTK_COST_BF16X3 ? 3 : 6, 0, {}, {}};
+    if (pb.terms) rc = prepare_split(&pb, scratch, s);
     if (rc) return rc;
-    rc = median_run(C64, I * J, nullptr, median_index_out, st, h, s);
+    const double *median = nullptr;
+    rc = distance_median(pb, false, med_ws, median_index_out, &median, s);
     if (rc) return rc;
-    rc = launch_normalise_transpose(C64, J, I, J, &st->median, 1.0, C, ldc, CT, ldct, s);
+    rc = launch_cost_write(pb, median, C, ldc, CT, ldct, s);
     if (rc) return rc;
-    if (median_out) WOTK_HIP(hipMemcpyAsync(median_out, &st->median, sizeof(double), hipMemcpyDeviceToDevice, s));
+    if (median_out) WOTK_HIP(hipMemcpyAsync(median_out, median, sizeof(double), hipMemcpyDeviceToDevice, s));
     return WOTK_OK;
 }
 
@@ -381,6 +299,5 @@ extern "C" int wotk_cost_import(const double *C64, int64_t I, int64_t J, int64_t
     int rc = check_cost_layout(I, J, 1, C, ldc, CT, ldct);
     if (rc) return rc;
     WOTK_REQUIRE(ld64 >= J, "ld64 < J");
-    return launch_normalise_transpose(C64, ld64, I, J, nullptr, scale, C, ldc, CT, ldct,
-                                      (hipStream_t)stream);
+    return launch_normalise_transpose(C64, ld64, I, J, scale, C, ldc, CT, ldct, (hipStream_t)stream);
 }

@@ -18,11 +18,11 @@
 // the batched sweep); rows whose sum under- or overflows are queued and
 // recomputed by a repair kernel from FP64 direct distances with an online
 // maximum.  The median of the exact FP64 distances (the reference's
-// normalisation) comes from a radix select that regenerates the distances in
-// every pass.
+// normalisation) comes from two passes that regenerate them (distance.hip).
 #include <type_traits>
 
 #include "common.h"
+#include "distance.h"
 #include "fused_problem.h"
 
 namespace wotk {
@@ -75,117 +75,6 @@ __global__ __launch_bounds__(256) void fz_split_kernel(const double *__restrict_
         if (npiece > 2) p2[(int64_t)i * kp + k] = (__bf16)(float)r2;
     }
     norm[i] = acc;
-}
-
-// ---------------------------------------------------------------------------
-// exact median of D_ij = sum_k (x_ik - y_jk)^2 without storing D: each pass
-// regenerates 64 x 64 tiles in FP64 and histograms the keys matching the
-// prefix found so far (same digit schedule as the stored-matrix select)
-// ---------------------------------------------------------------------------
-struct FzSelect {
-    unsigned long long prefix, mask;
-    long long rank;
-    unsigned long long eq, next;
-    double median;
-};
-
-template <int MODE>  // 0: histogram digit, 1: smallest key above the prefix
-__global__ __launch_bounds__(256) void fz_select_kernel(const double *__restrict__ X, const double *__restrict__ Y,
-                                                        int n_i, int n_j, int d, int shift, int width,
-                                                        FzSelect *__restrict__ st,
-                                                        unsigned long long *__restrict__ ghist) {
-    __shared__ double xs[32][64];
-    __shared__ double ys[32][64];
-    __shared__ unsigned int h[2048];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-    if (MODE == 0)
-        for (int b = tid; b < 2048; b += 256) h[b] = 0u;
-    double acc[4][4] = {};
-    for (int k0 = 0; k0 < d; k0 += 32) {
-        for (int e = tid; e < 64 * 32; e += 256) {
-            const int r = e / 32, kk = e % 32;
-            const bool kin = k0 + kk < d;
-            xs[kk][r] = (kin && i0 + r < n_i) ? X[(int64_t)(i0 + r) * d + k0 + kk] : 0.0;
-            ys[kk][r] = (kin && j0 + r < n_j) ? Y[(int64_t)(j0 + r) * d + k0 + kk] : 0.0;
-        }
-        __syncthreads();
-        const int km = min(32, d - k0);
-        for (int kk = 0; kk < km; ++kk)
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const double t = xs[kk][ty * 4 + a] - ys[kk][tx * 4 + b];
-                    acc[a][b] = fma(t, t, acc[a][b]);
-                }
-        __syncthreads();
-    }
-    const unsigned long long prefix = st->prefix, mask = st->mask;
-    unsigned long long best = ~0ull;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            if (i0 + ty * 4 + a >= n_i || j0 + tx * 4 + b >= n_j) continue;
-            const unsigned long long key = (unsigned long long)__double_as_longlong(acc[a][b]);
-            if (MODE == 0) {
-                if ((key & mask) == prefix) atomicAdd(&h[(key >> shift) & ((1ull << width) - 1ull)], 1u);
-            } else {
-                if (key > prefix && key < best) best = key;
-            }
-        }
-    if (MODE == 0) {
-        __syncthreads();
-        for (int b = tid; b < 2048; b += 256)
-            if (h[b]) atomicAdd(&ghist[b], (unsigned long long)h[b]);
-    } else {
-        for (int off = 32; off > 0; off >>= 1) {
-            const unsigned long long o = __shfl_xor(best, off);
-            best = o < best ? o : best;
-        }
-        if ((tid & 63) == 0 && best != ~0ull) atomicMin(&st->next, best);
-    }
-}
-
-__global__ void fz_select_init_kernel(FzSelect *st, long long rank, unsigned long long *hist) {
-    for (int b = threadIdx.x; b < 2048; b += blockDim.x) hist[b] = 0ull;
-    if (threadIdx.x) return;
-    st->prefix = 0ull;
-    st->mask = 0ull;
-    st->rank = rank;
-    st->eq = 0ull;
-    st->next = ~0ull;
-}
-
-__global__ __launch_bounds__(256) void fz_select_scan_kernel(unsigned long long *__restrict__ ghist, int shift,
-                                                             int width, int last, FzSelect *__restrict__ st) {
-    if (threadIdx.x == 0) {
-        const int nb = 1 << width;
-        long long rank = st->rank;
-        unsigned long long cum = 0;
-        int b = 0;
-        for (; b < nb - 1; ++b) {
-            if (cum + ghist[b] > (unsigned long long)rank) break;
-            cum += ghist[b];
-        }
-        st->prefix |= (unsigned long long)b << shift;
-        st->mask |= ((1ull << width) - 1ull) << shift;
-        st->rank = rank - (long long)cum;
-        if (last) st->eq = ghist[b];
-    }
-    __syncthreads();
-    for (int b = threadIdx.x; b < 2048; b += blockDim.x) ghist[b] = 0ull;
-}
-
-__global__ void fz_select_finish_kernel(FzSelect *st, int odd) {
-    const double lo = __longlong_as_double((long long)st->prefix);
-    double m = lo;
-    if (!odd) {
-        const bool tie = (unsigned long long)(st->rank + 1) < st->eq;
-        m = (lo + (tie ? lo : __longlong_as_double((long long)st->next))) / 2.0;
-    }
-    st->median = m;
 }
 
 // ---------------------------------------------------------------------------
@@ -474,9 +363,6 @@ __global__ void fz_zero_kernel(double *x, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) x[i] = 0.0;
 }
 
-static const int kFzShift[6] = {53, 42, 31, 20, 10, 0};
-static const int kFzWidth[6] = {11, 11, 11, 11, 10, 10};
-
 // column splits per sweep: enough blocks for ~3 waves per SIMD (the kernel
 // holds 166 VGPRs), at least 8 column tiles per split
 static int fused_splits(int n_rows, int n_cols) {
@@ -535,8 +421,7 @@ static void problem_carve(Arena &ar, int64_t I, int64_t J, int64_t d, FusedProbl
     fp->nbad2 = ar.take<int>(4);
     fp->part = ar.take<double>((size_t)kFusedMaxSplit * std::max(I, J));
     fp->part2 = ar.take<double>((size_t)kFusedMaxSplit * std::max(I, J));
-    fp->sel = ar.take<FzSelect>(1);
-    fp->hist = ar.take<unsigned long long>(2048);
+    fp->median_ws = ar.take<char>(distance_median_bytes(I, J, true));
 }
 
 size_t fused_problem_bytes(int64_t I, int64_t J, int64_t d) {
@@ -565,19 +450,9 @@ int fused_problem_setup(const double *X, const double *Y, int64_t I, int64_t J, 
     fp->terms = terms;
 
     // exact median of the FP64 distances, regenerated per pass
-    const long long n = (long long)I * J;
-    const long long rank = (n % 2) ? n / 2 : n / 2 - 1;
-    fz_select_init_kernel<<<1, 256, 0, s>>>(fp->sel, rank, fp->hist);
-    dim3 sgrid((unsigned)((J + 63) / 64), (unsigned)((I + 63) / 64));
-    for (int p = 0; p < 6; ++p) {
-        fz_select_kernel<0><<<sgrid, 256, 0, s>>>(X, Y, (int)I, (int)J, (int)d, kFzShift[p], kFzWidth[p], fp->sel,
-                                                  fp->hist);
-        fz_select_scan_kernel<<<1, 256, 0, s>>>(fp->hist, kFzShift[p], kFzWidth[p], p == 5, fp->sel);
-    }
-    if (n % 2 == 0) fz_select_kernel<1><<<sgrid, 256, 0, s>>>(X, Y, (int)I, (int)J, (int)d, 0, 0, fp->sel, fp->hist);
-    fz_select_finish_kernel<<<1, 1, 0, s>>>(fp->sel, (int)(n % 2));
-    WOTK_LAUNCH_CHECK();
-    fp->median = &fp->sel->median;
+    const DistanceProblem dp{X, Y, (int)I, (int)J, (int)d, 0, 0, {}, {}};
+    int rc = distance_median(dp, true, fp->median_ws, nullptr, &fp->median, s);
+    if (rc) return rc;
 
     // scaled, centred coordinates and their bf16 pieces
     fz_mean_kernel<<<(unsigned)d, 256, 0, s>>>(X, (int)I, Y, (int)J, (int)d, fp->mean);

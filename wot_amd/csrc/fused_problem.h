@@ -9,8 +9,6 @@
 
 namespace wotk {
 
-struct FzSelect;
-
 // C = sqeuclid(X, Y) / median(sqeuclid(X, Y)) regenerated per tile from the
 // scaled, centred coordinates' split-BF16 pieces; buffers carved from a
 // caller workspace by fused_problem_setup.
@@ -22,8 +20,7 @@ struct FusedProblem {
     int *bad = nullptr, *nbad = nullptr;    // repair list of the sweeps
     int *bad2 = nullptr, *nbad2 = nullptr;  // and of the sum passes (which may run on another stream)
     double *part = nullptr, *part2 = nullptr;
-    FzSelect *sel = nullptr;
-    unsigned long long *hist = nullptr;
+    void *median_ws = nullptr;
     const double *median = nullptr;  // device: the exact median of the FP64 distances
 };
 
