@@ -1,0 +1,101 @@
+"""The one-read iteration (pairs from 2^23 entries) against the two sweeps the
+no-allocation entry point keeps, at the edges of its column chunks and row
+steps, and where rows and columns leave its FP32 range."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# columns at and around the 3840-column chunks (1 to 5 chunks, 4 / 2 / 1 rows per step), the largest
+# width, rows that do not divide by the 256 workgroups or by the rows of a step, one row less than a round
+SHAPES = [(2049, 4095), (2500, 4096), (2051, 4097), (1100, 8192), (1023, 8193), (701, 12289), (513, 16384),
+          (515, 16389), (415, 20288), (9000, 1001)]
+# lanes sum in another order (FP32 partial sums of at most 60 terms each, then FP64): the plan moves by a few
+# 1e-9 per sum, as between the sweep's own tile variants (1e-6 is what those are held to)
+TOL = 1e-6
+
+
+def _run(fn, cost, G, prm, ws=None):
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    n_i, n_j = cost.shape
+    f = torch.empty(n_i, dtype=torch.float64, device='cuda')
+    g = torch.empty(n_j, dtype=torch.float64, device='cuda')
+    p = dev._ptr
+    st = _native.Stats()
+    args = [p(cost.C), cost.ldc, p(cost.CT), cost.ldct, n_i, n_j, p(G), prm['lambda1'], prm['lambda2'], prm['epsilon'],
+            prm['scaling_iter'], 1e4, prm['epsilon0'], prm['extra_iter'], prm['inner_iter_max'], None, n_j, None, p(f),
+            p(g)]
+    if ws is not None:
+        args += [p(ws), ws.numel()]
+    args += [ctypes.byref(st), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)]
+    _native.check(fn(*args))
+    return f, g, st.epsilon_final
+
+
+def _both(x, y, G, **kw):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, scaling_iter=150, extra_iter=20,
+               inner_iter_max=50)
+    prm.update(kw)
+    cost = ot.DeviceCost.from_coordinates(x, y)
+    Gd = torch.from_numpy(np.ascontiguousarray(G)).cuda()
+    L = _native.lib()
+    ws = dev.workspace(torch, L.wotk_solver_workspace_size(*cost.shape), 'cuda')
+    one = _run(L.wotk_transport_stablev2, cost, Gd, prm, ws)
+    two = _run(L.wotk_transport_stablev2_noalloc, cost, Gd, prm)
+    return cost, one, two
+
+
+def _plan(cost, r):
+    import torch
+    return torch.exp((r[0][:, None] + r[1][None, :] - cost.dense().double()) / r[2])
+
+
+@pytest.mark.parametrize('n_i,n_j', SHAPES)
+def test_one_read_iteration_matches_two_sweeps(n_i, n_j):
+    import torch
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(n_i, n_j, dim=30, n_components=5, seed=n_i)
+    cost, one, two = _both(dp.x, dp.y, dp.growth)
+    a, b = _plan(cost, one), _plan(cost, two)
+    assert float((a - b).norm() / b.norm()) < TOL
+    for d in (0, 1):
+        assert float(((a.sum(d) - b.sum(d)).abs() / b.sum(d)).max()) < TOL
+
+
+@pytest.mark.parametrize('eps', [0.05, 0.003])
+def test_rows_and_columns_out_of_range(eps):
+    """Outlier cells on both sides and a first eps far below the cost's scale: first sums under 2^-40."""
+    import torch
+    rng = np.random.default_rng(7)
+    x, y = rng.standard_normal((2100, 30)), rng.standard_normal((4100, 30))
+    x[::97] *= 12.0
+    y[5::113] *= 15.0
+    G = np.exp(0.3 * rng.standard_normal(2100))
+    cost, one, two = _both(x, y, G, epsilon=eps, epsilon0=eps, scaling_iter=0, extra_iter=30)
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.isfinite(a).all()
+        # potentials of the scale of the cost; both paths round exponents of up to |C| / eps at 2^-24
+        assert float((a - b).abs().max()) < 1e-6 * float(b.abs().max())
+
+
+def test_zero_and_nan_growth_travel_as_in_the_sweeps():
+    import torch
+    rng = np.random.default_rng(8)
+    x, y = rng.standard_normal((2100, 30)), rng.standard_normal((4100, 30))
+    G = np.ones(2100)
+    G[17] = 0.0
+    _, one, two = _both(x, y, G, scaling_iter=0, extra_iter=3)
+    assert torch.equal(torch.isinf(one[0]), torch.isinf(two[0])) and bool(torch.isinf(one[0])[17])
+    assert float((one[1] - two[1]).abs().max()) < 1e-7 * float(two[1].abs().max())
+    G[17] = np.nan
+    _, one, two = _both(x, y, G, scaling_iter=0, extra_iter=2)
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))

@@ -23,6 +23,7 @@
 
 #include "common.h"
 #include "fused_problem.h"
+#include "onepass.h"
 
 namespace wotk {
 
@@ -501,9 +502,11 @@ struct Work {
     double *fs, *gs, *us, *vs;  // snapshot of the last scaling's state (gap pass ahead of the next batch)
     long long *counter;
     int nparts;
+    float *col_part;  // column partials of the one-read iteration, or nullptr: two sweeps
 };
 
-static size_t carve(Arena &ar, int64_t I, int64_t J, Work *w) {
+// one_pass: with the column partials where the shape takes the one-read iteration
+static size_t carve(Arena &ar, int64_t I, int64_t J, bool one_pass, Work *w) {
     const int64_t I4 = round_up(I, 4), J4 = round_up(J, 4);
     w->f = ar.take<double>(I4);
     w->g = ar.take<double>(J4);
@@ -525,6 +528,8 @@ static size_t carve(Arena &ar, int64_t I, int64_t J, Work *w) {
     w->us = ar.take<double>(I4);
     w->vs = ar.take<double>(J4);
     w->counter = ar.take<long long>(4);
+    w->col_part = nullptr;
+    if (one_pass && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
     return ar.off;
 }
 
@@ -579,6 +584,10 @@ static int launch_lse(const float *A, int64_t lda, int nrows, int ncols, const d
 // one (a, b) iteration at eps: f from g over C, then g from f over C^T
 static int iterate(const Problem &pb, Work &w, double lambda1, double lambda2, double eps,
                    hipStream_t s) {
+    if (w.col_part)
+        return one_pass_iterate(OnePass{pb.C, pb.ldc, pb.CT, pb.ldct, pb.n_i, pb.n_j, w.f, w.g, w.logp, w.misc,
+                                        w.col_part},
+                                lambda1, lambda2, eps, s);
     RowEpilogue er{w.logp, nullptr, std::log((double)pb.n_j), lambda1 / (lambda1 + eps), eps, w.f,
                    nullptr};
     int rc = launch_lse(pb.C, pb.ldc, pb.n_i, pb.n_j, w.g, eps, er, s);
@@ -654,11 +663,11 @@ using namespace wotk;
 extern "C" size_t wotk_solver_workspace_size(int64_t I, int64_t J) {
     Arena ar(nullptr, 0);
     Work w;
-    return carve(ar, I, J, &w);
+    return carve(ar, I, J, true, &w);
 }
 
 static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
-                 const double *G, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
+                 const double *G, bool one_pass, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
                  hipStream_t s) {
     WOTK_REQUIRE(I > 0 && J > 0 && I < (1ll << 31) && J < (1ll << 31), "bad shape %lld x %lld",
                  (long long)I, (long long)J);
@@ -666,7 +675,7 @@ static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int
     int rc = check_problem(*pb);
     if (rc) return rc;
     Arena ar(workspace, ws_bytes);
-    carve(ar, I, J, w);
+    carve(ar, I, J, one_pass, w);
     if (!workspace || !ar.ok) return fail(WOTK_EWORKSPACE, "solver workspace too small");
     return init_state(*pb, *w, s);
 }
@@ -736,7 +745,7 @@ extern "C" int wotk_transport_stablev2(const float *C, int64_t ldc, const float 
     hipStream_t s = (hipStream_t)stream;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     (void)tau;  // absorption is exact in the log domain; tau only changes the FP64 reference's rounding
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
@@ -783,7 +792,9 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
                                                wotk_stats *stats, void *stream) {
     WOTK_REQUIRE(I > 0 && J > 0 && I < (1ll << 31) && J < (1ll << 31), "bad shape %lld x %lld", (long long)I,
                  (long long)J);
-    const size_t need = wotk_solver_workspace_size(I, J);
+    Arena count(nullptr, 0);
+    Work counted;
+    const size_t need = carve(count, I, J, false, &counted);
     WOTK_REQUIRE(need <= kScratchBytes,
                  "%lld x %lld needs %zu bytes of solver state; the no-allocation entry point holds %zu "
                  "(use wotk_transport_stablev2 with a workspace)",
@@ -794,7 +805,7 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
     if (rc) return rc;
     Problem pb;
     Work w;
-    rc = setup(C, ldc, CT, ldct, I, J, G, ws, kScratchBytes, &pb, &w, s);
+    rc = setup(C, ldc, CT, ldct, I, J, G, false, ws, kScratchBytes, &pb, &w, s);
     if (rc) return rc;
     (void)tau;
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
@@ -994,7 +1005,7 @@ extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const flo
     hipStream_t s = (hipStream_t)stream;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     WOTK_REQUIRE(!plan || ldp >= J, "ldp < J");
     StoredBackend be{pb, w, plan, ldp, row_sums, f_out, g_out};
@@ -1089,7 +1100,7 @@ struct FusedBackend {
 extern "C" size_t wotk_duality_gap_coords_workspace_size(int64_t I, int64_t J, int64_t d) {
     Arena ar(nullptr, 0);
     Work w;
-    return fused_problem_bytes(I, J, d) + 256 + carve(ar, I, J, &w);
+    return fused_problem_bytes(I, J, d) + 256 + carve(ar, I, J, false, &w);
 }
 
 extern "C" int wotk_transport_duality_gap_coords(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
@@ -1107,7 +1118,7 @@ extern "C" int wotk_transport_duality_gap_coords(const double *X, const double *
     used = (used + 255) & ~size_t(255);
     Arena ar(static_cast<char *>(workspace) + used, workspace_bytes > used ? workspace_bytes - used : 0);
     Work w;
-    carve(ar, I, J, &w);
+    carve(ar, I, J, false, &w);
     if (!ar.ok) return fail(WOTK_EWORKSPACE, "workspace too small");
     const Problem pb{nullptr, 0, nullptr, 0, (int)I, (int)J, G};
     rc = init_state(pb, w, s);
@@ -1136,7 +1147,7 @@ extern "C" int wotk_primal_dual(const float *C, int64_t ldc, const float *CT, in
     hipStream_t s = (hipStream_t)stream;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     WOTK_REQUIRE(out_host != nullptr, "out_host is required");
     copy2_kernel<<<64, 256, 0, s>>>(w.f, f, pb.n_i, w.g, g, pb.n_j);
