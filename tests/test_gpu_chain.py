@@ -65,3 +65,31 @@ def test_glue_reorders_intermediate_cells(tm):
     np.testing.assert_allclose(out32.X, x0 @ x1, rtol=1e-6)
     with pytest.raises(ValueError):
         tm.glue_transport_maps(t0, t1, precision='float16')
+
+
+@pytest.mark.parametrize('m,k,n', [(2945, 33, 3001), (2050, 64, 1900), (1025, 70, 1030), (1024, 31, 1024),
+                                   (64, 127, 64), (65, 1000, 63), (1, 1, 1), (513, 257, 2), (3, 96, 640)])
+def test_gemm_tiles_exact(tm, m, k, n):
+    """Every tile size and the shared-K groups, odd row starts, K tails: exact on small integers."""
+    import torch
+    g = torch.Generator(device='cuda').manual_seed(m + k + n)
+    A = torch.randint(-4, 5, (m, k + 3), device='cuda', generator=g).float()[:, 1:k + 1]
+    B = torch.randint(-4, 5, (k, n + 1), device='cuda', generator=g).float()[:, 1:]
+    C = torch.full((m, n + 5), -7.0, device='cuda')
+    import ctypes
+    from wot_amd import _native
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    _native.check(_native.lib().wotk_gemm_f32(p(A), A.stride(0), p(B), B.stride(0), p(C), C.stride(0), m, n, k,
+                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    ref = (A.double() @ B.double()).float()
+    assert torch.equal(C[:, :n], ref)
+    assert bool((C[:, n:] == -7.0).all())
+
+
+def test_gemm_nonfinite(tm):
+    import torch
+    A, B = torch.ones((70, 40), device='cuda'), torch.ones((40, 70), device='cuda')
+    A[3, 5], B[7, 9], A[69, 39] = float('inf'), float('nan'), float('-inf')
+    C = tm.gemm_f32(A, B).cpu()
+    ref = (A.cpu().double() @ B.cpu().double()).float()
+    assert torch.equal(torch.isnan(C), torch.isnan(ref)) and torch.equal(torch.isinf(C), torch.isinf(ref))
