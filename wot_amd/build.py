@@ -25,6 +25,9 @@ DEVICE_FLAGS = [
 # in ordinary VGPRs (no AGPR copies before the per-entry exponentials)
 SOURCE_FLAGS = {
     'fused.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    # the resident solver's registers hold the cost: constants of the logarithms and
+    # exponentials are formed where they are used, not kept across its loops
+    'resident.hip': ['-mllvm', '-disable-machine-licm'],
 }
 
 

@@ -16,14 +16,15 @@
 // exactly (ldexp) in FP64.  Absorption events are tracked only where the
 // reference's control flow observes them (the duality-gap solver's
 // dual-evolution check).
+#include <algorithm>
 #include <array>
-#include <utility>
-
 #include <mutex>
+#include <utility>
 
 #include "common.h"
 #include "fused_problem.h"
 #include "onepass.h"
+#include "resident.h"
 
 namespace wotk {
 
@@ -503,10 +504,11 @@ struct Work {
     long long *counter;
     int nparts;
     float *col_part;  // column partials of the one-read iteration, or nullptr: two sweeps
+    void *exchange;   // exchange buffers of the resident solver, or nullptr: launches per sweep
 };
 
-// one_pass: with the column partials where the shape takes the one-read iteration
-static size_t carve(Arena &ar, int64_t I, int64_t J, bool one_pass, Work *w) {
+// extras: with the buffers of the resident solver or the one-read iteration where the shape takes them
+static size_t carve(Arena &ar, int64_t I, int64_t J, bool extras, Work *w) {
     const int64_t I4 = round_up(I, 4), J4 = round_up(J, 4);
     w->f = ar.take<double>(I4);
     w->g = ar.take<double>(J4);
@@ -529,7 +531,9 @@ static size_t carve(Arena &ar, int64_t I, int64_t J, bool one_pass, Work *w) {
     w->vs = ar.take<double>(J4);
     w->counter = ar.take<long long>(4);
     w->col_part = nullptr;
-    if (one_pass && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
+    if (extras && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
+    w->exchange = nullptr;
+    if (extras && resident_fits(I, J)) w->exchange = ar.take<char>(resident_bytes(I, J));
     return ar.off;
 }
 
@@ -667,7 +671,7 @@ extern "C" size_t wotk_solver_workspace_size(int64_t I, int64_t J) {
 }
 
 static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
-                 const double *G, bool one_pass, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
+                 const double *G, bool extras, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
                  hipStream_t s) {
     WOTK_REQUIRE(I > 0 && J > 0 && I < (1ll << 31) && J < (1ll << 31), "bad shape %lld x %lld",
                  (long long)I, (long long)J);
@@ -675,7 +679,7 @@ static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int
     int rc = check_problem(*pb);
     if (rc) return rc;
     Arena ar(workspace, ws_bytes);
-    carve(ar, I, J, one_pass, w);
+    carve(ar, I, J, extras, w);
     if (!workspace || !ar.ok) return fail(WOTK_EWORKSPACE, "solver workspace too small");
     return init_state(*pb, *w, s);
 }
@@ -688,6 +692,10 @@ struct EventPair {
             if (e) (void)hipEventDestroy(e);
     }
 };
+
+static ResidentProblem resident_problem(const Problem &pb, const Work &w) {
+    return ResidentProblem{pb.C, pb.ldc, pb.CT, pb.ldct, pb.n_i, pb.n_j, pb.G, w.logp, w.misc, w.f, w.g, w.exchange};
+}
 
 // the fixed-iteration schedule on a set-up problem (shared by the workspace
 // and the scratch entry points); `timed` brackets the sweeps with events
@@ -709,14 +717,32 @@ static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambd
         WOTK_HIP(hipEventRecord(evs.ev[0], s));
     }
     int rc = 0;
-    for (int64_t n = 0; n < scaling_iter; ++n) {
-        rc = iterate(pb, w, lambda1, lambda2, reg(n / inner_iter_max), s);
-        if (rc) return rc;
-    }
     const double eps_end = reg(scaling_iter / inner_iter_max);
-    for (int64_t n = 0; n < extra_iter; ++n) {
-        rc = iterate(pb, w, lambda1, lambda2, eps_end, s);
+    bool done = false;
+    if (w.exchange) {
+        const ResidentProblem rp = resident_problem(pb, w);
+        int launched = 0;
+        rc = resident_fixed(rp, lambda1, lambda2, epsilon, epsilon0, scaling_iter, inner_iter_max, extra_iter,
+                            &launched, s);
         if (rc) return rc;
+        if (launched) {
+            ResidentResult r;
+            rc = resident_result(rp, &r, s);
+            if (rc) return rc;
+            done = !r.aborted;
+            if (!done) rc = init_state(pb, w, s);
+            if (rc) return rc;
+        }
+    }
+    if (!done) {
+        for (int64_t n = 0; n < scaling_iter; ++n) {
+            rc = iterate(pb, w, lambda1, lambda2, reg(n / inner_iter_max), s);
+            if (rc) return rc;
+        }
+        for (int64_t n = 0; n < extra_iter; ++n) {
+            rc = iterate(pb, w, lambda1, lambda2, eps_end, s);
+            if (rc) return rc;
+        }
     }
     if (timed) WOTK_HIP(hipEventRecord(evs.ev[1], s));
     rc = finish_outputs(pb, w, eps_end, (double)pb.n_j, plan, ldp, row_sums, f_out, g_out, s);
@@ -1009,6 +1035,42 @@ extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const flo
     if (rc) return rc;
     WOTK_REQUIRE(!plan || ldp >= J, "ldp < J");
     StoredBackend be{pb, w, plan, ldp, row_sums, f_out, g_out};
+    if (w.exchange) {
+        WOTK_REQUIRE(batch_size > 0, "batch_size must be positive");
+        const ResidentProblem rp = resident_problem(pb, w);
+        int launched = 0;
+        rc = resident_gap(rp, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, &launched, s);
+        if (rc) return rc;
+        if (launched) {
+            ResidentResult r;
+            rc = resident_result(rp, &r, s);
+            if (rc) return rc;
+            if (!r.aborted) {
+                if (stats) {
+                    *stats = wotk_stats{};
+                    stats->iterations = r.iterations;
+                    stats->stabilisations = r.stabilisations;
+                    stats->gap_checks = r.checks;
+                    stats->gap = r.gap;
+                    stats->epsilon_final = r.eps;
+                    stats->max_iter_reached = r.max_iter_reached;
+                    if (!r.max_iter_reached) {
+                        stats->primal = r.primal;
+                        stats->dual = r.dual;
+                    }
+                }
+                if (!r.max_iter_reached && std::isnan(r.gap))
+                    return fail(WOTK_ENAN,
+                                "Overflow encountered in duality gap computation, please report this incident");
+                rc = be.finish(r.eps, r.max_iter_reached ? 1.0 : (double)J, s);
+                if (rc) return rc;
+                WOTK_HIP(hipStreamSynchronize(s));
+                return WOTK_OK;
+            }
+            rc = init_state(pb, w, s);
+            if (rc) return rc;
+        }
+    }
     return gap_schedule(be, pb, w, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, stats,
                         s);
 }
