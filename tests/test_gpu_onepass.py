@@ -99,3 +99,29 @@ def test_zero_and_nan_growth_travel_as_in_the_sweeps():
     _, one, two = _both(x, y, G, scaling_iter=0, extra_iter=2)
     for a, b in zip(one[:2], two[:2]):
         assert torch.equal(torch.isnan(a), torch.isnan(b))
+
+
+@pytest.mark.parametrize('n_i,n_j,kw', [(2100, 4100, {}), (4300, 2049, dict(batch_size=3, epsilon=0.1)),
+                                        (2100, 4100, dict(tau=2.0)), (2100, 4100, dict(tau=2.0, max_iter=23)),
+                                        (2100, 4100, dict(max_iter=35)), (2100, 4100, dict(max_iter=452))])
+def test_duality_gap_schedule_matches_fp64(n_i, n_j, kw):
+    """Counts and plan of the schedule with the tau check inside the iteration, batches queued ahead of the
+    evolution checks and the one-read gap pass, against the FP64 restatement on the device."""
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import plain_gpu
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(n_i, n_j, dim=30, n_components=5, seed=n_j)
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, batch_size=5, tolerance=1e-8, tau=1e4, epsilon0=1.0,
+               max_iter=1e7)
+    prm.update(kw)
+    cost = ot.DeviceCost.from_coordinates(dp.x, dp.y)
+    st, so = {}, {}
+    R = ot.optimal_transport_duality_gap(cost, dp.growth, stats=st, device_out=True, **prm)
+    ref = plain_gpu.optimal_transport_duality_gap(cost.dense().double(), torch.from_numpy(dp.growth).cuda(), stats=so,
+                                                  **prm)
+    assert st['iterations'] == so['iterations']
+    assert bool(st['max_iter_reached']) == (st['iterations'] >= prm['max_iter'])
+    if 'stabilisations' in so:
+        assert st['stabilisations'] == so['stabilisations']
+    assert float((R - ref).norm() / ref.norm()) < 1e-6

@@ -58,6 +58,8 @@ struct RowArgs {
     double log_nj, alpha, eps, k;
     float *part;
     int ld_part;
+    TauTrack tau;
+    const int *skip;
 };
 
 typedef const __attribute__((address_space(4))) double *ScalarPtr;
@@ -285,6 +287,11 @@ struct RowPass {
 template <int R>
 __device__ void finish_rows(const RowArgs &ra, RowShared<R> &sh, int n) {
     const int lane = threadIdx.x & 63, r = lane >> 4;
+    const bool absorb = ra.tau.prev && tau_fired(*ra.tau.prev, ra.tau.tau);
+    if (ra.tau.prev && blockIdx.x == 0 && lane == 0) {
+        if (absorb) ra.tau.counter[0] += 1;
+        *ra.tau.cur = tau_key(-INFINITY);
+    }
     for (int it = 0; it < n; ++it) {
         const int row = first_row(it, R) + r;
         const bool mine = r < R && row < ra.n_i;
@@ -298,6 +305,7 @@ __device__ void finish_rows(const RowArgs &ra, RowShared<R> &sh, int n) {
         const double w = exp2(ra.k * fn + (double)N);
         if ((lane & 15) == 15 && r < R) {
             const bool out = S < kRowLo || S > kRowHi;
+            if (mine && absorb) ra.tau.u[row] = fo;
             if (mine && out) atomicOr(&sh.bad[(it * R + r) >> 5], 1u << ((it * R + r) & 31));
             if (mine && !out) ra.f[row] = fn;
             sh.wrow[it & 1][r] = mine && !out ? w : 0.0;
@@ -351,6 +359,7 @@ template <int NC, int R, int DEPTH, int T>
 __global__ __launch_bounds__(T) void one_pass_rows_kernel(RowArgs ra) {
     extern __shared__ __align__(16) double2 h_lds[];
     __shared__ RowShared<R> sh;
+    if (ra.skip && *ra.skip) return;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int waves = (int)blockDim.x >> 6, ct = (waves - 1) * 64;
@@ -404,6 +413,8 @@ struct ColArgs {
     double log_ni, alpha, eps, k;
     const float *part;
     int ld_part, n_part;
+    TauTrack tau;
+    const int *skip;
 };
 
 // g from the workgroups' column sums: 64 columns per workgroup, 16 threads per
@@ -413,6 +424,8 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
     __shared__ int bad[64];
     __shared__ int n_bad;
     __shared__ double wred[kW];
+    if (ca.skip && *ca.skip) return;
+    const bool absorb = ca.tau.prev && tau_fired(*ca.tau.prev, ca.tau.tau);
     const int c = threadIdx.x & 63, p = threadIdx.x >> 6;
     const int j = blockIdx.x * 64 + c;
     if (threadIdx.x == 0) n_bad = 0;
@@ -426,6 +439,7 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
     __syncthreads();
     if (p == 0 && j < ca.n_j) {
         for (int q = 1; q < kW; ++q) s += red[q][c];
+        if (absorb) ca.tau.v[j] = ca.g[j];
         if (s < kColLo || s > kColHi) {
             bad[atomicAdd(&n_bad, 1)] = j;
         } else {
@@ -458,6 +472,20 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
             ca.g[col] = ca.alpha * ca.eps * (*ca.logq_dev + ca.log_ni - (log2(t) + sh) * kLn2);
         }
         __syncthreads();
+    }
+    if (ca.tau.prev) {  // largest growth over this workgroup's columns and its share of the rows
+        double m = -INFINITY;
+        if (p == 0 && j < ca.n_j) m = (ca.g[j] - ca.tau.v[j]) * ca.tau.inv_eps;
+        for (int i = blockIdx.x * kT + threadIdx.x; i < ca.n_i; i += (int)gridDim.x * kT)
+            m = fmax(m, (ca.f[i] - ca.tau.u[i]) * ca.tau.inv_eps);
+        m = wave_max64(m);
+        __syncthreads();
+        if (c == 0) wred[p] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < kW; ++w) m = fmax(m, wred[w]);
+            atomicMax(ca.tau.cur, tau_key(m));
+        }
     }
 }
 
@@ -506,7 +534,7 @@ int one_pass_iterate(const OnePass &op, double lambda1, double lambda2, double e
     const double k = kLog2E / eps;
     const int grid = grid_of(op.n_i, op.n_j), ld = (int)round_up(op.n_j, 4);
     const RowArgs ra{op.C, op.ldc, op.n_i, op.n_j, op.f, op.g, op.logp, std::log((double)op.n_j),
-                     lambda1 / (lambda1 + eps), eps, k, op.part, ld};
+                     lambda1 / (lambda1 + eps), eps, k, op.part, ld, op.tau, op.skip};
     const bool narrow = waves_of(op.n_j) <= 12;
     int rc;
     switch (chunks_of(op.n_j)) {
@@ -518,7 +546,7 @@ int one_pass_iterate(const OnePass &op, double lambda1, double lambda2, double e
     }
     if (rc) return rc;
     const ColArgs ca{op.CT, op.ldct, op.n_i, op.n_j, op.f, op.g, op.logq_dev, std::log((double)op.n_i),
-                     lambda2 / (lambda2 + eps), eps, k, op.part, ld, grid};
+                     lambda2 / (lambda2 + eps), eps, k, op.part, ld, grid, op.tau, op.skip};
     one_pass_cols_kernel<<<(op.n_j + 63) / 64, kT, 0, s>>>(ca);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;

@@ -292,8 +292,10 @@ __global__ __launch_bounds__(1024) void stabilise_kernel(const double *__restric
     __shared__ int fire;
     // max over the exponents, then one exp (exp is increasing)
     double m = -INFINITY;
-    for (int i = threadIdx.x; i < n_i; i += blockDim.x) m = fmax(m, (f[i] - u[i]) * inv_eps);
-    for (int j = threadIdx.x; j < n_j; j += blockDim.x) m = fmax(m, (g[j] - v[j]) * inv_eps);
+#pragma unroll 8
+    for (int i = threadIdx.x; i < n_i; i += 1024) m = fmax(m, (f[i] - u[i]) * inv_eps);
+#pragma unroll 8
+    for (int j = threadIdx.x; j < n_j; j += 1024) m = fmax(m, (g[j] - v[j]) * inv_eps);
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -310,39 +312,89 @@ __global__ __launch_bounds__(1024) void stabilise_kernel(const double *__restric
     }
 }
 
-__global__ void zero_ll_kernel(long long *p, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
+// no absorptions, no growth yet, nothing to skip
+__global__ void clear_state_kernel(long long *counter, unsigned long long *slot, int *skip) {
+    const int i = threadIdx.x;
+    if (i < 4) {
+        counter[i] = 0;
+        slot[i] = tau_key(-INFINITY);
+        skip[i] = 0;
+    }
+}
+
+// Start of a scaling: absorb (u = f, v = g), no key, batches run.
+__global__ void scaling_begin_kernel(double *__restrict__ u, const double *__restrict__ f, int n_i,
+                                     double *__restrict__ v, const double *__restrict__ g, int n_j,
+                                     int *__restrict__ skip) {
+    const int stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int i = t; i < n_i; i += stride) u[i] = f[i];
+    for (int j = t; j < n_j; j += stride) v[j] = g[j];
+    if (t == 0) *skip = 0;
+}
+
+// (f, u, g, v) before the last iteration of a batch, with the absorption the iteration
+// before it may have called for (idempotent: the next iteration counts it)
+__global__ void before_last_kernel(const double *__restrict__ f, double *__restrict__ u, int n_i,
+                                   const double *__restrict__ g, double *__restrict__ v, int n_j,
+                                   double *__restrict__ fp, double *__restrict__ up, double *__restrict__ gp,
+                                   double *__restrict__ vp, const unsigned long long *__restrict__ slot, double tau,
+                                   const int *__restrict__ skip) {
+    if (*skip) return;
+    const int stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool fire = tau_fired(*slot, tau);
+    for (int i = t; i < n_i; i += stride) {
+        fp[i] = f[i];
+        if (fire) u[i] = f[i];
+        up[i] = u[i];
+    }
+    for (int j = t; j < n_j; j += stride) {
+        gp[j] = g[j];
+        if (fire) v[j] = g[j];
+        vp[j] = v[j];
+    }
+}
+
+// adds the absorption the last iteration called for (no iteration follows that would)
+__global__ void count_pending_kernel(const unsigned long long *slot, double tau, long long *counter) {
+    if (tau_fired(*slot, tau)) counter[0] += 1;
 }
 
 // state of the duality-gap solver's last scaling (f, g, u, v, stabilisation
-// count) to its snapshot (back = 0) or from it (back = 1: rolls back a batch
-// that ran ahead of its gap check)
+// count, growth key) to its snapshot (back = 0) or from it (back = 1: rolls back a
+// batch that ran ahead of its gap check)
 __global__ void snapshot_kernel(double *__restrict__ f, double *__restrict__ g, double *__restrict__ u,
                                 double *__restrict__ v, double *__restrict__ fs, double *__restrict__ gs,
                                 double *__restrict__ us, double *__restrict__ vs, int n_i, int n_j,
-                                long long *__restrict__ counter, int back) {
-    const int stride = gridDim.x * blockDim.x;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_i; i += stride) {
+                                long long *__restrict__ counter, unsigned long long *__restrict__ slots, int cur,
+                                double tau, int back) {
+    const int stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool fire = !back && tau_fired(slots[cur], tau);
+    for (int i = t; i < n_i; i += stride) {
         if (back) {
             f[i] = fs[i];
             u[i] = us[i];
         } else {
             fs[i] = f[i];
-            us[i] = u[i];
+            us[i] = fire ? f[i] : u[i];
         }
     }
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n_j; j += stride) {
+    for (int j = t; j < n_j; j += stride) {
         if (back) {
             g[j] = gs[j];
             v[j] = vs[j];
         } else {
             gs[j] = g[j];
-            vs[j] = v[j];
+            vs[j] = fire ? g[j] : v[j];
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (back) counter[0] = counter[1];
-        else counter[1] = counter[0];
+    if (t == 0) {
+        if (back) {
+            counter[0] = counter[1];
+            slots[cur] = slots[2];
+        } else {
+            counter[1] = counter[0];
+            slots[2] = slots[cur];
+        }
     }
 }
 
@@ -356,24 +408,29 @@ __global__ void copy2_kernel(double *__restrict__ d0, const double *__restrict__
 // dual-variable evolution check (optimal_transport.py:157-160):
 //   max(||A - A_old|| / (1 + ||A||), ||B - B_old|| / (1 + ||B||))
 // with A = exp(f/eps) and A_old = old_a * exp(u/eps) = exp((fp - up + u)/eps).
-__global__ __launch_bounds__(1024) void evolution_kernel(const double *__restrict__ f,
-                                                         const double *__restrict__ fp,
-                                                         const double *__restrict__ up,
-                                                         const double *__restrict__ u, int n_i,
-                                                         const double *__restrict__ g,
-                                                         const double *__restrict__ gp,
-                                                         const double *__restrict__ vp,
-                                                         const double *__restrict__ v, int n_j,
-                                                         double inv_eps, double *__restrict__ out) {
-    __shared__ double red[4][16];
+// Absorbs first, as the last iteration's growth calls for.  kEvoBlocks workgroups of
+// partial sums, then one (evolution_finish_kernel).
+__global__ __launch_bounds__(256) void evolution_kernel(const double *__restrict__ f, const double *__restrict__ fp,
+                                                        const double *__restrict__ up, double *__restrict__ u,
+                                                        int n_i, const double *__restrict__ g,
+                                                        const double *__restrict__ gp, const double *__restrict__ vp,
+                                                        double *__restrict__ v, int n_j, double inv_eps,
+                                                        const unsigned long long *__restrict__ slot, double tau,
+                                                        const int *__restrict__ skip, double *__restrict__ part) {
+    __shared__ double red[4][4];
+    if (skip && *skip) return;
+    const bool fire = tau_fired(*slot, tau);
+    const int stride = gridDim.x * 256, t0 = blockIdx.x * 256 + threadIdx.x;
     double d_a = 0.0, n_a = 0.0, d_b = 0.0, n_b = 0.0;
-    for (int i = threadIdx.x; i < n_i; i += blockDim.x) {
+    for (int i = t0; i < n_i; i += stride) {
+        if (fire) u[i] = f[i];
         const double A = exp(f[i] * inv_eps);
         const double Ao = exp((fp[i] - up[i]) * inv_eps) * exp(u[i] * inv_eps);
         d_a += (A - Ao) * (A - Ao);
         n_a += A * A;
     }
-    for (int j = threadIdx.x; j < n_j; j += blockDim.x) {
+    for (int j = t0; j < n_j; j += stride) {
+        if (fire) v[j] = g[j];
         const double B = exp(g[j] * inv_eps);
         const double Bo = exp((gp[j] - vp[j]) * inv_eps) * exp(v[j] * inv_eps);
         d_b += (B - Bo) * (B - Bo);
@@ -391,13 +448,27 @@ __global__ __launch_bounds__(1024) void evolution_kernel(const double *__restric
         red[3][w] = n_b;
     }
     __syncthreads();
+    if (threadIdx.x < 4) {
+        const double *r = red[threadIdx.x];
+        part[4 * blockIdx.x + threadIdx.x] = ((r[0] + r[1]) + r[2]) + r[3];
+    }
+}
+
+// out[0] = the evolution; *skip = 1 when it is no longer above `threshold`
+__global__ __launch_bounds__(64) void evolution_finish_kernel(const double *__restrict__ part, int n_part,
+                                                              double threshold, int *__restrict__ skip,
+                                                              double *__restrict__ out) {
+    if (*skip) return;
+    double t[4] = {0, 0, 0, 0};
+    if ((int)threadIdx.x < n_part)
+        for (int q = 0; q < 4; ++q) t[q] = part[4 * threadIdx.x + q];
+    for (int q = 0; q < 4; ++q) t[q] = wave_sum(t[q]);
     if (threadIdx.x == 0) {
-        double t[4] = {0, 0, 0, 0};
-        for (int q = 0; q < 4; ++q)
-            for (int k = 0; k < (int)(blockDim.x >> 6); ++k) t[q] += red[q][k];
         const double ga = sqrt(t[0]) / (1.0 + sqrt(t[1]));
         const double gb = sqrt(t[2]) / (1.0 + sqrt(t[3]));
-        out[0] = (gb > ga) ? gb : ga;  // python max(ga, gb): first argument unless gb > ga
+        const double gap = (gb > ga) ? gb : ga;  // python max(ga, gb): first argument unless gb > ga
+        out[0] = gap;
+        if (!(gap > threshold)) *skip = 1;
     }
 }
 
@@ -469,6 +540,190 @@ __global__ __launch_bounds__(1024) void gap_finish_kernel(GapArgs ga) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// The gap pass over one read of C (pairs that take the one-read iteration): the
+// row AND column sums of R = exp((f_i + g_j - C_ij)/eps) from one FP64 exponential
+// per entry.  128 rows x 1024 columns per workgroup, thread t the columns 4 t .. 4 t + 3:
+// column sums stay in registers, a row's sum is reduced over the wave; both go out as
+// partials per tile and are added in order.  Bound: FP64 issue, 28 operations per entry
+// (0.19 ms at 15000 x 15000) beside 0.17 ms of HBM; the two passes over C and C^T it
+// replaces took 0.25 + 0.21 ms alone and 0.47 + 0.28 ms next to the running sweeps.
+// ---------------------------------------------------------------------------
+constexpr int kGapRows = 128, kGapCols = 1024;
+
+// 2^x for x in [-1100, inf): x = n + r, exp(r ln 2) by its Taylor series to degree 13
+// (|r ln 2| <= 0.347: remainder under 5e-18), scaled by 2^n.  NaN stays NaN.
+__device__ __forceinline__ double exp2_f64(double x) {
+    const double n = rint(x), t = (x - n) * kLn2;
+    double p = 1.0 / 6227020800.0;
+    p = fma(p, t, 1.0 / 479001600.0);
+    p = fma(p, t, 1.0 / 39916800.0);
+    p = fma(p, t, 1.0 / 3628800.0);
+    p = fma(p, t, 1.0 / 362880.0);
+    p = fma(p, t, 1.0 / 40320.0);
+    p = fma(p, t, 1.0 / 5040.0);
+    p = fma(p, t, 1.0 / 720.0);
+    p = fma(p, t, 1.0 / 120.0);
+    p = fma(p, t, 1.0 / 24.0);
+    p = fma(p, t, 1.0 / 6.0);
+    p = fma(p, t, 0.5);
+    p = fma(p, t, 1.0);
+    p = fma(p, t, 1.0);
+    return ldexp(p, (int)n);
+}
+
+struct GapTileArgs {
+    const float *C;
+    int64_t ldc;
+    int n_i, n_j;
+    const double *f, *g;
+    double k;             // log2(e) / eps
+    double *row_part;     // [column tile][n_i]
+    double *col_part;     // [row tile][n_j]
+    double *partials;     // [tile][2]: sum R (f + g - C) k ln 2 = sum R log R, sum R C
+};
+
+__global__ __launch_bounds__(256) void gap_tiles_kernel(GapTileArgs ga) {
+    __shared__ double rs[kGapRows][4];
+    __shared__ double red[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c0 = blockIdx.x * kGapCols + 4 * tid, r0 = blockIdx.y * kGapRows;
+    const int rows = min(kGapRows, ga.n_i - r0);
+    const int cl = min(c0, (ga.n_j - 1) & ~3);  // lanes past the last column repeat it and add nothing
+    double gk[4], acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        gk[q] = c0 + q < ga.n_j ? ga.g[c0 + q] * ga.k : -INFINITY;
+        acc[q] = 0.0;
+    }
+    const float *base = ga.C + (int64_t)r0 * ga.ldc + cl;
+    double s_ry = 0.0, s_rc = 0.0;
+    float4 next = load_stream4(base);
+#pragma unroll 2
+    for (int r = 0; r < rows; ++r) {
+        const float4 a4 = next;
+        next = load_stream4(base + (int64_t)min(r + 1, rows - 1) * ga.ldc);
+        const double fk = ga.f[r0 + r] * ga.k;
+        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+        double sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double a = (double)av[q];
+            double y = fma(-ga.k, a, fk + gk[q]);
+            y = y < -1100.0 ? -1100.0 : y;
+            const double R = exp2_f64(y);
+            acc[q] += R;
+            sum += R;
+            s_ry = fma(R, y, s_ry);
+            s_rc = fma(R, a, s_rc);
+        }
+        sum = wave_sum(sum);
+        if (lane == 0) rs[r][wave] = sum;
+    }
+    double *co = ga.col_part + (int64_t)blockIdx.y * ga.n_j;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (c0 + q < ga.n_j) co[c0 + q] = acc[q];
+    s_ry = wave_sum(s_ry);
+    s_rc = wave_sum(s_rc);
+    if (lane == 0) {
+        red[0][wave] = s_ry;
+        red[1][wave] = s_rc;
+    }
+    __syncthreads();
+    if (tid < rows) ga.row_part[(int64_t)blockIdx.x * ga.n_i + r0 + tid] = ((rs[tid][0] + rs[tid][1]) + rs[tid][2]) + rs[tid][3];
+    if (tid < 2) {
+        const double t = ((red[tid][0] + red[tid][1]) + red[tid][2]) + red[tid][3];
+        ga.partials[2 * ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) + tid] = tid == 0 ? t * kLn2 : t;
+    }
+}
+
+// marginal terms of the objectives from the tiles' partials: 64 rows (or, past the row
+// workgroups, columns) per workgroup, four threads each over the partials in order
+struct GapMarginArgs {
+    const double *row_part, *col_part;
+    int n_row_part, n_col_part;
+    const double *f, *g, *G, *misc;
+    int n_i, n_j;
+    double lambda1, lambda2;
+    int row_blocks;
+    double *out;  // [workgroup][3]: penalty, conjugate, sum R
+};
+
+__global__ __launch_bounds__(256) void gap_margins_kernel(GapMarginArgs ga) {
+    __shared__ double red[4][64];
+    const int e = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const bool is_row = (int)blockIdx.x < ga.row_blocks;
+    const int n = is_row ? ga.n_i : ga.n_j, parts = is_row ? ga.n_row_part : ga.n_col_part;
+    const int i = ((int)blockIdx.x - (is_row ? 0 : ga.row_blocks)) * 64 + e;
+    const double *src = (is_row ? ga.row_part : ga.col_part) + i;
+    double s = 0.0;
+    if (i < n) {
+#pragma unroll 4
+        for (int q = part; q < parts; q += 4) s += src[(int64_t)q * n];
+    }
+    red[part][e] = s;
+    __syncthreads();
+    if (part) return;
+    const double r = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    double pen = 0.0, conj = 0.0, sum = 0.0;
+    if (i < n) {
+        const double x = r / (is_row ? ga.n_j : ga.n_i), inv = 1.0 / n;
+        const double p = is_row ? ga.G[i] : ga.misc[1];
+        pen = inv * (x * log(x / p) - x + p);
+        conj = (p * inv) * (exp(is_row ? -ga.f[i] / ga.lambda1 : -ga.g[i] / ga.lambda2) - 1.0);
+        sum = r;
+    }
+    pen = wave_sum(pen);
+    conj = wave_sum(conj);
+    sum = wave_sum(sum);
+    if (e == 0) {
+        ga.out[3 * blockIdx.x] = pen;
+        ga.out[3 * blockIdx.x + 1] = conj;
+        ga.out[3 * blockIdx.x + 2] = sum;
+    }
+}
+
+// [primal, dual, gap] from the margins' and tiles' partials
+__global__ __launch_bounds__(1024) void gap_total_kernel(const double *__restrict__ margins, int row_blocks,
+                                                         int col_blocks, const double *__restrict__ partials,
+                                                         int n_tiles, int n_i, int n_j, double lambda1,
+                                                         double lambda2, double eps, const double *__restrict__ skt_dev,
+                                                         double *__restrict__ out) {
+    __shared__ double red[7][16];
+    double t[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < row_blocks; b += 1024) {
+        t[0] += margins[3 * b];
+        t[2] += margins[3 * b + 1];
+        t[4] += margins[3 * b + 2];
+    }
+    for (int b = threadIdx.x; b < col_blocks; b += 1024) {
+        t[1] += margins[3 * (row_blocks + b)];
+        t[3] += margins[3 * (row_blocks + b) + 1];
+    }
+    for (int b = threadIdx.x; b < n_tiles; b += 1024) {
+        t[5] += partials[2 * b];
+        t[6] += partials[2 * b + 1];
+    }
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+        const double v = wave_sum(t[q]);
+        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int q = 0; q < 7; ++q) {
+        t[q] = 0.0;
+        for (int w = 0; w < 16; ++w) t[q] += red[q][w];
+    }
+    const double skt = *skt_dev, ij = (double)n_i * (double)n_j;
+    const double pri = lambda1 * t[0] + lambda2 * t[1] + (eps * (t[5] - t[4] + skt) + t[6]) / ij;
+    const double dua = -lambda1 * t[2] - lambda2 * t[3] - eps * (t[4] - skt) / ij;
+    out[0] = pri;
+    out[1] = dua;
+    out[2] = (pri - dua) / fabs(pri);
+}
+
 // sum of the K-tilde partials (slot 2 of each block) -> out
 // (one block of 1024 threads; thread t takes blocks t, t + 1024, ...: fixed order)
 __global__ __launch_bounds__(1024) void sum_slot_kernel(const double *__restrict__ partials, int nparts,
@@ -505,7 +760,15 @@ struct Work {
     int nparts;
     float *col_part;  // column partials of the one-read iteration, or nullptr: two sweeps
     void *exchange;   // exchange buffers of the resident solver, or nullptr: launches per sweep
+    // duality-gap schedule
+    unsigned long long *slot;  // growth keys: two iterations in turn, [2] the snapshot's
+    int *skip;                 // set when a batch that runs ahead must not run
+    bool run_ahead = false;    // the iteration's launches look at *skip
+    double *evo;               // partial sums of the evolution check
+    double *gap_rows, *gap_cols, *gap_margins;  // one-read gap pass: partials per tile (with col_part)
 };
+
+constexpr int kEvoBlocks = 64;
 
 // extras: with the buffers of the resident solver or the one-read iteration where the shape takes them
 static size_t carve(Arena &ar, int64_t I, int64_t J, bool extras, Work *w) {
@@ -530,8 +793,18 @@ static size_t carve(Arena &ar, int64_t I, int64_t J, bool extras, Work *w) {
     w->us = ar.take<double>(I4);
     w->vs = ar.take<double>(J4);
     w->counter = ar.take<long long>(4);
+    w->slot = ar.take<unsigned long long>(4);
+    w->skip = ar.take<int>(4);
+    w->evo = ar.take<double>(4 * kEvoBlocks);
     w->col_part = nullptr;
     if (extras && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
+    w->gap_rows = w->gap_cols = w->gap_margins = nullptr;
+    if (w->col_part || (!ar.base && extras && one_pass_fits(I, J))) {
+        const int64_t ti = (I + kGapRows - 1) / kGapRows, tj = (J + kGapCols - 1) / kGapCols;
+        w->gap_rows = ar.take<double>((size_t)tj * I);
+        w->gap_cols = ar.take<double>((size_t)ti * J);
+        w->gap_margins = ar.take<double>((size_t)3 * ((I + 63) / 64 + (J + 63) / 64) + 2 * ti * tj);
+    }
     w->exchange = nullptr;
     if (extras && resident_fits(I, J)) w->exchange = ar.take<char>(resident_bytes(I, J));
     return ar.off;
@@ -554,7 +827,7 @@ static int init_state(const Problem &pb, Work &w, hipStream_t s) {
     fill_pot_kernel<<<(I4 + 255) / 256, 256, 0, s>>>(w.u, pb.n_i, I4, 0.0);
     fill_pot_kernel<<<(J4 + 255) / 256, 256, 0, s>>>(w.v, pb.n_j, J4, 0.0);
     growth_prep_kernel<<<1, 1024, 0, s>>>(pb.G, pb.n_i, w.logp, w.misc);
-    zero_ll_kernel<<<1, 64, 0, s>>>(w.counter, 4);
+    clear_state_kernel<<<1, 64, 0, s>>>(w.counter, w.slot, w.skip);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
 }
@@ -587,10 +860,10 @@ static int launch_lse(const float *A, int64_t lda, int nrows, int ncols, const d
 
 // one (a, b) iteration at eps: f from g over C, then g from f over C^T
 static int iterate(const Problem &pb, Work &w, double lambda1, double lambda2, double eps,
-                   hipStream_t s) {
+                   hipStream_t s, const TauTrack &tau = TauTrack{}) {
     if (w.col_part)
         return one_pass_iterate(OnePass{pb.C, pb.ldc, pb.CT, pb.ldct, pb.n_i, pb.n_j, w.f, w.g, w.logp, w.misc,
-                                        w.col_part},
+                                        w.col_part, tau, w.run_ahead ? w.skip : nullptr},
                                 lambda1, lambda2, eps, s);
     RowEpilogue er{w.logp, nullptr, std::log((double)pb.n_j), lambda1 / (lambda1 + eps), eps, w.f,
                    nullptr};
@@ -625,6 +898,20 @@ int launch_plan_sums(const float *A, int64_t lda, int nrows, int ncols, const do
 // primal/dual/gap at potentials f, g and eps -> w.gapout[0..2] (device)
 static int gap_pass(const Problem &pb, Work &w, const double *f, const double *g, double lambda1,
                     double lambda2, double eps, const double *sum_kt_dev, hipStream_t s) {
+    if (w.gap_rows) {
+        const int ti = (pb.n_i + kGapRows - 1) / kGapRows, tj = (pb.n_j + kGapCols - 1) / kGapCols;
+        const int bi = (pb.n_i + 63) / 64, bj = (pb.n_j + 63) / 64;
+        double *tiles = w.gap_margins + 3 * (bi + bj);
+        const GapTileArgs gt{pb.C, pb.ldc, pb.n_i, pb.n_j, f, g, kLog2E / eps, w.gap_rows, w.gap_cols, tiles};
+        gap_tiles_kernel<<<dim3((unsigned)tj, (unsigned)ti), 256, 0, s>>>(gt);
+        const GapMarginArgs gm{w.gap_rows, w.gap_cols, tj, ti, f, g, pb.G, w.misc, pb.n_i, pb.n_j, lambda1, lambda2,
+                               bi, w.gap_margins};
+        gap_margins_kernel<<<bi + bj, 256, 0, s>>>(gm);
+        gap_total_kernel<<<1, 1024, 0, s>>>(w.gap_margins, bi, bj, tiles, ti * tj, pb.n_i, pb.n_j, lambda1, lambda2,
+                                            eps, sum_kt_dev, w.gapout);
+        WOTK_LAUNCH_CHECK();
+        return WOTK_OK;
+    }
     int rc = launch_plan(pb.C, pb.ldc, pb.n_i, pb.n_j, f, g, eps, 1.0, nullptr, 0, w.r, w.partials, 0, s);
     if (rc) return rc;
     rc = launch_plan(pb.CT, pb.ldct, pb.n_j, pb.n_i, g, f, eps, 1.0, nullptr, 0, w.c, nullptr, 0, s);
@@ -853,7 +1140,8 @@ struct SideStream {
 };
 
 // The duality-gap schedule (optimal_transport.py:67-164) over a backend that
-// owns the cost: B::iterate (one (a, b) iteration on w.f, w.g), B::gap_pass
+// owns the cost: B::iterate (one (a, b) iteration on w.f, w.g; with the tau check
+// inside where B::tracks_growth), B::gap_pass
 // (primal, dual, gap at given potentials -> w.gapout), B::ktilde_sum and
 // B::finish (outputs at eps, plan divided by div).
 template <class B>
@@ -870,18 +1158,31 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
     double *sum_kt = w.misc + 4;
     double inv_eps = 1.0 / eps_i;
     int rc = 0;
-    // one (a, b) iteration plus the tau check (optimal_transport.py:131-141)
+    // one (a, b) iteration plus the tau check (optimal_transport.py:131-141): inside the
+    // iteration where the backend tracks the growth, else a launch of its own
+    int cur = 0;  // growth key of the last iteration
     auto one_iteration = [&](double eps) -> int {
-        int r = be.iterate(lambda1, lambda2, eps, s);
+        if (be.tracks_growth()) {
+            const TauTrack tr{w.slot + cur, w.slot + (cur ^ 1), tau, inv_eps, w.u, w.v, w.counter};
+            cur ^= 1;
+            return be.iterate(lambda1, lambda2, eps, s, tr);
+        }
+        int r = be.iterate(lambda1, lambda2, eps, s, TauTrack{});
         if (r) return r;
         stabilise_kernel<<<1, 1024, 0, s>>>(w.f, w.u, pb.n_i, w.g, w.v, pb.n_j, inv_eps, tau, w.counter);
         WOTK_LAUNCH_CHECK();
         return WOTK_OK;
     };
+    const int vec_blocks = (int)std::min<int64_t>(256, (std::max(pb.n_i, pb.n_j) + 255) / 256);
+    const int evo_blocks = std::min(kEvoBlocks, vec_blocks);
+    SideStream side;
+    WOTK_HIP(hipStreamCreateWithFlags(&side.s, hipStreamNonBlocking));
+    WOTK_HIP(hipEventCreateWithFlags(&side.snap, hipEventDisableTiming));
     // early, un-normalised return (optimal_transport.py:143-145)
     auto max_iter_return = [&](double eps) -> int {
         int r = be.finish(eps, 1.0, s);
         if (r) return r;
+        count_pending_kernel<<<1, 1, 0, s>>>(w.slot + cur, tau, w.counter);
         long long nst = 0;
         WOTK_HIP(hipMemcpyAsync(&nst, w.counter, sizeof(long long), hipMemcpyDeviceToHost, s));
         WOTK_HIP(hipStreamSynchronize(s));
@@ -899,7 +1200,7 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
     for (int e = 0; e <= n_scal; ++e) {
         gap = INFINITY;
         // absorb: with a, b folded into the potentials, u = f and v = g
-        copy2_kernel<<<64, 256, 0, s>>>(w.u, w.f, pb.n_i, w.v, w.g, pb.n_j);
+        scaling_begin_kernel<<<vec_blocks, 256, 0, s>>>(w.u, w.f, pb.n_i, w.v, w.g, pb.n_j, w.skip);
         WOTK_LAUNCH_CHECK();
         eps_i = eps_i / factor;
         inv_eps = 1.0 / eps_i;
@@ -908,27 +1209,63 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
             if (rc) return rc;
         }
         if (e < n_scal) {
-            // dual-variable evolution checks every 5 iterations, threshold 1e-6
-            while (gap > 1e-6) {
-                for (int64_t t = 0; t < 5; ++t) {
-                    ++it;
-                    if (t == 4) {
-                        copy2_kernel<<<64, 256, 0, s>>>(w.fp, w.f, pb.n_i, w.up, w.u, pb.n_i);
-                        copy2_kernel<<<64, 256, 0, s>>>(w.gp, w.g, pb.n_j, w.vp, w.v, pb.n_j);
-                        WOTK_LAUNCH_CHECK();
-                    }
-                    rc = one_iteration(eps_i);
-                    if (rc) return rc;
-                    if (it >= max_iter) return max_iter_return(eps_i);
+            // Dual-variable evolution checks every 5 iterations, threshold 1e-6.  Where the
+            // iteration's launches look at *skip, the next batch is queued before the check's
+            // result is read; a check that ends the scaling sets *skip, and that batch does nothing.
+            w.run_ahead = be.tracks_growth();
+            int out = 4;  // the check's result: two places in turn, one read while the next is written
+            auto batch = [&]() -> int {  // 5 iterations and their check
+                out ^= 1;
+                for (int t = 0; t < 5; ++t) {
+                    if (t == 4)
+                        before_last_kernel<<<vec_blocks, 256, 0, s>>>(w.f, w.u, pb.n_i, w.g, w.v, pb.n_j, w.fp, w.up,
+                                                                      w.gp, w.vp, w.slot + cur, tau, w.skip);
+                    int r = one_iteration(eps_i);
+                    if (r) return r;
                 }
-                ++checks;
-                evolution_kernel<<<1, 1024, 0, s>>>(w.f, w.fp, w.up, w.u, pb.n_i, w.g, w.gp, w.vp, w.v,
-                                                    pb.n_j, inv_eps, w.gapout);
+                evolution_kernel<<<evo_blocks, 256, 0, s>>>(w.f, w.fp, w.up, w.u, pb.n_i, w.g, w.gp, w.vp, w.v,
+                                                            pb.n_j, inv_eps, w.slot + cur, tau, w.skip, w.evo);
+                evolution_finish_kernel<<<1, 64, 0, s>>>(w.evo, evo_blocks, 1e-6, w.skip, w.gapout + out);
                 WOTK_LAUNCH_CHECK();
-                WOTK_HIP(hipMemcpyAsync(host_out, w.gapout, sizeof(double), hipMemcpyDeviceToHost, s));
-                WOTK_HIP(hipStreamSynchronize(s));
+                return WOTK_OK;
+            };
+            bool queued = false;
+            int cur_queued = cur;
+            while (gap > 1e-6) {
+                if (it + 5 >= max_iter) {  // ends inside or after this batch: in step with the host
+                    for (int t = 0; t < 5; ++t) {
+                        ++it;
+                        if (t == 4)
+                            before_last_kernel<<<vec_blocks, 256, 0, s>>>(w.f, w.u, pb.n_i, w.g, w.v, pb.n_j, w.fp,
+                                                                          w.up, w.gp, w.vp, w.slot + cur, tau,
+                                                                          w.skip);
+                        rc = one_iteration(eps_i);
+                        if (rc) return rc;
+                        if (it >= max_iter) return max_iter_return(eps_i);
+                    }
+                }
+                if (!queued) {
+                    rc = batch();
+                    if (rc) return rc;
+                }
+                queued = false;
+                it += 5;
+                ++checks;
+                cur_queued = cur;
+                WOTK_HIP(hipEventRecord(side.snap, s));
+                WOTK_HIP(hipStreamWaitEvent(side.s, side.snap, 0));
+                const double *result = w.gapout + out;
+                if (w.run_ahead && it + 5 < max_iter) {
+                    rc = batch();
+                    if (rc) return rc;
+                    queued = true;
+                }
+                WOTK_HIP(hipMemcpyAsync(host_out, result, sizeof(double), hipMemcpyDeviceToHost, side.s));
+                WOTK_HIP(hipStreamSynchronize(side.s));
                 gap = host_out[0];
             }
+            if (queued) cur = cur_queued;  // the batch ahead did nothing
+            w.run_ahead = false;
             continue;
         }
         // Last scaling: a primal/dual gap pass after every batch of batch_size
@@ -938,10 +1275,7 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
         // that ran ahead is rolled back from the snapshot, so the result is that
         // of the sequential order.  No batch runs ahead when it would reach
         // max_iter (its early return needs the state at max_iter).
-        SideStream side;
-        WOTK_HIP(hipStreamCreateWithFlags(&side.s, hipStreamNonBlocking));
-        WOTK_HIP(hipEventCreateWithFlags(&side.snap, hipEventDisableTiming));
-        const int snap_blocks = (int)std::min<int64_t>(256, (std::max(pb.n_i, pb.n_j) + 255) / 256);
+        int cur_snap = cur;
         int64_t ahead = 0;  // iterations of the batch launched ahead of the last gap check
         while (gap > tolerance) {
             const int64_t nb = batch_size;
@@ -957,8 +1291,9 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
                 }
             }
             ++checks;
-            snapshot_kernel<<<snap_blocks, 256, 0, s>>>(w.f, w.g, w.u, w.v, w.fs, w.gs, w.us, w.vs, pb.n_i,
-                                                        pb.n_j, w.counter, 0);
+            cur_snap = cur;
+            snapshot_kernel<<<vec_blocks, 256, 0, s>>>(w.f, w.g, w.u, w.v, w.fs, w.gs, w.us, w.vs, pb.n_i,
+                                                       pb.n_j, w.counter, w.slot, cur, tau, 0);
             WOTK_LAUNCH_CHECK();
             WOTK_HIP(hipEventRecord(side.snap, s));
             WOTK_HIP(hipStreamWaitEvent(side.s, side.snap, 0));
@@ -976,11 +1311,14 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
             gap = host_out[2];
         }
         if (ahead) {
-            snapshot_kernel<<<snap_blocks, 256, 0, s>>>(w.f, w.g, w.u, w.v, w.fs, w.gs, w.us, w.vs, pb.n_i,
-                                                        pb.n_j, w.counter, 1);
+            cur = cur_snap;
+            snapshot_kernel<<<vec_blocks, 256, 0, s>>>(w.f, w.g, w.u, w.v, w.fs, w.gs, w.us, w.vs, pb.n_i,
+                                                       pb.n_j, w.counter, w.slot, cur, tau, 1);
             WOTK_LAUNCH_CHECK();
         }
     }
+    count_pending_kernel<<<1, 1, 0, s>>>(w.slot + cur, tau, w.counter);
+    WOTK_LAUNCH_CHECK();
     long long nst = 0;
     WOTK_HIP(hipMemcpyAsync(&nst, w.counter, sizeof(long long), hipMemcpyDeviceToHost, s));
     WOTK_HIP(hipStreamSynchronize(s));
@@ -1009,7 +1347,10 @@ struct StoredBackend {
     double *plan;
     int64_t ldp;
     double *row_sums, *f_out, *g_out;
-    int iterate(double l1, double l2, double eps, hipStream_t s) { return wotk::iterate(pb, w, l1, l2, eps, s); }
+    bool tracks_growth() const { return w.col_part != nullptr; }
+    int iterate(double l1, double l2, double eps, hipStream_t s, const TauTrack &tau) {
+        return wotk::iterate(pb, w, l1, l2, eps, s, tau);
+    }
     int gap_pass(const double *f, const double *g, double l1, double l2, double eps, const double *skt,
                  hipStream_t s) {
         return wotk::gap_pass(pb, w, f, g, l1, l2, eps, skt, s);
@@ -1125,7 +1466,8 @@ struct FusedBackend {
     Work &w;
     const FusedProblem &fp;
     double *row_sums, *f_out, *g_out;
-    int iterate(double l1, double l2, double eps, hipStream_t s) {
+    bool tracks_growth() const { return false; }
+    int iterate(double l1, double l2, double eps, hipStream_t s, const TauTrack &) {
         return fused_problem_iterate(fp, w.f, w.g, w.logp, w.misc, l1, l2, eps, s);
     }
     int gap_pass(const double *f, const double *g, double l1, double l2, double eps, const double *skt,
