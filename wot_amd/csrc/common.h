@@ -37,6 +37,46 @@ struct Arena {
     }
 };
 
+#ifdef __HIPCC__
+// 2^x for x in [-1100, inf): x = n + r, exp(r ln 2) by its Taylor series to degree 13
+// (|r ln 2| <= 0.347: remainder under 5e-18), scaled by 2^n.  NaN stays NaN.
+__device__ __forceinline__ double exp2_f64(double x) {
+    const double n = rint(x), t = (x - n) * kLn2;
+    double p = 1.0 / 6227020800.0;
+    p = fma(p, t, 1.0 / 479001600.0);
+    p = fma(p, t, 1.0 / 39916800.0);
+    p = fma(p, t, 1.0 / 3628800.0);
+    p = fma(p, t, 1.0 / 362880.0);
+    p = fma(p, t, 1.0 / 40320.0);
+    p = fma(p, t, 1.0 / 5040.0);
+    p = fma(p, t, 1.0 / 720.0);
+    p = fma(p, t, 1.0 / 120.0);
+    p = fma(p, t, 1.0 / 24.0);
+    p = fma(p, t, 1.0 / 6.0);
+    p = fma(p, t, 0.5);
+    p = fma(p, t, 1.0);
+    p = fma(p, t, 1.0);
+    return ldexp(p, (int)n);
+}
+
+// sums over a wave by DPP, no LDS permutes: row_shr 1, 2, 4, 8, then row_bcast 15 (lanes 31 and
+// 63 hold the sums of their 32 lanes), then row_bcast 31 (lane 63 holds the sum of all)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double half_wave_sum_dpp(double v) {
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    return dpp_add<0x142, 0xa>(v);
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) { return dpp_add<0x143, 0xc>(half_wave_sum_dpp(v)); }
+#endif
+
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // Compiled tile variants of the sweep kernels, (rows per workgroup, threads).

@@ -32,7 +32,12 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kFThreads = 256;
 constexpr int kFusedMaxSplit = 8;        // column splits per sweep, at most
-constexpr int kFusedTargetBlocks = 768;  // 3 waves per SIMD x 1024 SIMDs / 4 waves per block
+constexpr int kFusedTargetBlocks = 768;
+constexpr int kFusedCUs = 256;
+// waves per SIMD (workgroups per CU) that the registers of a wave's rows, two tiles' products
+// and the sums leave room for
+constexpr int fused_waves(int terms, int nks, bool exact) { return nks <= (terms == 3 ? 6 : 4) ? 2 : 1; }
+constexpr int kFusedBoxWords = 16 * kFThreads * (2 * kFusedCUs + 1);  // 8-byte words, FP32 sums
 
 // ---------------------------------------------------------------------------
 // preparation
@@ -50,39 +55,39 @@ __global__ __launch_bounds__(256) void fz_mean_kernel(const double *__restrict__
     if (threadIdx.x == 0) mean[k] = (red[0] + red[1] + red[2] + red[3]) / (n_i + n_j);
 }
 
-// x' = (x - mean) / sqrt(median): FP64 copy, FP64 norm, bf16 split into
-// nterm pieces (hi, mid, lo) with K padded to kp (pitch kp)
-__global__ __launch_bounds__(256) void fz_split_kernel(const double *__restrict__ X, int n, int d, int kp,
+// x' = (x - mean) / sqrt(median): FP64 copy ([d][n]), FP64 norm, bf16 split into
+// npiece pieces (hi, mid, lo), a point's pieces next to each other with K padded
+// to kp; n_pad - n points of zeros behind the last
+__global__ __launch_bounds__(256) void fz_split_kernel(const double *__restrict__ X, int n, int n_pad, int d, int kp,
                                                        const double *__restrict__ mean,
                                                        const double *__restrict__ median, int npiece,
-                                                       __bf16 *__restrict__ p0, __bf16 *__restrict__ p1,
-                                                       __bf16 *__restrict__ p2, double *__restrict__ xs,
+                                                       __bf16 *__restrict__ pieces, double *__restrict__ xs,
                                                        double *__restrict__ norm) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i >= n_pad) return;
     const double sc = 1.0 / sqrt(median[0]);
     double acc = 0.0;
+    __bf16 *out = pieces + (int64_t)i * npiece * kp;
     for (int k = 0; k < kp; ++k) {
-        const double v = k < d ? (X[(int64_t)i * d + k] - mean[k]) * sc : 0.0;
-        if (k < d) xs[(int64_t)i * d + k] = v;
+        const double v = i < n && k < d ? (X[(int64_t)i * d + k] - mean[k]) * sc : 0.0;
+        if (i < n && k < d) xs[(int64_t)k * n + i] = v;
         acc = fma(v, v, acc);
         const __bf16 h = (__bf16)(float)v;
         const double r1 = v - (double)(float)h;
         const __bf16 m = (__bf16)(float)r1;
         const double r2 = r1 - (double)(float)m;
-        p0[(int64_t)i * kp + k] = h;
-        p1[(int64_t)i * kp + k] = m;
-        if (npiece > 2) p2[(int64_t)i * kp + k] = (__bf16)(float)r2;
+        out[k] = h;
+        out[kp + k] = m;
+        if (npiece > 2) out[2 * kp + k] = (__bf16)(float)r2;
     }
-    norm[i] = acc;
+    if (i < n) norm[i] = acc;
 }
 
 // ---------------------------------------------------------------------------
 // fused sweep: row LSE over recomputed cost tiles, potential update epilogue
 // ---------------------------------------------------------------------------
 struct FusedArgs {
-    const __bf16 *A0, *A1, *A2;  // row points, pitch kp
-    const __bf16 *B0, *B1, *B2;  // column points, pitch kp
+    const __bf16 *A, *B;         // row and column points, pieces [point][piece][kp]
     const double *na, *nb;       // squared norms of the scaled coordinates
     int n_rows, n_cols, kp;
     const double *h;             // column potentials
@@ -90,256 +95,451 @@ struct FusedArgs {
     const double *logw;          // per-row log weight or nullptr -> *logw_dev
     const double *logw_dev;
     double log_n_other, alpha, eps, k;
-    int *bad_list;               // rows whose fixed-shift sum under/overflowed
-    int *n_bad;
     double *row_sums;            // row-sum mode: write sum_j R_ij / rs_div, leave pot unchanged
-    double *part;                // column split (gridDim.y > 1): per-split row sums, split-major
+    double *part;                // row sums per column split, split-major
     double rs_div;               // row-sum mode divisor (n_cols: rows of R / J; 1: of R)
+    int row_blocks, n_split, per_split, n_tiles;  // units: 128 rows x one split's column tiles
+    int whole;                   // one unit per workgroup; else an equal run of tiles each
+    unsigned long long *box;     // [workgroup][word][thread]: partial sums handed to the next workgroup
+    unsigned tag;                // this launch's mark on them
 };
 
-// Row epilogue of a sweep from the row's fixed-shift sum S: new potential
-// (or the plan's row sum in row-sum mode); rows whose sum under/overflowed
-// are queued for the repair kernel (a NaN sum leaves the row as it is).
-__device__ inline void fused_row_epilogue(const FusedArgs &fa, int row, double S) {
-    const double f_old = fa.pot[row];
-    if (isnan(S)) {  // NaN inputs (e.g. a NaN growth entry) propagate as in the reference's arithmetic
-        if (fa.row_sums) fa.row_sums[row] = S;
-        else fa.pot[row] = S;
-        return;
-    }
-    if (!(S > 0.0) || isinf(S)) {
-        fa.bad_list[atomicAdd(fa.n_bad, 1)] = row;
-        return;
-    }
-    if (fa.row_sums) {  // the shift is the final potential: S = sum_j R_ij
-        fa.row_sums[row] = S / fa.rs_div;
-        return;
-    }
-    const double lse = log(S) - f_old / fa.eps;  // ln sum_j exp((h_j - C_ij)/eps)
-    const double lw = fa.logw ? fa.logw[row] : *fa.logw_dev;
-    fa.pot[row] = fa.alpha * fa.eps * (lw + fa.log_n_other - lse);
+// tiles of the units, split-major, rows next: unit (x, y) starts at first_tile
+struct FusedUnit {
+    int x, t0, len;
+    int64_t first;
+    int y;
+};
+__device__ __forceinline__ FusedUnit fused_unit(const FusedArgs &fa, int64_t pos) {
+    FusedUnit u;
+    const int64_t per = (int64_t)fa.row_blocks * fa.per_split;
+    u.y = (int)(pos / per);
+    u.t0 = u.y * fa.per_split;
+    u.len = min(fa.per_split, fa.n_tiles - u.t0);
+    u.x = (int)((pos - u.y * per) / u.len);
+    u.first = u.y * per + (int64_t)u.x * u.len;
+    return u;
 }
 
+// Partial sums passed between workgroups: 32 bits of value and the launch's mark
+// in one 8-byte word, so a word is either whole or not yet there and no fence is
+// needed.  The wait is bounded: after kFusedPolls looks (about 0.2 ms) the caller
+// computes the missing part itself, so progress never depends on which workgroups
+// the chip holds at once.
+constexpr int kFusedPolls = 128;
+__device__ __forceinline__ unsigned long long fused_word(unsigned v, unsigned tag) {
+    return (unsigned long long)tag << 32 | v;
+}
+template <typename T>
+__device__ __forceinline__ void fused_send(unsigned long long *box, unsigned tag, const T (&s)[16]) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if constexpr (sizeof(T) == 4) {
+            __hip_atomic_store(box + r * kFThreads, fused_word(__float_as_uint(s[r]), tag),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            __hip_atomic_store(box + (2 * r) * kFThreads,
+                               fused_word((unsigned)__double2loint(s[r]), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(box + (2 * r + 1) * kFThreads,
+                               fused_word((unsigned)__double2hiint(s[r]), tag), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+template <typename T>
+__device__ __forceinline__ bool fused_take(unsigned long long *box, unsigned tag, T (&s)[16]) {
+    constexpr int W = sizeof(T) / 4;
+    for (int q = 0; q < kFusedPolls; ++q) {
+        bool there = true;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            unsigned v[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const unsigned long long m = __hip_atomic_load(box + (W * r + w) * kFThreads,
+                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                there = there && (unsigned)(m >> 32) == tag;
+                v[w] = (unsigned)m;
+            }
+            if constexpr (W == 1) s[r] = __uint_as_float(v[0]);
+            else s[r] = __hiloint2double((int)v[1], (int)v[0]);
+        }
+        if (__syncthreads_and(there)) return true;
+    }
+    return false;
+}
+
+// 128 rows (32 per wave) x a run of 32-column tiles.  Bound: the matrix cores at the clock they
+// sustain.  A tile of a wave takes TERMS * NKS MFMAs and 8 vector instructions for each of its 16
+// entries per lane; with 6 terms at d = 50 the products alone (no exponentials) take 383 us of a
+// 24576 x 24576 sweep's 393 (1.2 PFLOP/s of padded products, what a large bf16 product reaches).
+// So both are in the loop body at once, the products of tile t beside the exponentials of tile
+// t - 1 (six stages of four entries, each behind an MFMA); one after the other, with the next
+// tile's constants waited for at its start, a sweep took 463 us.  Kept out: three waves per SIMD
+// without the overlap (434), column tiles by DMA to LDS two at a time (425).
+// Work: the tiles of all units (128 rows x one column split) are dealt out in equal runs, one per
+// resident workgroup: 20000 x 20000 has 785 units for 512 places, 291 us as equal runs and 329 as
+// whole units in turn.  A run that ends inside a unit leaves the lanes' sums to the next workgroup,
+// which goes on from them, so the sums are bit for bit those of one workgroup per unit.  Each
+// workgroup takes its last unit (whose rest another waits for) first and the unit it continues last.
 // EXACT: FP64 exponential (exp2 of the FP64 exponent) and FP64 lane sums, for
 // the row and column sums of the duality-gap pass; otherwise v_exp_f32 of the
 // exponent rounded to FP32 and FP32 lane sums (the sweeps)
-template <int TERMS, int NKS, bool EXACT = false>
-__global__ __launch_bounds__(kFThreads) void fused_lse_kernel(FusedArgs fa) {
+template <int TERMS, int NKS, bool EXACT>
+__global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS, EXACT)) void fused_lse_kernel(FusedArgs fa) {
     constexpr int NP = TERMS == 3 ? 2 : 3;  // pieces per point
     constexpr int KP = NKS * 16;
-    constexpr int PITCH = KP + 8;            // 16-byte pad: spreads lanes over LDS banks
-    constexpr int TILE = NP * 32 * PITCH;
-    __shared__ __bf16 bsh[2 * TILE];         // double-buffered column tile
+    constexpr int CHUNKS = NP * KP / 8;      // 16-byte chunks per point
+    constexpr int PITCH = NP * KP + 8;       // an odd number of chunks: conflict-free 16-byte reads
+    constexpr int NCHUNK = (32 * CHUNKS + kFThreads - 1) / kFThreads;
+    constexpr bool RAGGED = 32 * CHUNKS % kFThreads != 0;
+    using acc_t = typename std::conditional<EXACT, double, float>::type;
+    __shared__ __bf16 bsh[2][32 * PITCH];    // double-buffered column tile
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, kg = (lane >> 5) * 8;
-    const int r0 = blockIdx.x * 128 + wave * 32;
-    const __bf16 *Ap[3] = {fa.A0, fa.A1, fa.A2};
-    const __bf16 *Bp[3] = {fa.B0, fa.B1, fa.B2};
-
-    // row constants for this lane's 16 accumulator rows: (f_old - |x'|^2) * k
-    double wf[16];
-    using acc_t = typename std::conditional<EXACT, double, float>::type;
-    acc_t s[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = min(r0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4), fa.n_rows - 1);
-        wf[r] = (fa.pot[row] - fa.na[row]) * fa.k;
-        s[r] = 0.f;
-    }
-    // this wave's 32 rows stay in registers for the whole sweep
-    const int arow = min(r0 + lr, fa.n_rows - 1);
-    bf16x8 afr[NKS][NP];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-            afr[ks][p] = *reinterpret_cast<const bf16x8 *>(Ap[p] + (int64_t)arow * KP + ks * 16 + kg);
     const double k2 = 2.0 * fa.k;
 
-    // column tiles stream through two LDS buffers: the next tile's global
-    // loads are issued into registers before the current tile's MFMA and
-    // exponentials, and written to LDS only afterwards, so the load latency
-    // hides behind the compute
-    constexpr int PER_PIECE = 32 * KP / 8;                       // bf16x8 chunks per piece
-    constexpr int NCHUNK = (NP * PER_PIECE + kFThreads - 1) / kFThreads;
-    bf16x8 stage[NCHUNK];
-    auto fetch = [&](int c0) {
-#pragma unroll
-        for (int u = 0; u < NCHUNK; ++u) {
-            const int e = tid + u * kFThreads;
-            if (e < NP * PER_PIECE) {
-                const int p = e / PER_PIECE, rem = e % PER_PIECE;
-                const int col = rem / (KP / 8), kk = (rem % (KP / 8)) * 8;
-                const int gcol = min(c0 + col, fa.n_cols - 1);
-                stage[u] = *reinterpret_cast<const bf16x8 *>(Bp[p] + (int64_t)gcol * KP + kk);
-            }
-        }
-    };
-    auto commit = [&](int buf) {
-#pragma unroll
-        for (int u = 0; u < NCHUNK; ++u) {
-            const int e = tid + u * kFThreads;
-            if (e < NP * PER_PIECE) {
-                const int p = e / PER_PIECE, rem = e % PER_PIECE;
-                const int col = rem / (KP / 8), kk = (rem % (KP / 8)) * 8;
-                *reinterpret_cast<bf16x8 *>(bsh + buf * TILE + (p * 32 + col) * PITCH + kk) = stage[u];
-            }
-        }
-    };
+    const int64_t total = (int64_t)fa.row_blocks * fa.n_tiles;
+    int64_t lo, hi;
+    if (fa.whole) {
+        const int y = (int)blockIdx.x / fa.row_blocks, x = (int)blockIdx.x % fa.row_blocks;
+        const int len = min(fa.per_split, fa.n_tiles - y * fa.per_split);
+        lo = (int64_t)fa.row_blocks * fa.per_split * y + (int64_t)x * len;
+        hi = lo + len;
+    } else {
+        lo = total * blockIdx.x / gridDim.x;
+        hi = total * (blockIdx.x + 1) / gridDim.x;
+    }
 
-    // column split: block (x, y) takes the column tiles [t_begin, t_end) of its rows
-    const int ntiles_all = (fa.n_cols + 31) / 32;
-    const int per_split = (ntiles_all + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int t_begin = min(ntiles_all, (int)blockIdx.y * per_split);
-    const int t_end = min(ntiles_all, t_begin + per_split);
-    auto col_const = [&](int t, double &hv, double &nv) {  // this lane's column of tile t
-        const int col = min(t * 32 + lr, fa.n_cols - 1);
-        hv = fa.h[col];
-        nv = fa.nb[col];
-    };
-    double h_cur, n_cur, h_nxt = 0.0, n_nxt = 0.0;
-    col_const(t_begin, h_cur, n_cur);
-    fetch(t_begin * 32);
-    commit(0);
-    __syncthreads();
-    for (int t = t_begin; t < t_end; ++t) {
-        const int buf = (t - t_begin) & 1;
-        if (t + 1 < t_end) {
-            fetch((t + 1) * 32);
-            col_const(t + 1, h_nxt, n_nxt);
+    constexpr int kWords = 16 * kFThreads * (EXACT ? 2 : 1);
+    while (hi > lo) {
+        const FusedUnit un = fused_unit(fa, hi - 1);
+        const int64_t begin = max(un.first, lo);
+        int ta = un.t0 + (int)(begin - un.first);
+        const int tb = un.t0 + (int)(hi - un.first);
+        const bool ends = hi == un.first + un.len;
+        hi = begin;
+
+        // row constants for this lane's 16 accumulator rows: (f_old - |x'|^2) * k
+        const int r0 = un.x * 128 + wave * 32;
+        double wf[16];
+        acc_t s[16];
+        bool taken = false;
+        if (begin > un.first) {
+            int64_t at = (int64_t)blockIdx.x * kWords + tid;
+            asm volatile("" : "+v"(at));  // the words' 16 addresses are not kept in registers over the tiles
+            taken = fused_take(fa.box + at, fa.tag, s);
+            if (!taken) ta = un.t0;
         }
-        floatx16 acc, acc2;  // two independent accumulation chains
+        if (!taken) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 0;
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            acc[r] = 0.f;
-            acc2[r] = 0.f;
+            const int row = min(r0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4), fa.n_rows - 1);
+            wf[r] = (fa.pot[row] - fa.na[row]) * fa.k;
         }
-        const __bf16 *bt = bsh + buf * TILE;
+        // this wave's 32 rows stay in registers
+        bf16x8 afr[NKS][NP];
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const int ko = ks * 16 + kg;
-            bf16x8 b[NP];
+        for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-            for (int p = 0; p < NP; ++p) b[p] = *reinterpret_cast<const bf16x8 *>(bt + (p * 32 + lr) * PITCH + ko);
-            const bf16x8 *a = afr[ks];
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc2, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc2, 0, 0, 0);
-            if (TERMS == 6) {
-                acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[NP - 1], acc2, 0, 0, 0);
-                acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[NP - 1], b[0], acc2, 0, 0, 0);
-                acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc2, 0, 0, 0);
+            for (int p = 0; p < NP; ++p)
+                afr[ks][p] = *reinterpret_cast<const bf16x8 *>(fa.A + ((int64_t)(r0 + lr) * NP + p) * KP + ks * 16 + kg);
+
+        // column tiles stream through two LDS buffers: the next tile's global loads are issued
+        // before this tile's products and written to LDS after them
+        bf16x8 stage[NCHUNK];
+        double h_next, nb_next;
+        int col_next;
+        auto fetch = [&](int t) {
+            const __bf16 *src = fa.B + (int64_t)t * 32 * NP * KP;
+#pragma unroll
+            for (int u = 0; u < NCHUNK; ++u) {
+                const int e = RAGGED ? min(tid + u * kFThreads, 32 * CHUNKS - 1) : tid + u * kFThreads;
+                stage[u] = *reinterpret_cast<const bf16x8 *>(src + 8 * e);
             }
-        }
-        const int col = t * 32 + lr;
-        if (col < fa.n_cols) {
-            const double uc = (h_cur - n_cur) * fa.k;
+            col_next = t * 32 + lr;
+            const int c = min(col_next, fa.n_cols - 1);
+            h_next = fa.h[c];
+            nb_next = fa.nb[c];
+        };
+        // h - |y'|^2 of the fetched tile's column; columns past the last add exp(-inf) = 0
+        auto col_const = [&]() { return col_next < fa.n_cols ? h_next - nb_next : -INFINITY; };
+        auto commit = [&](int buf) {
+#pragma unroll
+            for (int u = 0; u < NCHUNK; ++u) {
+                const int e = RAGGED ? min(tid + u * kFThreads, 32 * CHUNKS - 1) : tid + u * kFThreads;
+                *reinterpret_cast<bf16x8 *>(&bsh[buf][(e / CHUNKS) * PITCH + (e % CHUNKS) * 8]) = stage[u];
+            }
+        };
+        auto read_b = [&](int buf, int ks, bf16x8 (&b)[NP]) {
+            const __bf16 *bt = &bsh[buf][lr * PITCH + ks * 16 + kg];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) b[p] = *reinterpret_cast<const bf16x8 *>(bt + p * KP);
+        };
+        // product m of a K step: hi.hi in p0, the smaller ones in p1
+        auto product = [&](int m, const bf16x8 *a, const bf16x8 (&b)[NP], floatx16 &p0, floatx16 &p1) {
+            if (m == 0) p0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], p0, 0, 0, 0);
+            if (m == 1) p1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], p1, 0, 0, 0);
+            if (m == 2) p1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], p1, 0, 0, 0);
+            if (m == 3) p1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[NP - 1], p1, 0, 0, 0);
+            if (m == 4) p1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[NP - 1], b[0], p1, 0, 0, 0);
+            if (m == 5) p1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], p1, 0, 0, 0);
+        };
+        // 6 terms: the chains added in FP64; 3 terms (2^-16 of the cross term already
+        // lost to the missing products): one FP32 add and one widening
+        auto add_entries = [&](const floatx16 &p0, const floatx16 &p1, double d) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                // 6 terms: the chains added in FP64; 3 terms (2^-16 of the cross term already
-                // lost to the missing products): one FP32 add and one widening
-                const double xy = TERMS == 6 ? (double)acc[r] + (double)acc2[r] : (double)(acc[r] + acc2[r]);
-                const double y = fma(k2, xy, uc + wf[r]);
-                if constexpr (EXACT)
-                    s[r] += exp2(y);
-                else
+                const double xy = TERMS == 6 ? (double)p0[r] + (double)p1[r] : (double)(p0[r] + p1[r]);
+                const double y = fma(k2, xy, fma(fa.k, d, wf[r]));
+                if constexpr (EXACT) {
+                    const double z = y < -1100.0 ? -1100.0 : y;
+                    s[r] += exp2_f64(z > 2000.0 ? 2000.0 : z);
+                } else {
                     s[r] += __builtin_amdgcn_exp2f((float)y);
+                }
             }
-        }
-        if (t + 1 < t_end) commit(buf ^ 1);  // the other buffer was released by the previous barrier
-        h_cur = h_nxt;
-        n_cur = n_nxt;
+        };
+        // tile t's products into (n0, n1) beside the exponentials of tile t - 1 in (o0, o1): per K
+        // step its share of the 16 entries in six stages, one or two behind each MFMA
+        auto step = [&](int buf, floatx16 &n0, floatx16 &n1, const floatx16 &o0, const floatx16 &o1, double d) {
+            bf16x8 b[2][NP];
+            read_b(buf, 0, b[0]);
+            n0 = floatx16{};
+            n1 = floatx16{};
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                constexpr int kMost = (16 + NKS - 1) / NKS;
+                const int rb = 16 * ks / NKS, re = 16 * (ks + 1) / NKS;
+                if (ks + 1 < NKS) read_b(buf, ks + 1, b[(ks + 1) & 1]);
+                double u[kMost], v[kMost];
+                float e[kMost];
+#pragma unroll
+                for (int m = 0; m < TERMS; ++m) {
+                    product(m, afr[ks], b[ks & 1], n0, n1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int st = 6 * m / TERMS; st < 6 * (m + 1) / TERMS; ++st) {
+#pragma unroll
+                        for (int r = rb; r < re; ++r) {
+                            const int i = r - rb;
+                            if (st == 0) u[i] = TERMS == 6 ? (double)o0[r] : (double)(o0[r] + o1[r]);
+                            if (st == 1 && TERMS == 6) v[i] = (double)o1[r];
+                            if (st == 2 && TERMS == 6) u[i] = u[i] + v[i];
+                            if (st == 2) v[i] = fma(fa.k, d, wf[r]);
+                            if (st == 3) v[i] = fma(k2, u[i], v[i]);
+                            if (st == 4) e[i] = (float)v[i];
+                            if (st == 4) e[i] = __builtin_amdgcn_exp2f(e[i]);
+                            if (st == 5) s[r] += (acc_t)e[i];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        };
+        floatx16 pa0, pa1, pb0, pb1;
+        __syncthreads();  // the buffers are free
+        fetch(ta);
+        commit(0);
+        double d_old = col_const(), d_cur;
         __syncthreads();
-    }
-    // sum over the 32 lanes that share a row set
-    double sd[16];
+        if constexpr (EXACT) {  // 28 FP64 instructions per entry: the products are the smaller part
+            for (int t = ta; t < tb; ++t) {
+                const int buf = (t - ta) & 1;
+                fetch(min(t + 1, tb - 1));
+                pa0 = floatx16{};
+                pa1 = floatx16{};
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        double v = (double)s[r];
+                for (int ks = 0; ks < NKS; ++ks) {
+                    bf16x8 b[NP];
+                    read_b(buf, ks, b);
 #pragma unroll
-        for (int off = 1; off < 32; off <<= 1) v += __shfl_xor(v, off);
-        sd[r] = v;
-    }
-    if (lr == 0) {
+                    for (int m = 0; m < TERMS; ++m) product(m, afr[ks], b, pa0, pa1);
+                }
+                add_entries(pa0, pa1, d_old);
+                commit(buf ^ 1);
+                d_old = col_const();
+                __syncthreads();
+            }
+        } else {
+            fetch(min(ta + 1, tb - 1));
+            pa0 = floatx16{};
+            pa1 = floatx16{};
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                bf16x8 b[NP];
+                read_b(0, ks, b);
+#pragma unroll
+                for (int m = 0; m < TERMS; ++m) product(m, afr[ks], b, pa0, pa1);
+            }
+            commit(1);
+            d_cur = col_const();
+            __syncthreads();
+            auto turn = [&](int t, floatx16 &n0, floatx16 &n1, const floatx16 &o0, const floatx16 &o1) {
+                const int buf = (t - ta) & 1;
+                fetch(min(t + 1, tb - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                step(buf, n0, n1, o0, o1, d_old);
+                commit(buf ^ 1);
+                d_old = d_cur;
+                d_cur = col_const();
+                __syncthreads();
+            };
+            int t = ta + 1;
+            for (; t + 1 < tb; t += 2) {
+                turn(t, pb0, pb1, pa0, pa1);
+                turn(t + 1, pa0, pa1, pb0, pb1);
+            }
+            if (t < tb) {
+                turn(t, pb0, pb1, pa0, pa1);
+                pa0 = pb0;
+                pa1 = pb1;
+            }
+            add_entries(pa0, pa1, d_old);
+        }
+
+        if (!ends) {
+            int64_t at = ((int64_t)blockIdx.x + 1) * kWords + tid;
+            asm volatile("" : "+v"(at));
+            fused_send(fa.box + at, fa.tag, s);
+            continue;
+        }
+        // sum over the 32 lanes that share a row set
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
+            const double v = half_wave_sum_dpp((double)s[r]);
             const int row = r0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-            if (row >= fa.n_rows) continue;
-            if (gridDim.y > 1) fa.part[(int64_t)blockIdx.y * fa.n_rows + row] = sd[r];
-            else fused_row_epilogue(fa, row, sd[r]);
+            if (lr == 31 && row < fa.n_rows) fa.part[(int64_t)un.y * fa.n_rows + row] = v;
         }
     }
 }
 
-// column-split sweeps: the splits' row sums added in a fixed order, then the
-// row epilogue
-__global__ __launch_bounds__(256) void fused_finalize_kernel(FusedArgs fa, int n_split) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= fa.n_rows) return;
-    double S = 0.0;
-    for (int q = 0; q < n_split; ++q) S += fa.part[(int64_t)q * fa.n_rows + row];
-    fused_row_epilogue(fa, row, S);
-}
+// From the rows' fixed-shift sums S (the splits' added in order): the new potential, or the
+// plan's row sum in row-sum mode.  A NaN sum propagates as in the reference's arithmetic.  Rows
+// whose sum under- or overflowed are computed again by their workgroup from FP64 direct
+// distances of the scaled coordinates ([d][n], read coalesced) with a per-lane online maximum.
+// Such a row costs one read of all column points through one CU (8 MB at 20000 x 50), so up to
+// four share it.  One launch behind a sweep; clearing a list, adding the splits and repairing by
+// three took 20 us of a sweep at 20000 x 20000, this takes 6.
+constexpr int kFinishRows = 32, kFinishThreads = 1024, kFinishWaves = kFinishThreads / 64, kRepairRows = 4;
 
-// repair: rows whose fixed-shift sum under/overflowed, from FP64 direct
-// distances of the scaled coordinates with a per-lane online maximum
-__global__ __launch_bounds__(256) void fused_repair_kernel(const int *__restrict__ bad_list, const int *__restrict__ n_bad,
-                                                           const double *__restrict__ xr, const double *__restrict__ xc,
-                                                           int n_cols, int d, const double *__restrict__ h,
-                                                           double *__restrict__ pot, const double *__restrict__ logw,
-                                                           const double *__restrict__ logw_dev, double log_n_other,
-                                                           double alpha, double eps, double k,
-                                                           double *__restrict__ row_sums, double rs_div) {
-    __shared__ double sg_sh[4], sd_sh[4];
-    const int nb = *n_bad;
-    for (int q = blockIdx.x; q < nb; q += gridDim.x) {
-        const int row = bad_list[q];
-        double sg = -1.0e6, sd = 0.0;
-        for (int j = threadIdx.x; j < n_cols; j += blockDim.x) {
-            double c = 0.0;
-            for (int t = 0; t < d; ++t) {
-                const double z = xr[(int64_t)row * d + t] - xc[(int64_t)j * d + t];
-                c = fma(z, z, c);
+template <int NB>
+__device__ void repair_rows(const FusedArgs &fa, const int *rows, const double *__restrict__ xr,
+                            const double *__restrict__ xc, int d, double (*x_sh)[kRepairRows],
+                            double (*sg_sh)[kFinishWaves], double (*sd_sh)[kFinishWaves]) {
+    const int tid = threadIdx.x;
+    for (int e = tid; e < d * NB; e += kFinishThreads) x_sh[e / NB][e % NB] = xr[(int64_t)(e / NB) * fa.n_rows + rows[e % NB]];
+    __syncthreads();
+    double sg[NB], sd[NB];
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+        sg[q] = -1.0e6;
+        sd[q] = 0.0;
+    }
+    for (int j = tid; j < fa.n_cols; j += kFinishThreads) {
+        double c[NB];
+#pragma unroll
+        for (int q = 0; q < NB; ++q) c[q] = 0.0;
+        for (int t0 = 0; t0 < d; t0 += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = xc[(int64_t)min(t0 + u, d - 1) * fa.n_cols + j];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (t0 + u >= d) continue;  // uniform
+#pragma unroll
+                for (int q = 0; q < NB; ++q) {
+                    const double z = x_sh[t0 + u][q] - v[u];
+                    c[q] = fma(z, z, c[q]);
+                }
             }
-            const double y = (h[j] - c) * k;
-            if (y > sg) {
+        }
+        const double hj = fa.h[j];
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const double y = (hj - c[q]) * fa.k;
+            if (y > sg[q]) {
                 const double ns = ceil(y);
-                sd = ldexp(sd, (int)(sg - ns));
-                sg = ns;
+                sd[q] = ldexp(sd[q], (int)(sg[q] - ns));
+                sg[q] = ns;
             }
-            sd += exp2(y - sg);
+            sd[q] += exp2(y - sg[q]);
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            const double og = __shfl_xor(sg, off), os = __shfl_xor(sd, off);
-            const double ng = fmax(sg, og);
-            sd = ldexp(sd, (int)(sg - ng)) + ldexp(os, (int)(og - ng));
-            sg = ng;
-        }
-        if ((threadIdx.x & 63) == 0) {
-            sg_sh[threadIdx.x >> 6] = sg;
-            sd_sh[threadIdx.x >> 6] = sd;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double g = sg_sh[0], s = sd_sh[0];
-            for (int w = 1; w < 4; ++w) {
-                const double ng = fmax(g, sg_sh[w]);
-                s = ldexp(s, (int)(g - ng)) + ldexp(sd_sh[w], (int)(sg_sh[w] - ng));
-                g = ng;
-            }
-            const double lse = (g + log2(s)) * kLn2;
-            if (row_sums) {
-                row_sums[row] = exp(pot[row] / eps + lse) / rs_div;
-            } else {
-                const double lw = logw ? logw[row] : *logw_dev;
-                pot[row] = alpha * eps * (lw + log_n_other - lse);
-            }
-        }
-        __syncthreads();
     }
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+        for (int off = 32; off > 0; off >>= 1) {
+            const double og = __shfl_xor(sg[q], off), os = __shfl_xor(sd[q], off);
+            const double ng = fmax(sg[q], og);
+            sd[q] = ldexp(sd[q], (int)(sg[q] - ng)) + ldexp(os, (int)(og - ng));
+            sg[q] = ng;
+        }
+        if ((tid & 63) == 0) {
+            sg_sh[q][tid >> 6] = sg[q];
+            sd_sh[q][tid >> 6] = sd[q];
+        }
+    }
+    __syncthreads();
+    if (tid < NB) {
+        double g = sg_sh[tid][0], v = sd_sh[tid][0];
+        for (int w = 1; w < kFinishWaves; ++w) {
+            const double ng = fmax(g, sg_sh[tid][w]);
+            v = ldexp(v, (int)(g - ng)) + ldexp(sd_sh[tid][w], (int)(sg_sh[tid][w] - ng));
+            g = ng;
+        }
+        const double lse = (g + log2(v)) * kLn2;
+        const int row = rows[tid];
+        if (fa.row_sums) {
+            fa.row_sums[row] = exp(fa.pot[row] / fa.eps + lse) / fa.rs_div;
+        } else {
+            const double lw = fa.logw ? fa.logw[row] : *fa.logw_dev;
+            fa.pot[row] = fa.alpha * fa.eps * (lw + fa.log_n_other - lse);
+        }
+    }
+    __syncthreads();
 }
 
-__global__ void fused_clear_kernel(int *n_bad) { *n_bad = 0; }
+__global__ __launch_bounds__(kFinishThreads) void fused_finish_kernel(FusedArgs fa, const double *__restrict__ xr,
+                                                                      const double *__restrict__ xc, int d) {
+    __shared__ double x_sh[128][kRepairRows];
+    __shared__ double sg_sh[kRepairRows][kFinishWaves], sd_sh[kRepairRows][kFinishWaves];
+    __shared__ int bad[kFinishRows];
+    __shared__ int n_bad;
+    const int tid = threadIdx.x;
+    if (tid == 0) n_bad = 0;
+    __syncthreads();
+    const int row = blockIdx.x * kFinishRows + tid;
+    if (tid < kFinishRows && row < fa.n_rows) {
+        double S = 0.0;
+        for (int q = 0; q < fa.n_split; ++q) S += fa.part[(int64_t)q * fa.n_rows + row];
+        if (isnan(S)) {
+            if (fa.row_sums) fa.row_sums[row] = S;
+            else fa.pot[row] = S;
+        } else if (!(S > 0.0) || isinf(S)) {
+            bad[atomicAdd(&n_bad, 1)] = row;
+        } else if (fa.row_sums) {  // the shift is the final potential: S = sum_j R_ij
+            fa.row_sums[row] = S / fa.rs_div;
+        } else {
+            const double lse = log(S) - fa.pot[row] / fa.eps;  // ln sum_j exp((h_j - C_ij)/eps)
+            const double lw = fa.logw ? fa.logw[row] : *fa.logw_dev;
+            fa.pot[row] = fa.alpha * fa.eps * (lw + fa.log_n_other - lse);
+        }
+    }
+    __syncthreads();
+    int q = 0;
+    for (; q + 1 < n_bad; q += kRepairRows) {
+        // a short batch repeats its last row
+        __shared__ int batch[kRepairRows];
+        if (tid < kRepairRows) batch[tid] = bad[min(q + tid, n_bad - 1)];
+        __syncthreads();
+        repair_rows<kRepairRows>(fa, batch, xr, xc, d, x_sh, sg_sh, sd_sh);
+    }
+    if (q < n_bad) repair_rows<1>(fa, bad + q, xr, xc, d, x_sh, sg_sh, sd_sh);
+}
 
 __global__ __launch_bounds__(1024) void fz_growth_kernel(const double *__restrict__ G, int n, double *__restrict__ logp,
                                                          double *__restrict__ misc) {
@@ -363,8 +563,8 @@ __global__ void fz_zero_kernel(double *x, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) x[i] = 0.0;
 }
 
-// column splits per sweep: enough blocks for ~3 waves per SIMD (the kernel
-// holds 166 VGPRs), at least 8 column tiles per split
+// Column splits per sweep: 768 units of 128 rows x one split if the columns give as many, at least
+// 8 column tiles and at most kFusedMaxSplit splits
 static int fused_splits(int n_rows, int n_cols) {
     const int blocks = (n_rows + 127) / 128;
     const int ntiles = (n_cols + 31) / 32;
@@ -372,32 +572,41 @@ static int fused_splits(int n_rows, int n_cols) {
     return std::max(1, std::min(std::min(want, kFusedMaxSplit), ntiles / 8));
 }
 
-template <int TERMS, bool EXACT>
-static void launch_fused(const FusedArgs &fa, int n_split, hipStream_t s) {
-    const dim3 grid((unsigned)((fa.n_rows + 127) / 128), (unsigned)n_split);
-    switch (fa.kp / 16) {
-        case 1: fused_lse_kernel<TERMS, 1, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 2: fused_lse_kernel<TERMS, 2, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 3: fused_lse_kernel<TERMS, 3, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 4: fused_lse_kernel<TERMS, 4, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 5: fused_lse_kernel<TERMS, 5, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 6: fused_lse_kernel<TERMS, 6, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        case 7: fused_lse_kernel<TERMS, 7, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-        default: fused_lse_kernel<TERMS, 8, EXACT><<<grid, kFThreads, 0, s>>>(fa); break;
-    }
+template <int TERMS, int NKS, bool EXACT>
+static void launch_fused(FusedArgs fa, hipStream_t s) {
+    // equal runs once every place has a unit (568 units: 79 us, as whole units 82); below that cutting
+    // only adds hand-overs (376 units on 256 places: 49 us, whole units 42)
+    const int units = fa.row_blocks * fa.n_split;
+    const int resident = kFusedCUs * fused_waves(TERMS, NKS, EXACT);
+    const int grid = std::min(units, resident);
+    fa.whole = units == grid;
+    fused_lse_kernel<TERMS, NKS, EXACT><<<(unsigned)grid, kFThreads, 0, s>>>(fa);
 }
 
-template <int TERMS, bool EXACT = false>
-static int fused_sweep(const FusedArgs &fa, const double *xr, const double *xc, int d, hipStream_t s) {
-    fused_clear_kernel<<<1, 1, 0, s>>>(fa.n_bad);
-    const int n_split = fused_splits(fa.n_rows, fa.n_cols);
-    launch_fused<TERMS, EXACT>(fa, n_split, s);
-    if (n_split > 1) fused_finalize_kernel<<<(fa.n_rows + 255) / 256, 256, 0, s>>>(fa, n_split);
-    fused_repair_kernel<<<64, 256, 0, s>>>(fa.bad_list, fa.n_bad, xr, xc, fa.n_cols, d, fa.h, fa.pot, fa.logw,
-                                           fa.logw_dev, fa.log_n_other, fa.alpha, fa.eps, fa.k, fa.row_sums,
-                                           fa.rs_div);
+template <int TERMS, bool EXACT>
+static int fused_sweep(FusedArgs fa, const double *xr, const double *xc, int d, hipStream_t s) {
+    fa.row_blocks = (fa.n_rows + 127) / 128;
+    fa.n_tiles = (fa.n_cols + 31) / 32;
+    fa.per_split = (fa.n_tiles + fused_splits(fa.n_rows, fa.n_cols) - 1) / fused_splits(fa.n_rows, fa.n_cols);
+    fa.n_split = (fa.n_tiles + fa.per_split - 1) / fa.per_split;
+    switch (fa.kp / 16) {
+        case 1: launch_fused<TERMS, 1, EXACT>(fa, s); break;
+        case 2: launch_fused<TERMS, 2, EXACT>(fa, s); break;
+        case 3: launch_fused<TERMS, 3, EXACT>(fa, s); break;
+        case 4: launch_fused<TERMS, 4, EXACT>(fa, s); break;
+        case 5: launch_fused<TERMS, 5, EXACT>(fa, s); break;
+        case 6: launch_fused<TERMS, 6, EXACT>(fa, s); break;
+        case 7: launch_fused<TERMS, 7, EXACT>(fa, s); break;
+        default: launch_fused<TERMS, 8, EXACT>(fa, s); break;
+    }
+    fused_finish_kernel<<<(fa.n_rows + kFinishRows - 1) / kFinishRows, kFinishThreads, 0, s>>>(fa, xr, xc, d);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
+}
+
+// whether a sweep's units outnumber the places of any instance, so that sums are handed over
+static bool fused_hands_over(int64_t n_rows, int64_t n_cols) {
+    return (n_rows + 127) / 128 * fused_splits((int)n_rows, (int)n_cols) > kFusedCUs;
 }
 
 // ---------------------------------------------------------------------------
@@ -411,16 +620,14 @@ static void problem_carve(Arena &ar, int64_t I, int64_t J, int64_t d, FusedProbl
     fp->nx = ar.take<double>(I);
     fp->ny = ar.take<double>(J);
     fp->zeros = ar.take<double>(std::max(I, J));
-    for (int p = 0; p < 3; ++p) {
-        fp->xp[p] = ar.take<__bf16>((size_t)I * kp);
-        fp->yp[p] = ar.take<__bf16>((size_t)J * kp);
-    }
-    fp->bad = ar.take<int>(std::max(I, J));
-    fp->nbad = ar.take<int>(4);
-    fp->bad2 = ar.take<int>(std::max(I, J));
-    fp->nbad2 = ar.take<int>(4);
+    // padded to whole row blocks (and so to whole column tiles)
+    fp->xp = ar.take<__bf16>((size_t)3 * kp * round_up(I, 128));
+    fp->yp = ar.take<__bf16>((size_t)3 * kp * round_up(J, 128));
     fp->part = ar.take<double>((size_t)kFusedMaxSplit * std::max(I, J));
     fp->part2 = ar.take<double>((size_t)kFusedMaxSplit * std::max(I, J));
+    fp->box_words = fused_hands_over(I, J) || fused_hands_over(J, I) ? kFusedBoxWords : 0;
+    fp->box = ar.take<unsigned long long>((size_t)fp->box_words);
+    fp->box2 = ar.take<unsigned long long>((size_t)2 * fp->box_words);
     fp->median_ws = ar.take<char>(distance_median_bytes(I, J, true));
 }
 
@@ -457,11 +664,17 @@ int fused_problem_setup(const double *X, const double *Y, int64_t I, int64_t J, 
     // scaled, centred coordinates and their bf16 pieces
     fz_mean_kernel<<<(unsigned)d, 256, 0, s>>>(X, (int)I, Y, (int)J, (int)d, fp->mean);
     const int np = terms == 3 ? 2 : 3;
-    __bf16 *const *xp = fp->xp, *const *yp = fp->yp;
-    fz_split_kernel<<<(unsigned)((I + 255) / 256), 256, 0, s>>>(X, (int)I, (int)d, fp->kp, fp->mean, fp->median, np,
-                                                                xp[0], xp[1], xp[2], fp->xs, fp->nx);
-    fz_split_kernel<<<(unsigned)((J + 255) / 256), 256, 0, s>>>(Y, (int)J, (int)d, fp->kp, fp->mean, fp->median, np,
-                                                                yp[0], yp[1], yp[2], fp->ys, fp->ny);
+    const int pi = (int)round_up(I, 128), pj = (int)round_up(J, 128);
+    fz_split_kernel<<<(unsigned)((pi + 255) / 256), 256, 0, s>>>(X, (int)I, pi, (int)d, fp->kp, fp->mean, fp->median,
+                                                                 np, fp->xp, fp->xs, fp->nx);
+    fz_split_kernel<<<(unsigned)((pj + 255) / 256), 256, 0, s>>>(Y, (int)J, pj, (int)d, fp->kp, fp->mean, fp->median,
+                                                                 np, fp->yp, fp->ys, fp->ny);
+    // no word of the boxes carries a launch's mark yet
+    if (fp->box_words) {
+        fz_zero_kernel<<<1024, 256, 0, s>>>(reinterpret_cast<double *>(fp->box), fp->box_words);
+        fz_zero_kernel<<<1024, 256, 0, s>>>(reinterpret_cast<double *>(fp->box2), 2 * fp->box_words);
+    }
+    fp->tag = 0;
     fz_zero_kernel<<<64, 256, 0, s>>>(fp->zeros, (int)std::max(I, J));
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
@@ -470,14 +683,12 @@ int fused_problem_setup(const double *X, const double *Y, int64_t I, int64_t J, 
 // FusedArgs of a sweep over source rows (over_targets = false) or target rows
 static FusedArgs problem_args(const FusedProblem &fp, bool target_rows, const double *h, double *pot,
                               const double *logw, const double *logw_dev, double alpha, double eps, double *row_sums,
-                              double rs_div, bool second_list) {
-    __bf16 *const *A = target_rows ? fp.yp : fp.xp;
-    __bf16 *const *B = target_rows ? fp.xp : fp.yp;
+                              double rs_div, bool second_set) {
     const int nr = target_rows ? fp.J : fp.I, nc = target_rows ? fp.I : fp.J;
-    return FusedArgs{A[0], A[1], A[2], B[0], B[1], B[2], target_rows ? fp.ny : fp.nx, target_rows ? fp.nx : fp.ny,
-                     nr, nc, fp.kp, h, pot, logw, logw_dev, std::log((double)nc), alpha, eps, kLog2E / eps,
-                     second_list ? fp.bad2 : fp.bad, second_list ? fp.nbad2 : fp.nbad, row_sums,
-                     second_list ? fp.part2 : fp.part, rs_div};
+    return FusedArgs{target_rows ? fp.yp : fp.xp, target_rows ? fp.xp : fp.yp, target_rows ? fp.ny : fp.nx,
+                     target_rows ? fp.nx : fp.ny, nr, nc, fp.kp, h, pot, logw, logw_dev, std::log((double)nc), alpha,
+                     eps, kLog2E / eps, row_sums, second_set ? fp.part2 : fp.part, rs_div, 0, 0, 0, 0, 0,
+                     second_set ? fp.box2 : fp.box, ++fp.tag};
 }
 
 template <bool EXACT>

@@ -16,10 +16,12 @@ struct FusedProblem {
     const double *X = nullptr, *Y = nullptr;
     int I = 0, J = 0, d = 0, kp = 0, terms = 6;
     double *mean = nullptr, *xs = nullptr, *ys = nullptr, *nx = nullptr, *ny = nullptr, *zeros = nullptr;
-    __bf16 *xp[3] = {nullptr, nullptr, nullptr}, *yp[3] = {nullptr, nullptr, nullptr};
-    int *bad = nullptr, *nbad = nullptr;    // repair list of the sweeps
-    int *bad2 = nullptr, *nbad2 = nullptr;  // and of the sum passes (which may run on another stream)
+    __bf16 *xp = nullptr, *yp = nullptr;    // split pieces [point][piece][kp], points padded to 128
+    // the sweeps' buffers and (2) those of the sum passes, which may run on another stream
     double *part = nullptr, *part2 = nullptr;
+    unsigned long long *box = nullptr, *box2 = nullptr;  // sums handed between workgroups
+    int box_words = 0;
+    mutable unsigned tag = 0;                            // the last launch's mark on them
     void *median_ws = nullptr;
     const double *median = nullptr;  // device: the exact median of the FP64 distances
 };
@@ -40,7 +42,7 @@ int fused_problem_iterate(const FusedProblem &fp, double *f, double *g, const do
 // sums of exp((f_i + g_j - C_ij)/eps) / div over the targets of every source
 // (over_targets false: out has I entries) or over the sources of every target
 // (true: J entries).  exact: FP64 exponentials and sums (the gap pass), else
-// the sweeps' arithmetic.  Uses the second repair list: it may run on another
+// the sweeps' arithmetic.  Uses the second set of buffers: it may run on another
 // stream than fused_problem_iterate.
 int fused_problem_sums(const FusedProblem &fp, bool over_targets, const double *f, const double *g, double eps,
                        double div, bool exact, double *out, hipStream_t s);

@@ -551,43 +551,6 @@ __global__ __launch_bounds__(1024) void gap_finish_kernel(GapArgs ga) {
 // ---------------------------------------------------------------------------
 constexpr int kGapRows = 128, kGapCols = 1024;
 
-// 2^x for x in [-1100, inf): x = n + r, exp(r ln 2) by its Taylor series to degree 13
-// (|r ln 2| <= 0.347: remainder under 5e-18), scaled by 2^n.  NaN stays NaN.
-__device__ __forceinline__ double exp2_f64(double x) {
-    const double n = rint(x), t = (x - n) * kLn2;
-    double p = 1.0 / 6227020800.0;
-    p = fma(p, t, 1.0 / 479001600.0);
-    p = fma(p, t, 1.0 / 39916800.0);
-    p = fma(p, t, 1.0 / 3628800.0);
-    p = fma(p, t, 1.0 / 362880.0);
-    p = fma(p, t, 1.0 / 40320.0);
-    p = fma(p, t, 1.0 / 5040.0);
-    p = fma(p, t, 1.0 / 720.0);
-    p = fma(p, t, 1.0 / 120.0);
-    p = fma(p, t, 1.0 / 24.0);
-    p = fma(p, t, 1.0 / 6.0);
-    p = fma(p, t, 0.5);
-    p = fma(p, t, 1.0);
-    p = fma(p, t, 1.0);
-    return ldexp(p, (int)n);
-}
-
-// sum over the wave in lane 63, by DPP (row_shr 1, 2, 4, 8, row_bcast 15, 31): no LDS permutes
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
-    return v + __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-    v = dpp_add<0x111, 0xf>(v);
-    v = dpp_add<0x112, 0xf>(v);
-    v = dpp_add<0x114, 0xf>(v);
-    v = dpp_add<0x118, 0xf>(v);
-    v = dpp_add<0x142, 0xa>(v);
-    return dpp_add<0x143, 0xc>(v);
-}
-
 struct GapTileArgs {
     const float *C;
     int64_t ldc;
