@@ -351,3 +351,38 @@ def test_model_get_coupling_chains_in_fp64(tm):
     assert list(cp.obs.index) == ids[0] and list(cp.var.index) == ids[3]
     cp = model.get_coupling(1.0, 3.0)
     assert rel(cp.X, ot_oracle.chain(maps[1:])) < 1e-14
+
+
+@pytest.mark.parametrize('dtype', ['float64', 'float32'])
+@pytest.mark.parametrize('sizes,k', [((1, 1, 2), 1), ((63, 65, 64, 257), 16), ((300, 511, 64, 130), 17),
+                                     ((1025, 2049, 129), 33), ((70, 5003, 71), 3)])
+def test_propagate_at_the_edges_of_its_splits(sizes, k, dtype):
+    """Cells at the edges of the reduction's blocks (64), of a workgroup's row shares (64 and 256) and of
+    the column tiles; one, two and three population groups; outputs kept and not kept on the way."""
+    import torch
+    import wot_amd.tmap as tmap
+    gen = torch.Generator(device='cuda').manual_seed(sum(sizes) + k)
+    maps = [torch.rand((a, b), dtype=getattr(torch, dtype), device='cuda', generator=gen)
+            for a, b in zip(sizes, sizes[1:])]
+    for direction, order in ((tmap.PUSH_FORWARD, maps), (tmap.PULL_BACK, [m.T.contiguous() for m in maps])):
+        for transposed in (False, True) if direction == tmap.PULL_BACK else (False,):
+            held = [tmap.DeviceMap.upload(m, dtype) for m in order]
+            if transposed:
+                for m in held:
+                    m.make_transposed()
+            p = torch.rand((sizes[0], k), dtype=torch.float64, device='cuda', generator=gen)
+            outs = [None if s % 2 else torch.empty((n, k), dtype=torch.float64, device='cuda')
+                    for s, n in enumerate(sizes[1:], start=len(sizes) % 2)]
+            for normalize in (True, False):
+                got = tmap.propagate(held, p, direction, normalize=normalize, outs=outs)
+                ref = p
+                for s, m in enumerate(maps):
+                    ref = m.double().T @ ref
+                    if normalize:
+                        ref = ref / ref.sum(0, keepdim=True)
+                    if outs[s] is not None:
+                        # positive terms: a map's sums take at most one rounding per cell in (products) and
+                        # out (total) and a few more, on either side
+                        tol = 2 * (2 * sum(sizes) + 8 * len(maps)) * 2.0 ** -53
+                        assert float(((outs[s] - ref) / ref).abs().max()) < tol
+                assert got is outs[-1]

@@ -22,9 +22,11 @@ DEVICE_FLAGS = [
 
 
 # per-source device flags: the never-stored sweep keeps its MFMA accumulators
-# in ordinary VGPRs (no AGPR copies before the per-entry exponentials)
+# in ordinary VGPRs (no AGPR copies before the per-entry exponentials), and so do
+# the map products (24 populations through FP32 maps: 388 us, with AGPRs 416)
 SOURCE_FLAGS = {
     'fused.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    'tmap.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
     # the resident solver's registers hold the cost: constants of the logarithms and
     # exponentials are formed where they are used, not kept across its loops
     'resident.hip': ['-mllvm', '-disable-machine-licm'],

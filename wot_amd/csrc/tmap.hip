@@ -28,7 +28,10 @@ namespace {
 
 constexpr int kPopTile = 16;          // populations per MFMA tile
 constexpr int kWaves = 4;             // waves per workgroup (no LDS, no barriers)
-constexpr int kTargetWaves = 4096;    // ~4 waves per SIMD on 256 CUs
+// Waves of a product: two per SIMD, all resident at once.  Splits are rounded down, so that no
+// second round of a few waves follows (seven maps of 3900 to 12001 cells, 10 populations: 596 us;
+// 607 at three per SIMD, 669 at one and a half; 684 at three and 708 at four rounded up)
+constexpr int kTargetWaves = 2048;
 constexpr int kPushBlocks = 4;        // 16-column MFMA blocks per push wave (4 or 8)
 constexpr int kPushCols = 16 * kPushBlocks;
 constexpr int kPushSteps = 4;         // MFMA k-steps (4 rows each) per push trip
@@ -36,7 +39,7 @@ constexpr bool kPushPipelined = false; // push trips double-buffered (measured s
 constexpr int kPullRowBlocks = 4;     // 16-row MFMA blocks per pull wave
 constexpr int kPullVecs = 2;          // 16-byte loads per lane, row and pull step
 constexpr bool kPullPipelined = true; // pull steps double-buffered
-constexpr int kReduceCells = 256 / 16; // cells per reduce workgroup (one thread per cell and population)
+constexpr int kReduceCells = 64;     // cells per reduce workgroup
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
@@ -46,10 +49,40 @@ __device__ inline d4 mfma_f64(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Sums of the populations over blocks of cells, as pops_reduce_kernel leaves them
+// ([group][block][16]); null: not normalised.  Every workgroup that needs a total adds the
+// blocks (one per 64 cells) itself: a launch of its own for the totals took 5 us between
+// two maps.
+struct PopSums {
+    const double *sums;
+    int n_blocks, n_pops;
+};
+
+// total of population group * 16 + l % 16 in every lane l (1 where there is none); all WAVES
+// waves of the workgroup
+template <int WAVES>
+__device__ inline double pop_total(const PopSums &ps, int group) {
+    __shared__ double share[WAVES][kPopTile];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = lane & 15;
+    const double *src = ps.sums + (int64_t)group * ps.n_blocks * kPopTile + m;
+    double t = 0.0;
+#pragma unroll 8
+    for (int b = threadIdx.x >> 4; b < ps.n_blocks; b += 4 * WAVES) t += src[(int64_t)b * kPopTile];
+    t += __shfl_xor(t, 16);
+    t += __shfl_xor(t, 32);
+    __syncthreads();  // a total of another group may still be read
+    if (lane < kPopTile) share[wave][m] = t;
+    __syncthreads();
+    t = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) t += share[w][m];
+    return group * kPopTile + m < ps.n_pops ? t : 1.0;
+}
+
 // B operand scale: the reference divides every population by its sum before
 // the next map (p / sum); the products use p * (1 / sum), hoisted per lane
-__device__ inline double pop_scale(const double *__restrict__ scale, int group, int pop) {
-    return scale ? 1.0 / scale[group * kPopTile + pop] : 1.0;
+__device__ inline double pop_scale(const PopSums &ps, int group) {
+    return ps.sums ? 1.0 / pop_total<kWaves>(ps, group) : 1.0;
 }
 
 template <typename T> struct Vec16;  // 16 bytes of map entries
@@ -182,20 +215,22 @@ __device__ inline void push_tile(const T *__restrict__ map, int64_t ld, int64_t 
     }
 }
 
+// The workgroup's waves share its columns and take a quarter of the split's rows each; their sums
+// meet in LDS, so the partials are a fourth of what one per wave would be (with a column tile per
+// wave the partials of a 7500 x 7500 map were 33 MB written and read beside its 450 MB).
 template <typename T, bool VEC, int NGW>
 __global__ __launch_bounds__(256) void push_partial_kernel(const T *__restrict__ map, int64_t ld, int64_t n_rows,
                                                            int64_t n_cols, const double *__restrict__ pops,
-                                                           const double *__restrict__ scale,
-                                                           double *__restrict__ part, int64_t split_rows,
-                                                           int n_tiles, int n_groups) {
-    const int lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (tile >= n_tiles) return;
+                                                           PopSums scale, double *__restrict__ part,
+                                                           int64_t split_rows, int n_groups) {
+    static_assert(kPushBlocks == kWaves, "wave w adds up MFMA block w");
+    __shared__ double red[kWaves][kPushBlocks][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int split = blockIdx.y, g0 = blockIdx.z * NGW;
     const int m = lane & 15, q = lane >> 4;
-    const int64_t j0 = (int64_t)tile * kPushCols;
-    const int64_t i_begin = (int64_t)split * split_rows;
-    const int64_t i_end = min(n_rows, i_begin + split_rows);
+    const int64_t j0 = (int64_t)blockIdx.x * kPushCols;
+    const int64_t i_begin = min(n_rows, (int64_t)split * split_rows + wave * (split_rows / kWaves));
+    const int64_t i_end = min(n_rows, i_begin + split_rows / kWaves);
     // a group past the last one multiplies group g0's values by 0 and is not written
     const double *P[NGW];
     double inv[NGW];
@@ -203,7 +238,7 @@ __global__ __launch_bounds__(256) void push_partial_kernel(const T *__restrict__
     for (int g = 0; g < NGW; ++g) {
         const bool valid = g0 + g < n_groups;
         P[g] = pops + (int64_t)(valid ? g0 + g : g0) * n_rows * kPopTile;
-        inv[g] = valid ? pop_scale(scale, g0 + g, m) : 0.0;
+        inv[g] = pop_scale(scale, valid ? g0 + g : g0) * (valid ? 1.0 : 0.0);
     }
 
     d4 acc[NGW][kPushBlocks];
@@ -218,15 +253,22 @@ __global__ __launch_bounds__(256) void push_partial_kernel(const T *__restrict__
 
 #pragma unroll
     for (int g = 0; g < NGW; ++g) {
-        if (g0 + g >= n_groups) break;
-        double *out = part + ((int64_t)split * n_groups + g0 + g) * n_cols * kPopTile;
+        if (g0 + g >= n_groups) break;  // uniform
+        if (g) __syncthreads();
 #pragma unroll
         for (int b = 0; b < kPushBlocks; ++b)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t j = push_col<T>(j0, b, q + 4 * r);
-                if (j < n_cols) out[j * kPopTile + m] = acc[g][b][r];
-            }
+            for (int r = 0; r < 4; ++r) red[wave][b][r][lane] = acc[g][b][r];
+        __syncthreads();
+        double *out = part + ((int64_t)split * n_groups + g0 + g) * n_cols * kPopTile;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t j = push_col<T>(j0, wave, q + 4 * r);
+            double v = red[0][wave][r][lane];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) v += red[w][wave][r][lane];
+            if (j < n_cols) out[j * kPopTile + m] = v;
+        }
     }
 }
 
@@ -316,21 +358,21 @@ __device__ inline void pull_step_mfma(const PullStep<T> &st, double inv, d4 acc[
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void pull_partial_kernel(const T *__restrict__ map, int64_t ld, int64_t n_rows,
                                                            int64_t n_cols, const double *__restrict__ pops,
-                                                           const double *__restrict__ scale,
+                                                           PopSums scale,
                                                            double *__restrict__ part, int64_t split_cols,
                                                            int n_tiles) {
     constexpr int KS = 4 * PullStep<T>::E;  // columns per step
     constexpr int RB = kPullRowBlocks;
     const int lane = threadIdx.x & 63;
+    const int split = blockIdx.y, group = blockIdx.z, n_groups = gridDim.z;
+    const double inv = pop_scale(scale, group);
     const int tile = blockIdx.x * kWaves + (threadIdx.x >> 6);
     if (tile >= n_tiles) return;
-    const int split = blockIdx.y, group = blockIdx.z, n_groups = gridDim.z;
     const int m = lane & 15, q = lane >> 4;
     const int64_t i0 = (int64_t)tile * 16 * RB;
     const int64_t j_begin = (int64_t)split * split_cols;
     const int64_t j_end = min(n_cols, j_begin + split_cols);
     const double *P = pops + (int64_t)group * n_cols * kPopTile;
-    const double inv = pop_scale(scale, group, m);
 
     const T *rows[RB];
     bool row_ok[RB];
@@ -393,79 +435,69 @@ __global__ __launch_bounds__(256) void pops_import_kernel(const double *__restri
     dst[(int64_t)group * n * kPopTile + t] = pop < k ? src[cell * ld + pop] : 0.0;
 }
 
-// sum of the split partials in split order, one thread per (cell, population);
-// per-workgroup partial sums of every population (16 cells) for the
-// normalisation (fixed order: deterministic)
-__global__ __launch_bounds__(256) void pops_reduce_kernel(const double *__restrict__ part, int n_split, int64_t n,
-                                                          double *__restrict__ dst, double *__restrict__ block_sums) {
-    __shared__ double red[256];
+// internal -> external cells x pops (ld), divided by the totals when given
+struct PopExport {
+    const double *src;
+    int64_t n;      // cells
+    int n_pops;
+    PopSums sums;
+    double *dst;    // null: nothing to write
+    int64_t ld;
+};
+
+constexpr int kReduceThreads = kReduceCells * kPopTile;
+
+// one workgroup's kReduceCells cells
+__device__ inline void export_cells(const PopExport &ex, int group, int64_t block) {
+    const int64_t t = block * kReduceThreads + threadIdx.x;
+    const int pop = group * kPopTile + threadIdx.x % kPopTile;
+    const bool mine = t < ex.n * kPopTile && pop < ex.n_pops;
+    const double v = mine ? ex.src[(int64_t)group * ex.n * kPopTile + t] : 0.0;
+    const double total = ex.sums.sums ? pop_total<kReduceThreads / 64>(ex.sums, group) : 1.0;
+    if (mine) ex.dst[t / kPopTile * ex.ld + pop] = ex.sums.sums ? v / total : v;
+}
+
+// First n_blocks workgroups: the split partials added in split order, kReduceCells cells each, and
+// those cells' sums of every population for the normalisation (fixed order: deterministic).  The
+// others write out the populations that the map took in, which need the sums over all cells and so
+// wait for the launch after theirs.  With launches of their own for sums and output, and four times
+// the partials, seven maps of 3900 to 12001 cells took 731 us, with this 596 (eight of 600 to 1500
+// cells: 147, 110).
+__global__ __launch_bounds__(kReduceThreads) void pops_reduce_kernel(const double *__restrict__ part, int n_split,
+                                                                     int64_t n, int n_blocks,
+                                                                     double *__restrict__ dst,
+                                                                     double *__restrict__ block_sums, PopExport ex) {
+    __shared__ double red[kReduceThreads / 64][kPopTile];
     const int group = blockIdx.y, n_groups = gridDim.y;
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;  // cell * 16 + pop
-    const int64_t stride = n * kPopTile;                        // one split's slice of a group
+    if ((int)blockIdx.x >= n_blocks) {
+        export_cells(ex, group, (int)blockIdx.x - n_blocks);
+        return;
+    }
+    const int64_t t = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x;  // cell * 16 + pop
+    const int64_t stride = n * kPopTile;                                   // one split's slice of a group
+    const int64_t step = (int64_t)n_groups * stride;
     double v = 0.0;
     if (t < stride) {
         const double *src = part + (int64_t)group * stride + t;
-        const int64_t step = (int64_t)n_groups * stride;
-        int s = 0;
-        for (; s + 4 <= n_split; s += 4) {
-            const double a = src[(int64_t)s * step], b = src[(int64_t)(s + 1) * step];
-            const double c = src[(int64_t)(s + 2) * step], d = src[(int64_t)(s + 3) * step];
-            v = (((v + a) + b) + c) + d;
-        }
-        for (; s < n_split; ++s) v += src[(int64_t)s * step];
+#pragma unroll 8
+        for (int s = 0; s < n_split; ++s) v += src[(int64_t)s * step];
         dst[(int64_t)group * stride + t] = v;
     }
-    red[threadIdx.x] = v;
+    // over the wave's four cells, then over the waves
+    v += __shfl_xor(v, 16);
+    v += __shfl_xor(v, 32);
+    if ((threadIdx.x & 63) < kPopTile) red[threadIdx.x >> 6][threadIdx.x & 63] = v;
     __syncthreads();
-    for (int w = 128; w >= kPopTile; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x < kPopTile)
-        block_sums[((int64_t)group * gridDim.x + blockIdx.x) * kPopTile + threadIdx.x] = red[threadIdx.x];
-}
-
-// totals[group*16 + pop] = sum of the block sums (padded populations: 1);
-// 1024 threads, 4 independent partial sums each, combined in a fixed order
-constexpr int kTotalsThreads = 1024;
-__global__ __launch_bounds__(kTotalsThreads) void pops_totals_kernel(const double *__restrict__ block_sums,
-                                                                     int n_blocks, int k,
-                                                                     double *__restrict__ totals) {
-    __shared__ double red[kTotalsThreads];
-    const int group = blockIdx.x;
-    const int pop = threadIdx.x % kPopTile;
-    constexpr int lanes = kTotalsThreads / kPopTile;  // threads per population
-    const double *src = block_sums + (int64_t)group * n_blocks * kPopTile + pop;
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    int b = threadIdx.x / kPopTile;
-    for (; b + 3 * lanes < n_blocks; b += 4 * lanes)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] += src[(int64_t)(b + u * lanes) * kPopTile];
-    for (; b < n_blocks; b += lanes) t[0] += src[(int64_t)b * kPopTile];
-    red[threadIdx.x] = (t[0] + t[1]) + (t[2] + t[3]);
-    __syncthreads();
-    for (int w = kTotalsThreads / 2; w >= kPopTile; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
     if (threadIdx.x < kPopTile) {
-        const int p = group * kPopTile + threadIdx.x;
-        totals[p] = p < k ? red[threadIdx.x] : 1.0;
+        double total = 0.0;
+#pragma unroll
+        for (int w = 0; w < kReduceThreads / 64; ++w) total += red[w][threadIdx.x];
+        block_sums[((int64_t)group * n_blocks + blockIdx.x) * kPopTile + threadIdx.x] = total;
     }
 }
 
-// internal -> external cells x pops (ld), divided by the totals when given
-__global__ __launch_bounds__(256) void pops_export_kernel(const double *__restrict__ src, int64_t n, int k,
-                                                          const double *__restrict__ totals, double *__restrict__ dst,
-                                                          int64_t ld) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int group = blockIdx.y;
-    if (t >= n * kPopTile) return;
-    const int64_t cell = t / kPopTile;
-    const int pop = group * kPopTile + (int)(t % kPopTile);
-    if (pop >= k) return;
-    const double v = src[(int64_t)group * n * kPopTile + t];
-    dst[cell * ld + pop] = totals ? v / totals[pop] : v;
+__global__ __launch_bounds__(kReduceThreads) void pops_export_kernel(PopExport ex) {
+    export_cells(ex, blockIdx.y, blockIdx.x);
 }
 
 // dst[j][i] = src[i][j] through a padded 32 x 32 LDS tile (reads and writes coalesced)
@@ -535,10 +567,13 @@ StepShape step_shape(const wotk_tmap &m, int direction, int n_groups) {
     const int64_t tiles = push ? (m.cols + kPushCols - 1) / kPushCols
                                : (m.rows + 16 * kPullRowBlocks - 1) / (16 * kPullRowBlocks);
     s.n_tiles = (int)tiles;
-    const int64_t quantum = push ? 16 : pull_step_cols(m.dtype);
-    // enough splits to put ~kTargetWaves waves in flight, each reduction chunk >= 8 quanta
-    int64_t want = (kTargetWaves + tiles * n_groups - 1) / (tiles * n_groups);
-    int64_t most = std::max<int64_t>(1, s.reduce_len / (8 * quantum));
+    // push: a workgroup's waves share the split's rows, four row trips at least for each wave
+    const int64_t quantum = push ? 16 * kWaves : pull_step_cols(m.dtype);
+    const int64_t waves = push ? kWaves : 1, least = push ? 4 : 8;
+    // as many splits as kTargetWaves waves hold, each reduction chunk >= `least` quanta
+    const int64_t layers = push ? (n_groups + 1) / 2 : n_groups;  // a push wave takes two groups
+    int64_t want = kTargetWaves / (waves * tiles * layers);
+    int64_t most = std::max<int64_t>(1, s.reduce_len / (least * quantum));
     int64_t splits = std::max<int64_t>(1, std::min(want, most));
     s.split_len = round_up((s.reduce_len + splits - 1) / splits, quantum);
     if (s.split_len <= 0) s.split_len = quantum;
@@ -547,7 +582,7 @@ StepShape step_shape(const wotk_tmap &m, int direction, int n_groups) {
 }
 
 struct Layout {
-    double *part = nullptr, *pop_a = nullptr, *pop_b = nullptr, *block_sums = nullptr, *totals = nullptr;
+    double *part = nullptr, *pop_a = nullptr, *pop_b = nullptr, *block_sums[2] = {nullptr, nullptr};
 };
 
 int check_chain(const wotk_tmap *maps, int32_t n_maps, int32_t direction, int32_t n_pops) {
@@ -588,8 +623,7 @@ Layout carve(Arena &ar, const wotk_tmap *maps, int32_t n_maps, int32_t direction
     L.part = ar.take<double>((size_t)max_part * n_groups * kPopTile);
     L.pop_a = ar.take<double>((size_t)max_cells * n_groups * kPopTile);
     L.pop_b = ar.take<double>((size_t)max_cells * n_groups * kPopTile);
-    L.block_sums = ar.take<double>((size_t)max_blocks * n_groups * kPopTile);
-    L.totals = ar.take<double>((size_t)2 * n_groups * kPopTile);
+    for (double *&sums : L.block_sums) sums = ar.take<double>((size_t)max_blocks * n_groups * kPopTile);
     return L;
 }
 
@@ -600,26 +634,27 @@ bool vec_ok(const wotk_tmap &m) {
 
 template <typename T>
 void launch_partial(const wotk_tmap &m, int direction, const StepShape &sh, int n_groups, const double *pops,
-                    const double *scale, double *part, hipStream_t st) {
+                    const PopSums &scale, double *part, hipStream_t st) {
     const T *map = static_cast<const T *>(m.data);
     dim3 grid((sh.n_tiles + kWaves - 1) / kWaves, sh.n_split, n_groups);
     const bool vec = vec_ok<T>(m);
     if (direction == WOTK_PUSH_FORWARD) {
+        grid.x = (unsigned)sh.n_tiles;
         // two population groups per wave when there are several: one read of the map for both
         if (n_groups > 1) {
             grid.z = (n_groups + 1) / 2;
             if (vec)
                 push_partial_kernel<T, true, 2><<<grid, 256, 0, st>>>(map, m.ld, m.rows, m.cols, pops, scale, part,
-                                                                     sh.split_len, sh.n_tiles, n_groups);
+                                                                     sh.split_len, n_groups);
             else
                 push_partial_kernel<T, false, 2><<<grid, 256, 0, st>>>(map, m.ld, m.rows, m.cols, pops, scale, part,
-                                                                      sh.split_len, sh.n_tiles, n_groups);
+                                                                      sh.split_len, n_groups);
         } else if (vec) {
             push_partial_kernel<T, true, 1><<<grid, 256, 0, st>>>(map, m.ld, m.rows, m.cols, pops, scale, part,
-                                                                 sh.split_len, sh.n_tiles, n_groups);
+                                                                 sh.split_len, n_groups);
         } else {
             push_partial_kernel<T, false, 1><<<grid, 256, 0, st>>>(map, m.ld, m.rows, m.cols, pops, scale, part,
-                                                                  sh.split_len, sh.n_tiles, n_groups);
+                                                                  sh.split_len, n_groups);
         }
     } else {
         if (vec)
@@ -673,7 +708,8 @@ extern "C" int wotk_tmap_propagate(const wotk_tmap *maps, int32_t n_maps, int32_
         for (auto &e : ev) WOTK_HIP(hipEventCreate(&e));
     }
     double *cur = L.pop_a, *nxt = L.pop_b;
-    const double *scale = nullptr;  // totals of the previous map (normalising chains)
+    PopSums scale{nullptr, 0, n_pops};  // sums behind the previous map (normalising chains)
+    PopExport ex{};                     // the previous map's output, not written yet
     for (int s = 0; s < n_maps; ++s) {
         int dir;
         const wotk_tmap m = effective_map(maps[s], direction, &dir);
@@ -686,23 +722,17 @@ extern "C" int wotk_tmap_propagate(const wotk_tmap *maps, int32_t n_maps, int32_
         WOTK_LAUNCH_CHECK();
         if (stats) WOTK_HIP(hipEventRecord(ev[2 * s + 1], st));
         const int n_blocks = (int)((sh.n_out + kReduceCells - 1) / kReduceCells);
-        pops_reduce_kernel<<<dim3(n_blocks, n_groups), 256, 0, st>>>(L.part, sh.n_split, sh.n_out, nxt,
-                                                                    L.block_sums);
+        const int n_export = ex.dst ? (int)((ex.n + kReduceCells - 1) / kReduceCells) : 0;
+        double *sums = L.block_sums[s & 1];
+        pops_reduce_kernel<<<dim3(n_blocks + n_export, n_groups), kReduceThreads, 0, st>>>(
+            L.part, sh.n_split, sh.n_out, n_blocks, nxt, sums, ex);
         WOTK_LAUNCH_CHECK();
-        double *tot = nullptr;
-        if (normalize) {
-            tot = L.totals + (s & 1) * n_groups * kPopTile;
-            pops_totals_kernel<<<n_groups, kTotalsThreads, 0, st>>>(L.block_sums, n_blocks, n_pops, tot);
-            WOTK_LAUNCH_CHECK();
-        }
-        if (outs[s]) {
-            dim3 grid((unsigned)((sh.n_out * kPopTile + 255) / 256), n_groups);
-            pops_export_kernel<<<grid, 256, 0, st>>>(nxt, sh.n_out, n_pops, tot, outs[s], ldo);
-            WOTK_LAUNCH_CHECK();
-        }
-        scale = tot;
+        scale = PopSums{normalize ? sums : nullptr, n_blocks, n_pops};
+        ex = PopExport{nxt, sh.n_out, n_pops, scale, outs[s], ldo};
         std::swap(cur, nxt);
     }
+    pops_export_kernel<<<dim3((unsigned)((ex.n + kReduceCells - 1) / kReduceCells), n_groups), kReduceThreads, 0, st>>>(ex);
+    WOTK_LAUNCH_CHECK();
     if (stats) {
         *stats = wotk_stats{};
         WOTK_HIP(hipStreamSynchronize(st));
