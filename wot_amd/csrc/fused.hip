@@ -102,6 +102,10 @@ struct FusedArgs {
     int whole;                   // one unit per workgroup; else an equal run of tiles each
     unsigned long long *box;     // [workgroup][word][thread]: partial sums handed to the next workgroup
     unsigned tag;                // this launch's mark on them
+    TauTrack tau;                // growth of the potentials (prev null: not tracked)
+    double *base;                // what they grow from: u or v
+    int opens;                   // the iteration's first sweep
+    const int *skip;             // device flag: the launches do nothing when it is set (null: never)
 };
 
 // tiles of the units, split-major, rows next: unit (x, y) starts at first_tile
@@ -199,6 +203,11 @@ __global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS, EXACT)) void fus
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, kg = (lane >> 5) * 8;
     const double k2 = 2.0 * fa.k;
+    if (fa.skip && *fa.skip) return;
+    if (fa.tau.prev && fa.opens && blockIdx.x == 0 && tid == 0) {
+        if (tau_fired(*fa.tau.prev, fa.tau.tau)) fa.tau.counter[0] += 1;
+        *fa.tau.cur = tau_key(-INFINITY);
+    }
 
     const int64_t total = (int64_t)fa.row_blocks * fa.n_tiles;
     int64_t lo, hi;
@@ -424,7 +433,9 @@ __global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS, EXACT)) void fus
 // distances of the scaled coordinates ([d][n], read coalesced) with a per-lane online maximum.
 // Such a row costs one read of all column points through one CU (8 MB at 20000 x 50), so up to
 // four share it.  One launch behind a sweep; clearing a list, adding the splits and repairing by
-// three took 20 us of a sweep at 20000 x 20000, this takes 6.
+// three took 20 us of a sweep at 20000 x 20000, this takes 6.  The growth that the tau check looks at
+// is kept here too: a launch of its own per iteration made a 3000 x 3000 duality-gap solve 22.9 ms,
+// now 21.2.
 constexpr int kFinishRows = 32, kFinishThreads = 1024, kFinishWaves = kFinishThreads / 64, kRepairRows = 4;
 
 template <int NB>
@@ -510,10 +521,13 @@ __global__ __launch_bounds__(kFinishThreads) void fused_finish_kernel(FusedArgs 
     __shared__ int bad[kFinishRows];
     __shared__ int n_bad;
     const int tid = threadIdx.x;
+    if (fa.skip && *fa.skip) return;
+    const bool absorb = fa.tau.prev && tau_fired(*fa.tau.prev, fa.tau.tau);
     if (tid == 0) n_bad = 0;
     __syncthreads();
     const int row = blockIdx.x * kFinishRows + tid;
     if (tid < kFinishRows && row < fa.n_rows) {
+        if (absorb) fa.base[row] = fa.pot[row];
         double S = 0.0;
         for (int q = 0; q < fa.n_split; ++q) S += fa.part[(int64_t)q * fa.n_rows + row];
         if (isnan(S)) {
@@ -539,6 +553,12 @@ __global__ __launch_bounds__(kFinishThreads) void fused_finish_kernel(FusedArgs 
         repair_rows<kRepairRows>(fa, batch, xr, xc, d, x_sh, sg_sh, sd_sh);
     }
     if (q < n_bad) repair_rows<1>(fa, bad + q, xr, xc, d, x_sh, sg_sh, sd_sh);
+    if (fa.tau.prev && tid < 64) {  // largest growth over the workgroup's rows
+        double m = -INFINITY;
+        if (tid < kFinishRows && row < fa.n_rows) m = (fa.pot[row] - fa.base[row]) * fa.tau.inv_eps;
+        for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+        if (tid == 0) atomicMax(fa.tau.cur, tau_key(m));
+    }
 }
 
 __global__ __launch_bounds__(1024) void fz_growth_kernel(const double *__restrict__ G, int n, double *__restrict__ logp,
@@ -688,7 +708,7 @@ static FusedArgs problem_args(const FusedProblem &fp, bool target_rows, const do
     return FusedArgs{target_rows ? fp.yp : fp.xp, target_rows ? fp.xp : fp.yp, target_rows ? fp.ny : fp.nx,
                      target_rows ? fp.nx : fp.ny, nr, nc, fp.kp, h, pot, logw, logw_dev, std::log((double)nc), alpha,
                      eps, kLog2E / eps, row_sums, second_set ? fp.part2 : fp.part, rs_div, 0, 0, 0, 0, 0,
-                     second_set ? fp.box2 : fp.box, ++fp.tag};
+                     second_set ? fp.box2 : fp.box, ++fp.tag, TauTrack{}, nullptr, 0, nullptr};
 }
 
 template <bool EXACT>
@@ -698,13 +718,21 @@ static int problem_sweep(const FusedProblem &fp, const FusedArgs &fa, bool targe
 }
 
 int fused_problem_iterate(const FusedProblem &fp, double *f, double *g, const double *logp,
-                          const double *logq_dev, double lambda1, double lambda2, double eps, hipStream_t s) {
-    const FusedArgs fr = problem_args(fp, false, g, f, logp, nullptr, lambda1 / (lambda1 + eps), eps, nullptr, 1.0,
+                          const double *logq_dev, double lambda1, double lambda2, double eps, const TauTrack &tau,
+                          const int *skip, hipStream_t s) {
+    FusedArgs fr = problem_args(fp, false, g, f, logp, nullptr, lambda1 / (lambda1 + eps), eps, nullptr, 1.0,
                                       false);
+    fr.tau = tau;
+    fr.base = tau.u;
+    fr.opens = 1;
+    fr.skip = skip;
     int rc = problem_sweep<false>(fp, fr, false, s);
     if (rc) return rc;
-    const FusedArgs fc = problem_args(fp, true, f, g, nullptr, logq_dev, lambda2 / (lambda2 + eps), eps, nullptr, 1.0,
+    FusedArgs fc = problem_args(fp, true, f, g, nullptr, logq_dev, lambda2 / (lambda2 + eps), eps, nullptr, 1.0,
                                       false);
+    fc.tau = tau;
+    fc.base = tau.v;
+    fc.skip = skip;
     return problem_sweep<false>(fp, fc, true, s);
 }
 
@@ -781,7 +809,7 @@ extern "C" int wotk_transport_stablev2_coords(const double *X, const double *Y, 
     const int64_t n_iter = scaling_iter + extra_iter;
     for (int64_t it = 0; it < n_iter; ++it) {
         const double eps = it < scaling_iter ? reg(it / inner_iter_max) : reg(scaling_iter / inner_iter_max);
-        rc = fused_problem_iterate(fp, w.f, w.g, w.logp, w.misc, lambda1, lambda2, eps, s);
+        rc = fused_problem_iterate(fp, w.f, w.g, w.logp, w.misc, lambda1, lambda2, eps, TauTrack{}, nullptr, s);
         if (rc) return rc;
     }
     WOTK_HIP(hipEventRecord(ev[1], s));

@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "onepass.h"
+
 namespace wotk {
 
 // C = sqeuclid(X, Y) / median(sqeuclid(X, Y)) regenerated per tile from the
@@ -35,9 +37,11 @@ int fused_problem_setup(const double *X, const double *Y, int64_t I, int64_t J, 
                         void *workspace, size_t workspace_bytes, FusedProblem *fp, size_t *used, hipStream_t s);
 
 // one (a, b) iteration at eps: f from g (source rows, log weights logp), then
-// g from f (target rows, log q at logq_dev[0])
+// g from f (target rows, log q at logq_dev[0]); tau: its growth is kept; skip: a device
+// flag that turns it into nothing
 int fused_problem_iterate(const FusedProblem &fp, double *f, double *g, const double *logp,
-                          const double *logq_dev, double lambda1, double lambda2, double eps, hipStream_t s);
+                          const double *logq_dev, double lambda1, double lambda2, double eps, const TauTrack &tau,
+                          const int *skip, hipStream_t s);
 
 // sums of exp((f_i + g_j - C_ij)/eps) / div over the targets of every source
 // (over_targets false: out has I entries) or over the sources of every target

@@ -524,10 +524,11 @@ int launch_rows(const RowArgs &ra, int grid, hipStream_t s) {
 }  // namespace
 
 // Where one read of C beats two sweeps over C and C^T (us per iteration, two sweeps against one
-// read): 2900 x 2900 20.0 / 17.5, 6000 x 5000 44 / 33, 10000 x 8001 105 / 64.5, 15000 x 15000
-// 272 / 153.6, 19000 x 19000 (the widest rows whose sums fit in registers) about 436 / 234.  Pairs
-// under 2^23 entries go to the resident solver instead (14.5 us at 2749 x 3001); the ones of
-// them that it does not take keep the two sweeps, whose FP32 sums their FP64 maps are held to.
+// read): 2900 x 2900 19.2 / 17.9, 9000 x 1001 24.8 / 22.6, 600 x 19000 42.4 / 30.5, 6000 x 5000
+// 43.7 / 33.1, 10000 x 8001 105 / 64.9, 15000 x 15000 275 / 154, 19000 x 19000 (the widest rows whose
+// sums fit in registers) 439 / 236.  Pairs under 2^23 entries go to the resident solver instead
+// (14.4 us at 2749 x 3001); the ones of them that it does not take keep the two sweeps, whose FP32
+// sums their FP64 maps are held to.
 bool one_pass_fits(int64_t I, int64_t J) {
     if (chunks_of(J) > kMaxChunks || I > (int64_t)kCus * kMaxRows) return false;
     return I * J >= (1ll << 23);

@@ -686,9 +686,9 @@ int clear(const ResidentProblem &rp, hipStream_t s) {
 }  // namespace
 
 // Where the resident solver beats launched sweeps: everywhere its registers hold the pair (us per
-// iteration, launched / resident): 50 x 60 8.1 / 4.6, 300 x 400 8.4 / 5.1, 1000 x 1000 8.9 / 6.2,
-// 2000 x 2500 15.8 / 11.0, 2749 x 3001 20.0 / 14.5, 900 x 8000 22.9 / 15.5.  From 2^23 entries on
-// the one-read iteration is the other side: 17.5 us at 2900 x 2900.
+// iteration, launched / resident): 50 x 60 8.0 / 4.5, 300 x 400 8.3 / 5.2, 1000 x 1000 8.9 / 6.2,
+// 2000 x 2500 15.8 / 10.9, 2890 x 2890 19.8 / 14.5, 900 x 8000 23.1 / 15.4.  From 2^23 entries on
+// the one-read iteration is the other side: 17.9 us at 2900 x 2900.
 bool resident_fits(int64_t I, int64_t J) {
     if (I > kMaxSide || J > kMaxSide || I * J > (1ll << 23)) return false;
     const Shape s = shape_of(I, J);

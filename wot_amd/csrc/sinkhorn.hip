@@ -1458,9 +1458,10 @@ struct FusedBackend {
     Work &w;
     const FusedProblem &fp;
     double *row_sums, *f_out, *g_out;
-    bool tracks_growth() const { return false; }
-    int iterate(double l1, double l2, double eps, hipStream_t s, const TauTrack &) {
-        return fused_problem_iterate(fp, w.f, w.g, w.logp, w.misc, l1, l2, eps, s);
+    bool tracks_growth() const { return true; }
+    int iterate(double l1, double l2, double eps, hipStream_t s, const TauTrack &tau) {
+        return fused_problem_iterate(fp, w.f, w.g, w.logp, w.misc, l1, l2, eps, tau, w.run_ahead ? w.skip : nullptr,
+                                     s);
     }
     int gap_pass(const double *f, const double *g, double l1, double l2, double eps, const double *skt,
                  hipStream_t s) {
