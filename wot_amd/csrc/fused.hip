@@ -13,12 +13,12 @@
 // round at 2^-24 of the cross term; in FP64 the marginals of a 97 x 131, d = 7
 // pair at eps = 0.05 move from 1.6e-6 to 6.7e-7 of the FP64 oracle's, for 6 %
 // more sweep time at 60k); with 3 terms, whose missing products already cost
-// 2^-16, in FP32.  Per entry the exponent is
-// formed in FP64 against the row's previous potential (a fixed shift, as in
-// the batched sweep); rows whose sum under- or overflows are queued and
-// recomputed by a repair kernel from FP64 direct distances with an online
-// maximum.  The median of the exact FP64 distances (the reference's
-// normalisation) comes from two passes that regenerate them (distance.hip).
+// 2^-16, in FP32.  Per entry the exponent is formed in FP64 against the row's
+// previous potential (a fixed shift, as in the batched sweep); rows whose sum
+// under- or overflows are recomputed behind the sweep from FP64 direct distances
+// with an online maximum.  The median of the exact FP64 distances (the
+// reference's normalisation) comes from two passes that regenerate them
+// (distance.hip).
 #include <type_traits>
 
 #include "common.h"
@@ -34,9 +34,11 @@ constexpr int kFThreads = 256;
 constexpr int kFusedMaxSplit = 8;        // column splits per sweep, at most
 constexpr int kFusedTargetBlocks = 768;
 constexpr int kFusedCUs = 256;
-// waves per SIMD (workgroups per CU) that the registers of a wave's rows, two tiles' products
-// and the sums leave room for
-constexpr int fused_waves(int terms, int nks, bool exact) { return nks <= (terms == 3 ? 6 : 4) ? 2 : 1; }
+// Waves per SIMD (workgroups per CU) that the registers of a wave's rows, two tiles' products
+// and the sums leave room for.  One is enough beside the overlap (us per 20000 x 20000 sweep, before
+// it at two waves / now at one): d = 66 with 6 terms 413 / 346, d = 96 485 / 394, d = 120 769 / 527
+// (with 3 terms 367 / 320).
+constexpr int fused_waves(int terms, int nks) { return nks <= (terms == 3 ? 6 : 4) ? 2 : 1; }
 constexpr int kFusedBoxWords = 16 * kFThreads * (2 * kFusedCUs + 1);  // 8-byte words, FP32 sums
 
 // ---------------------------------------------------------------------------
@@ -191,7 +193,7 @@ __device__ __forceinline__ bool fused_take(unsigned long long *box, unsigned tag
 // the row and column sums of the duality-gap pass; otherwise v_exp_f32 of the
 // exponent rounded to FP32 and FP32 lane sums (the sweeps)
 template <int TERMS, int NKS, bool EXACT>
-__global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS, EXACT)) void fused_lse_kernel(FusedArgs fa) {
+__global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS)) void fused_lse_kernel(FusedArgs fa) {
     constexpr int NP = TERMS == 3 ? 2 : 3;  // pieces per point
     constexpr int KP = NKS * 16;
     constexpr int CHUNKS = NP * KP / 8;      // 16-byte chunks per point
@@ -597,7 +599,7 @@ static void launch_fused(FusedArgs fa, hipStream_t s) {
     // equal runs once every place has a unit (568 units: 79 us, as whole units 82); below that cutting
     // only adds hand-overs (376 units on 256 places: 49 us, whole units 42)
     const int units = fa.row_blocks * fa.n_split;
-    const int resident = kFusedCUs * fused_waves(TERMS, NKS, EXACT);
+    const int resident = kFusedCUs * fused_waves(TERMS, NKS);
     const int grid = std::min(units, resident);
     fa.whole = units == grid;
     fused_lse_kernel<TERMS, NKS, EXACT><<<(unsigned)grid, kFThreads, 0, s>>>(fa);

@@ -547,7 +547,8 @@ __global__ __launch_bounds__(1024) void gap_finish_kernel(GapArgs ga) {
 // column sums stay in registers, a row's sum is reduced over the wave; both go out as
 // partials per tile and are added in order.  Bound: FP64 issue, 28 operations per entry
 // (0.19 ms at 15000 x 15000) beside 0.17 ms of HBM; the two passes over C and C^T it
-// replaces took 0.25 + 0.21 ms alone and 0.47 + 0.28 ms next to the running sweeps.
+// replaces took 0.25 + 0.21 ms alone and 0.47 + 0.28 ms next to the running sweeps; this takes
+// 0.40 ms next to them.
 // ---------------------------------------------------------------------------
 constexpr int kGapRows = 128, kGapCols = 1024;
 
