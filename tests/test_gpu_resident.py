@@ -110,3 +110,19 @@ def test_two_streams_and_threads_at_once():
     for t in ts:
         t.join()
     assert torch.equal(out[0], ref) and torch.equal(out[1], ref)
+
+
+@pytest.mark.parametrize('kw', [dict(tolerance=1e-2), dict(batch_size=1000)])
+def test_first_duality_check_converges(kw):
+    """The check behind the sum of K-tilde decides: its sums are complete in every workgroup or the solve stalls."""
+    from oracle import ot_oracle as O
+    import wot_amd.ot as ot
+    x, y, g = _pair(300, 360, 1)
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, batch_size=5, tolerance=1e-8, tau=1e4, epsilon0=1.0,
+               max_iter=1e7)
+    prm.update(kw)
+    st, so = {}, {}
+    R = ot.optimal_transport_duality_gap(ot.DeviceCost.from_coordinates(x, y), g, stats=st, **prm)
+    ref = O.optimal_transport_duality_gap(O.default_cost_matrix(x, y), G=g, stats=so, **prm)
+    assert st['iterations'] == so['iterations']
+    assert np.linalg.norm(R - ref) / np.linalg.norm(ref) < 1e-5

@@ -362,13 +362,13 @@ struct Solver {
             if (lane == 0) sh.wsum[tid >> 6][q] = t;
         }
         __syncthreads();
+        // the next check's buffer held the check before the last one, which everybody had added up
+        // before publishing the last one's sums; all its words, whatever the checks' widths
+        if (tid < kSums) store_x(a.sums + ((int64_t)after * kMaxWg + wg) * kSums + tid, kEmpty);
         if (tid < n) {
             double t = sh.wsum[0][tid];
             for (int w = 1; w < 16; ++w) t += sh.wsum[w][tid];
-            // the next check's buffer held the check before the last one, which everybody had
-            // added up before publishing the last one's sums
-            store_x(a.sums + ((int64_t)after * kMaxWg + wg) * kSums + tid, kEmpty);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied words of this wave first
             store_x(a.sums + ((int64_t)p * kMaxWg + wg) * kSums + tid, pack(t));
         }
         const int w = tid >> 6;
