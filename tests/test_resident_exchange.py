@@ -12,10 +12,20 @@ KSUMS = 8
 class Rules:
     """What the kernel does; the defects the model has to see are variants of it."""
     words_emptied = staticmethod(lambda n: KSUMS)   # of the next check's sums, at a check of n values
+    read_all = False        # workgroups without rows on a side take the other side's potentials too
+    flag_buffers = 3        # of the tau check's maxima
 
 
 class NarrowSums(Rules):
     words_emptied = staticmethod(lambda n: n)
+
+
+class ReadAll(Rules):
+    read_all = True
+
+
+class TwoFlagBuffers(Rules):
+    flag_buffers = 2
 
 
 def program(wg, own, steps, rules):
@@ -24,7 +34,9 @@ def program(wg, own, steps, rules):
     f_own, g_own = [w for w in range(n_wg) if own[w][0]], [w for w in range(n_wg) if own[w][1]]
     has_f, has_g = own[wg]
     ops = []
-    it = chk = 0
+    it = chk = published = 0
+    flags_open = False
+    tau = any(s != 'iterate' for s in steps)  # the duality-gap schedule
 
     def sums(n):
         nonlocal chk
@@ -37,30 +49,48 @@ def program(wg, own, steps, rules):
             for b in range(n_wg):
                 ops.append(('r', ('s', chk % 3, b, q), chk))
 
+    def absorb():
+        nonlocal flags_open
+        if flags_open:
+            for b in range(n_wg):
+                ops.append(('r', ('t', published % rules.flag_buffers, b), published))
+        flags_open = False
+
     for step in steps:
         if step == 'iterate':
             it += 1
             p, old = it % 2, (it - 1) % 2
-            if it > 1:
+            if it > 1 and (has_f or rules.read_all):
                 for b in g_own:
                     ops.append(('r', ('g', old, b), it - 1))
-                if has_f:
-                    ops.append(('w', ('f', old, wg), None))
+            absorb()
             if has_f:
+                if it > 1:
+                    ops.append(('w', ('f', old, wg), None))
                 ops.append(('w', ('f', p, wg), it))
-            for b in f_own:
-                ops.append(('r', ('f', p, b), it))
+            if has_g or rules.read_all:
+                for b in f_own:
+                    ops.append(('r', ('f', p, b), it))
             if has_g and it > 1:
                 ops.append(('w', ('g', old, wg), None))
+            if rules.flag_buffers == 2 and tau and it > 1:
+                ops.append(('w', ('t', old, wg), None))
             if has_g:
                 ops.append(('w', ('g', p, wg), it))
+            if tau:
+                if rules.flag_buffers == 3:
+                    ops.append(('w', ('t', (it + 1) % 3, wg), None))
+                ops.append(('w', ('t', it % rules.flag_buffers, wg), it))
+                flags_open, published = True, it
         elif step == 'duality':
+            absorb()
             for b in g_own:
                 ops.append(('r', ('g', it % 2, b), it))
             for b in f_own:
                 ops.append(('r', ('f', it % 2, b), it))
             sums(7)
         else:  # a check of so many sums
+            absorb()
             sums(step)
     return ops
 
@@ -117,7 +147,28 @@ def outcomes(own, steps, rules):
 GAP = (['iterate'] * 3 + [4]) * 2 + [1] + ['iterate'] * 2 + ['duality'] + ['iterate'] * 2 + ['duality']
 
 
+FIXED = ['iterate'] * 7
+# workgroups 2 and 3 without rows of C (300 x 400, 900 x 8000), without rows of C^T
+WIDE = [(True, True)] * 2 + [(False, True)] * 2
+TALL = [(True, True)] * 2 + [(True, False)] * 2
+
+
 def test_sums_of_checks_of_different_widths():
     own = [(True, True)] * 4
     assert outcomes(own, GAP, Rules) == set()
     assert 'stale' in outcomes(own, GAP, NarrowSums)
+
+
+@pytest.mark.parametrize('own', [WIDE, TALL, [(True, True), (False, True)], [(True, False), (True, True)]])
+@pytest.mark.parametrize('steps', [FIXED, GAP])
+def test_workgroups_without_rows_on_a_side(own, steps):
+    assert outcomes(own, steps, Rules) == set()
+
+
+@pytest.mark.parametrize('own,steps', [(WIDE, FIXED), (WIDE, GAP), (TALL, FIXED)])
+def test_reading_what_one_does_not_need_stalls(own, steps):
+    assert 'stall' in outcomes(own, steps, ReadAll)
+
+
+def test_two_buffers_of_maxima_stall():
+    assert 'stall' in outcomes(WIDE, GAP, TwoFlagBuffers)

@@ -17,12 +17,17 @@
 // Exchange.  A potential travels as its 8 bytes in one of two buffers (parity of the
 // iteration); a buffer not yet written holds kEmpty, a NaN pattern no result has, and
 // readers poll the values themselves: one store and one load stand between a producer
-// and a consumer, no counter, no barrier.  Reuse is safe by data flow: whoever has all
-// of g_n knows that every workgroup has read all of f_n, since each published its part of
-// g_n after that; so the owner of f_n+1 may empty the buffer of f_n then, and
-// waits for those stores before it publishes f_n+1, which every poller of f_n+2 has
-// read.  The tau check's maxima and the gap sums travel the same way, once per
-// workgroup; every workgroup adds them up in the same order and takes the same decisions.
+// and a consumer, no counter, no barrier.  Reuse is safe by data flow: only workgroups with rows of
+// C read g_n, and each publishes its part of f_n+1 after that, so whoever has all of f_n+1 knows
+// that g_n has been read and may empty its part of it; it waits for those stores before it
+// publishes its part of g_n+1, which every poller of g_n+2 has read.  The same holds for f_n, its
+// readers (the workgroups with rows of C^T) and g_n.  (A workgroup without rows on a side, such as
+// 25 of 100 at 300 x 400, publishes nothing there that could tell that it has read the other
+// side, so it does not read it.)  The tau check's maxima and the gap sums are read by every workgroup
+// and published by every workgroup, in three buffers: whoever has all of one step's has proof that
+// everybody has read the step before, and empties that one's buffer, the next step's, before it
+// publishes its own.  Every workgroup adds them up in the same order and takes the same decisions.
+// tests/test_resident_exchange.py holds a model of this that delays workgroups at will.
 //
 // Progress.  The launch is cooperative: all workgroups are resident or none runs, and
 // two such launches do not share the device.  Every wait is bounded (kWaitSeconds): a
@@ -67,7 +72,7 @@ struct GapParams {
 struct Args {
     ResidentProblem rp;
     u64 *fx, *gx;     // [2][n] exchange
-    u64 *flags;       // [2][kMaxWg]
+    u64 *flags;       // [3][kMaxWg]
     u64 *sums;        // [3][kMaxWg * kSums]
     ResidentResult *res;
     int n_wg;
@@ -156,7 +161,9 @@ struct Solver {
     f4 c[S], ct[S];               // this thread's pieces of its team's C and C^T rows
     // owner threads (tid < kMaxOwn): the workgroup's rows tid
     int row_f, row_g;             // or -1
+    bool has_f, has_g;            // whether the workgroup owns rows of C / of C^T
     int pf;                       // parity of the last published f and g
+    int pt;                       // buffer of the last published maxima
     int pc;                       // buffer of the last published sums
     bool flag_open;               // the last iteration's maxima have not been read yet
 
@@ -270,55 +277,64 @@ struct Solver {
         return alpha * eps * (lw + log_n - lse);
     }
 
-    // one (a, b) iteration; tau >= 0 also publishes the workgroup's largest growth since the absorption
+    // one (a, b) iteration; checks: also publishes the workgroup's largest growth since the absorption
     __device__ bool iterate(double eps, bool first, bool checks) {
         const double k = kLog2E / eps, inv_eps = 1.0 / eps;
         const double al1 = a.lambda1 / (a.lambda1 + eps), al2 = a.lambda2 / (a.lambda2 + eps);
         const int n_i = a.rp.n_i, n_j = a.rp.n_j;
-        if (first) {
-            for (int j = tid; j < n_j; j += kT) hg[place(j)] = a.rp.g[j] * k;
-        } else {
-            take(a.gx + (int64_t)pf * n_j, n_j, hg, k);
+        if (has_f) {
+            if (first) {
+                for (int j = tid; j < n_j; j += kT) hg[place(j)] = a.rp.g[j] * k;
+            } else {
+                take(a.gx + (int64_t)pf * n_j, n_j, hg, k);
+            }
         }
         if (!sync_ok()) return false;
         if (checks && flag_open && !absorb()) return false;
-        const int p = pf ^ 1;  // this iteration's buffers; the other ones hold what everybody has read
-        if (row_f >= 0 && !first) store_x(a.fx + (int64_t)pf * n_i + row_f, kEmpty);
-        sweep(c, a.rf, a.cf, hg, k);
-        __syncthreads();
-        if (row_f >= 0) {
-            sh.fp[tid] = sh.f[tid];
-            sh.up[tid] = sh.u[tid];
-            const double f = potential(sh.lw[tid], a.log_nj, al1, eps);
-            sh.f[tid] = f;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied buffer first
-            store_x(a.fx + (int64_t)p * n_i + row_f, pack(f));
+        const int p = pf ^ 1;  // this iteration's buffers; the other ones hold what their readers have read
+        if (has_f) {
+            if (row_f >= 0 && !first) store_x(a.fx + (int64_t)pf * n_i + row_f, kEmpty);
+            sweep(c, a.rf, a.cf, hg, k);
+            __syncthreads();
+            if (row_f >= 0) {
+                sh.fp[tid] = sh.f[tid];
+                sh.up[tid] = sh.u[tid];
+                const double f = potential(sh.lw[tid], a.log_nj, al1, eps);
+                sh.f[tid] = f;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied buffer first
+                store_x(a.fx + (int64_t)p * n_i + row_f, pack(f));
+            }
         }
-        take(a.fx + (int64_t)p * n_i, n_i, hf, k);
+        if (has_g) take(a.fx + (int64_t)p * n_i, n_i, hf, k);
         if (!sync_ok()) return false;
-        if (!first) {
-            if (row_g >= 0) store_x(a.gx + (int64_t)pf * n_j + row_g, kEmpty);
-            if (checks && tid == 0) store_x(a.flags + (int64_t)pf * kMaxWg + wg, kEmpty);
-        }
-        sweep(ct, a.rg, a.cg, hf, k);
-        __syncthreads();
         double grown = -INFINITY;
-        if (row_g >= 0) {
-            sh.gp[tid] = sh.g[tid];
-            sh.vp[tid] = sh.v[tid];
-            const double g = potential(a.rp.misc[0], a.log_ni, al2, eps);
-            sh.g[tid] = g;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            store_x(a.gx + (int64_t)p * n_j + row_g, pack(g));
-            grown = (g - sh.v[tid]) * inv_eps;
+        if (has_g) {
+            if (row_g >= 0 && !first) store_x(a.gx + (int64_t)pf * n_j + row_g, kEmpty);
+            sweep(ct, a.rg, a.cg, hf, k);
+            __syncthreads();
+            if (row_g >= 0) {
+                sh.gp[tid] = sh.g[tid];
+                sh.vp[tid] = sh.v[tid];
+                const double g = potential(a.rp.misc[0], a.log_ni, al2, eps);
+                sh.g[tid] = g;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                store_x(a.gx + (int64_t)p * n_j + row_g, pack(g));
+                grown = (g - sh.v[tid]) * inv_eps;
+            }
         }
         if (checks) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (row_f >= 0) grown = fmax(grown, (sh.f[tid] - sh.u[tid]) * inv_eps);
+            const int q = pt == 2 ? 0 : pt + 1, after = q == 2 ? 0 : q + 1;
             if (tid < 64) {
                 grown = wave_max64(grown);
-                if (tid == 0) store_x(a.flags + (int64_t)p * kMaxWg + wg, pack(grown));
+                if (tid == 0) {
+                    // the next iteration's buffer held the maxima before the last ones
+                    store_x(a.flags + (int64_t)after * kMaxWg + wg, kEmpty);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    store_x(a.flags + (int64_t)q * kMaxWg + wg, pack(grown));
+                }
             }
+            pt = q;
             flag_open = true;
         }
         pf = p;
@@ -330,8 +346,8 @@ struct Solver {
     __device__ bool absorb() {
         double m = -INFINITY;
         if (tid < a.n_wg) {
-            u64 x = load_x(a.flags + (int64_t)pf * kMaxWg + tid);
-            if (wait_value(a.flags + (int64_t)pf * kMaxWg + tid, x)) m = unpack(x);
+            u64 x = load_x(a.flags + (int64_t)pt * kMaxWg + tid);
+            if (wait_value(a.flags + (int64_t)pt * kMaxWg + tid, x)) m = unpack(x);
         }
         m = wave_max64(m);
         if (lane == 0) sh.wsum[tid >> 6][0] = m;
@@ -562,7 +578,10 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
         sh.g[tid] = sh.v[tid] = sh.gp[tid] = sh.vp[tid] = so.row_g >= 0 ? a.rp.g[so.row_g] : 0.0;
         sh.lw[tid] = so.row_f >= 0 ? a.rp.logp[so.row_f] : 0.0;
     }
+    so.has_f = wg * kTeams < n_i;
+    so.has_g = wg * kTeams < n_j;
     so.pf = 1;
+    so.pt = 2;
     so.pc = 2;
     so.flag_open = false;
     so.n_stab = 0;
@@ -625,7 +644,7 @@ Exchange carve(void *base, int64_t I, int64_t J) {
     Exchange e;
     e.res = static_cast<ResidentResult *>(base);
     e.x = reinterpret_cast<u64 *>(static_cast<char *>(base) + 256);
-    e.n = 2 * (I + J) + 2 * kMaxWg + 3 * kMaxWg * kSums;
+    e.n = 2 * (I + J) + 3 * kMaxWg + 3 * kMaxWg * kSums;
     return e;
 }
 
@@ -662,7 +681,7 @@ Args make_args(const ResidentProblem &rp, const Shape &sh, double lambda1, doubl
     a.fx = e.x;
     a.gx = a.fx + 2 * (int64_t)rp.n_i;
     a.flags = a.gx + 2 * (int64_t)rp.n_j;
-    a.sums = a.flags + 2 * kMaxWg;
+    a.sums = a.flags + 3 * kMaxWg;
     a.res = e.res;
     a.n_wg = sh.n_wg;
     a.rf = sh.rf;
