@@ -149,7 +149,7 @@ struct Shared {
     // owned rows: potentials, absorbed potentials, both before the last iteration, log weight
     double f[kMaxOwn], u[kMaxOwn], fp[kMaxOwn], up[kMaxOwn], lw[kMaxOwn];
     double g[kMaxOwn], v[kMaxOwn], gp[kMaxOwn], vp[kMaxOwn];
-    int aborted;
+    int aborted[2];               // by the parity of sync_ok's calls
 };
 
 template <int S>
@@ -165,6 +165,7 @@ struct Solver {
     int pf;                       // parity of the last published f and g
     int pt;                       // buffer of the last published maxima
     int pc;                       // buffer of the last published sums
+    int phase;                    // of sync_ok
     bool flag_open;               // the last iteration's maxima have not been read yet
 
     // LDS place of potential j: float4 group t of chunk m, halves apart (16-byte lane stride)
@@ -197,7 +198,7 @@ struct Solver {
                 if (__hip_atomic_load(&a.res->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
                     wall_clock64() - start > kWaitTicks) {
                     __hip_atomic_store(&a.res->aborted, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    sh.aborted = 1;
+                    sh.aborted[phase] = 1;
                     return false;
                 }
             }
@@ -220,10 +221,14 @@ struct Solver {
         }
     }
 
-    // ends the workgroup when any wait was given up; every thread calls it
+    // ends the workgroup when any wait was given up; every thread calls it.  Two flags in turn: a
+    // wave that is past the barrier and gives up its next wait must not change what a slower wave
+    // is about to read here, or the workgroup's waves part.
     __device__ bool sync_ok() {
         __syncthreads();
-        return sh.aborted == 0;
+        const bool ok = sh.aborted[phase] == 0;
+        phase ^= 1;
+        return ok;
     }
 
     // log-sum-exp of the team's rows over the potentials in h (times k), wave results to sh.red
@@ -514,8 +519,8 @@ struct Solver {
         return true;
     }
 
-    // the duality-gap schedule
-    __device__ void run_gap(ResidentResult &out) {
+    // the duality-gap schedule; false when a wait was given up
+    __device__ bool run_gap(ResidentResult &out) {
         const GapParams &gp_ = a.gap;
         const int n_scal = 5;
         double eps = gp_.eps0 * gp_.factor, skt = 0.0;
@@ -529,32 +534,33 @@ struct Solver {
             }
             eps = eps / gp_.factor;
             out.eps = eps;
-            if (e == n_scal && !ktilde(eps, skt)) return;
+            if (e == n_scal && !ktilde(eps, skt)) return false;
             const double thr = e == n_scal ? gp_.tolerance : 1e-6;
             const long long nb = e == n_scal ? gp_.batch : 5;
             while (out.gap > thr) {
                 for (long long t = 0; t < nb; ++t) {
                     ++out.iterations;
-                    if (!iterate(eps, first, true)) return;
+                    if (!iterate(eps, first, true)) return false;
                     first = false;
                     if (out.iterations >= gp_.max_iter) {
-                        if (!absorb()) return;
+                        if (!absorb()) return false;
                         out.max_iter_reached = 1;
                         out.stabilisations = n_stab;
-                        return;
+                        return true;
                     }
                 }
-                if (!absorb()) return;
+                if (!absorb()) return false;
                 ++out.checks;
                 if (e < n_scal) {
-                    if (!evolution(eps, out.gap)) return;
+                    if (!evolution(eps, out.gap)) return false;
                     __syncthreads();
                 } else if (!duality(eps, skt, out.primal, out.dual, out.gap)) {
-                    return;
+                    return false;
                 }
             }
         }
         out.stabilisations = n_stab;
+        return true;
     }
 };
 
@@ -565,7 +571,7 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
     const int tid = threadIdx.x, wg = blockIdx.x, n_teams = a.n_wg * kTeams;
     const int n_i = a.rp.n_i, n_j = a.rp.n_j;
     double *hf = h_lds, *hg = h_lds + 1024 * a.cg;  // cg chunks of the source side, cf of the target side
-    if (tid == 0) sh.aborted = 0;
+    if (tid < 2) sh.aborted[tid] = 0;
     for (int j = tid; j < 1024 * (a.cg + a.cf); j += kT) h_lds[j] = -INFINITY;  // padding stays so
     Solver<S> so{a, sh, hf, hg, tid, tid & 255, __builtin_amdgcn_readfirstlane(tid >> 8), (tid >> 6) & 3, tid & 63, wg,
                  n_teams};
@@ -583,12 +589,13 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
     so.pf = 1;
     so.pt = 2;
     so.pc = 2;
+    so.phase = 0;
     so.flag_open = false;
     so.n_stab = 0;
     __syncthreads();
     ResidentResult out{};
     if constexpr (GAP) {
-        so.run_gap(out);
+        if (!so.run_gap(out)) return;
     } else {
         bool first = true;
         for (int q = 0; q < seg.count; ++q)
@@ -597,7 +604,6 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
                 first = false;
             }
     }
-    if (sh.aborted) return;
     if (so.row_f >= 0) a.rp.f[so.row_f] = sh.f[tid];
     if (so.row_g >= 0) a.rp.g[so.row_g] = sh.g[tid];
     if (GAP && wg == 0 && tid == 0) {
