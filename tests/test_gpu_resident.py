@@ -126,3 +126,32 @@ def test_first_duality_check_converges(kw):
     ref = O.optimal_transport_duality_gap(O.default_cost_matrix(x, y), G=g, stats=so, **prm)
     assert st['iterations'] == so['iterations']
     assert np.linalg.norm(R - ref) / np.linalg.norm(ref) < 1e-5
+
+
+def test_threads_with_different_shapes():
+    """Pairs that need different amounts of LDS in the same instance of the kernel, from several threads."""
+    import threading
+    import torch
+    import wot_amd.ot as ot
+    shapes = [(60, 50), (1000, 900), (40, 2000), (2000, 30)]
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, scaling_iter=40, extra_iter=0, inner_iter_max=50,
+               tau=1e4, device_out=True)
+    pairs = [_pair(i, j, 3) for i, j in shapes]
+    costs = [ot.DeviceCost.from_coordinates(x, y) for x, y, _ in pairs]
+    refs = [ot.transport_stablev2(c, G=p[2], **prm) for c, p in zip(costs, pairs)]
+    torch.cuda.synchronize()
+    same = [True] * len(shapes)
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(5):
+                out = ot.transport_stablev2(costs[k], G=pairs[k][2], **prm)
+                torch.cuda.current_stream().synchronize()
+                same[k] = same[k] and torch.equal(out, refs[k])
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert all(same)

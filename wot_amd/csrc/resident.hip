@@ -50,6 +50,7 @@ constexpr int kMaxWg = 256;              // one workgroup per CU
 constexpr int kMaxSlots = 9;             // float4 per thread and side held in registers
 constexpr int kMaxOwn = 36;              // rows a workgroup may own per side (kTeams x kMaxSlots)
 constexpr int kMaxSide = 8704;           // potentials of one side in LDS (two sides: 139 KB)
+constexpr int kMaxLds = 2 * 8 * 1024 * ((kMaxSide + 1023) / 1024);  // bytes of both sides' potentials
 constexpr int kSums = 8;                 // values a workgroup contributes to a check
 constexpr int kSegments = 96;            // eps segments per launch
 constexpr int64_t kLaunchIters = 16384;  // iterations per launch
@@ -658,7 +659,9 @@ template <int S, bool GAP>
 int launch(Args &a, Segments &seg, int *launched, hipStream_t s) {
     const int lds = (int)sizeof(double) * 1024 * (a.cf + a.cg);
     const void *fn = reinterpret_cast<const void *>(resident_kernel<S, GAP>);
-    WOTK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    // the limit belongs to the function, not to the launch: the largest any pair needs, so that
+    // threads with pairs of different shapes set the same
+    WOTK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
     int per_cu = 0, dev = 0, cus = 0, coop = 0;
     WOTK_HIP(hipGetDevice(&dev));
     WOTK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
