@@ -155,3 +155,17 @@ def test_threads_with_different_shapes():
     for t in ts:
         t.join()
     assert all(same)
+
+
+def test_duality_gap_over_several_launches():
+    """An unattainable tolerance: more iterations than one launch takes, with absorptions on both sides of the cut."""
+    from oracle import ot_oracle as O
+    import wot_amd.ot as ot
+    x, y, g = _pair(60, 50, 1)
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, batch_size=7, tolerance=-1.0, tau=1.0, epsilon0=1.0,
+               max_iter=16390)
+    st, so = {}, {}
+    R = ot.optimal_transport_duality_gap(ot.DeviceCost.from_coordinates(x, y), g, stats=st, **prm)
+    ref = O.optimal_transport_duality_gap(O.default_cost_matrix(x, y), G=g, stats=so, **prm)
+    assert st['iterations'] == so['iterations'] == 16390 and st['max_iter_reached'] and so['max_iter_reached']
+    assert np.linalg.norm(R - ref) / np.linalg.norm(ref) < 1e-5

@@ -26,6 +26,7 @@ struct ResidentProblem {
     const double *logp;  // log G_i
     const double *misc;  // [0] log mean G, [1] mean G
     double *f, *g;       // potentials: start values in, results out
+    double *u, *v;       // absorbed potentials where a launch of the duality-gap schedule stopped
     void *exchange;      // resident_bytes
 };
 
@@ -35,6 +36,11 @@ struct ResidentResult {
     int max_iter_reached;
     long long iterations, stabilisations, checks;
     double gap, primal, dual, eps;
+    // duality-gap schedule: the launch has done its iterations and the next one goes on from f, g, u,
+    // v, this scaling, so many iterations into its batch
+    int stopped, scaling;
+    long long in_batch;
+    double sum_ktilde;
 };
 
 // The fixed-iteration schedule (optimal_transport.py:167-236).  *launched is 0 when the
@@ -42,9 +48,11 @@ struct ResidentResult {
 int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, double epsilon0,
                    int64_t scaling_iter, int64_t inner_iter_max, int64_t extra_iter, int *launched, hipStream_t s);
 
-// the duality-gap schedule (optimal_transport.py:67-164) up to its last iteration
+// the duality-gap schedule (optimal_transport.py:67-164) up to its last iteration; *out is its
+// outcome when *launched (waits for it)
 int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, long long batch_size,
-                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched, hipStream_t s);
+                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched,
+                 ResidentResult *out, hipStream_t s);
 
 // the result of the last resident launch on rp (waits for it)
 int resident_result(const ResidentProblem &rp, ResidentResult *out, hipStream_t s);

@@ -53,7 +53,9 @@ constexpr int kMaxSide = 8704;           // potentials of one side in LDS (two s
 constexpr int kMaxLds = 2 * 8 * 1024 * ((kMaxSide + 1023) / 1024);  // bytes of both sides' potentials
 constexpr int kSums = 8;                 // values a workgroup contributes to a check
 constexpr int kSegments = 96;            // eps segments per launch
-constexpr int64_t kLaunchIters = 16384;  // iterations per launch
+// iterations per launch: 0.08 to 0.25 s, so that no launch holds the chip for long however many
+// iterations a schedule takes
+constexpr int64_t kLaunchIters = 16384;
 constexpr u64 kEmpty = 0x7ffddeadc0ffee01ull;
 constexpr u64 kPlainNan = 0x7ff8000000000000ull;
 constexpr long long kWaitTicks = 20ll * 100000000ll;  // 20 s of the 100 MHz clock
@@ -66,8 +68,9 @@ struct Segments {
 };
 
 struct GapParams {
-    double factor, eps0, tolerance, tau;
-    long long batch, max_iter;
+    double factor, tolerance, tau;
+    long long batch, max_iter, launch_iters;
+    ResidentResult from;  // the state at the launch: all zero but eps, or where the last launch stopped
 };
 
 struct Args {
@@ -520,28 +523,40 @@ struct Solver {
         return true;
     }
 
-    // the duality-gap schedule; false when a wait was given up
+    // the duality-gap schedule, at most launch_iters iterations of it; false when a wait was given up
     __device__ bool run_gap(ResidentResult &out) {
         const GapParams &gp_ = a.gap;
         const int n_scal = 5;
-        double eps = gp_.eps0 * gp_.factor, skt = 0.0;
-        bool first = true;
-        out.gap = INFINITY;
-        for (int e = 0; e <= n_scal; ++e) {
-            out.gap = INFINITY;
-            if (tid < kMaxOwn) {
-                sh.u[tid] = sh.f[tid];
-                sh.v[tid] = sh.g[tid];
+        out = gp_.from;
+        out.stopped = 0;
+        bool resumed = gp_.from.stopped, first = true;
+        const long long stop_at = out.iterations + gp_.launch_iters;
+        long long t = out.in_batch;
+        for (int e = out.scaling; e <= n_scal; ++e) {
+            if (!resumed) {
+                out.gap = INFINITY;
+                if (tid < kMaxOwn) {
+                    sh.u[tid] = sh.f[tid];
+                    sh.v[tid] = sh.g[tid];
+                }
+                out.eps = out.eps / gp_.factor;
+                if (e == n_scal && !ktilde(out.eps, out.sum_ktilde)) return false;
             }
-            eps = eps / gp_.factor;
-            out.eps = eps;
-            if (e == n_scal && !ktilde(eps, skt)) return false;
+            resumed = false;
             const double thr = e == n_scal ? gp_.tolerance : 1e-6;
             const long long nb = e == n_scal ? gp_.batch : 5;
             while (out.gap > thr) {
-                for (long long t = 0; t < nb; ++t) {
+                for (; t < nb; ++t) {
+                    if (out.iterations == stop_at) {  // every workgroup counts the same
+                        if (flag_open && !absorb()) return false;
+                        out.stopped = 1;
+                        out.scaling = e;
+                        out.in_batch = t;
+                        out.stabilisations = n_stab;
+                        return true;
+                    }
                     ++out.iterations;
-                    if (!iterate(eps, first, true)) return false;
+                    if (!iterate(out.eps, first, true)) return false;
                     first = false;
                     if (out.iterations >= gp_.max_iter) {
                         if (!absorb()) return false;
@@ -550,12 +565,13 @@ struct Solver {
                         return true;
                     }
                 }
+                t = 0;
                 if (!absorb()) return false;
                 ++out.checks;
                 if (e < n_scal) {
-                    if (!evolution(eps, out.gap)) return false;
+                    if (!evolution(out.eps, out.gap)) return false;
                     __syncthreads();
-                } else if (!duality(eps, skt, out.primal, out.dual, out.gap)) {
+                } else if (!duality(out.eps, out.sum_ktilde, out.primal, out.dual, out.gap)) {
                     return false;
                 }
             }
@@ -584,6 +600,10 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
         sh.f[tid] = sh.u[tid] = sh.fp[tid] = sh.up[tid] = so.row_f >= 0 ? a.rp.f[so.row_f] : 0.0;
         sh.g[tid] = sh.v[tid] = sh.gp[tid] = sh.vp[tid] = so.row_g >= 0 ? a.rp.g[so.row_g] : 0.0;
         sh.lw[tid] = so.row_f >= 0 ? a.rp.logp[so.row_f] : 0.0;
+        if (GAP && a.gap.from.stopped) {
+            if (so.row_f >= 0) sh.u[tid] = a.rp.u[so.row_f];
+            if (so.row_g >= 0) sh.v[tid] = a.rp.v[so.row_g];
+        }
     }
     so.has_f = wg * kTeams < n_i;
     so.has_g = wg * kTeams < n_j;
@@ -592,7 +612,7 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
     so.pc = 2;
     so.phase = 0;
     so.flag_open = false;
-    so.n_stab = 0;
+    so.n_stab = a.gap.from.stabilisations;
     __syncthreads();
     ResidentResult out{};
     if constexpr (GAP) {
@@ -607,15 +627,26 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
     }
     if (so.row_f >= 0) a.rp.f[so.row_f] = sh.f[tid];
     if (so.row_g >= 0) a.rp.g[so.row_g] = sh.g[tid];
-    if (GAP && wg == 0 && tid == 0) {
-        a.res->max_iter_reached = out.max_iter_reached;
-        a.res->iterations = out.iterations;
-        a.res->stabilisations = out.stabilisations;
-        a.res->checks = out.checks;
-        a.res->gap = out.gap;
-        a.res->primal = out.primal;
-        a.res->dual = out.dual;
-        a.res->eps = out.eps;
+    if constexpr (GAP) {
+        if (out.stopped) {
+            if (so.row_f >= 0) a.rp.u[so.row_f] = sh.u[tid];
+            if (so.row_g >= 0) a.rp.v[so.row_g] = sh.v[tid];
+        }
+        if (wg == 0 && tid == 0) {
+            ResidentResult &r = *a.res;  // all but the flag that any workgroup may raise
+            r.max_iter_reached = out.max_iter_reached;
+            r.iterations = out.iterations;
+            r.stabilisations = out.stabilisations;
+            r.checks = out.checks;
+            r.gap = out.gap;
+            r.primal = out.primal;
+            r.dual = out.dual;
+            r.eps = out.eps;
+            r.stopped = out.stopped;
+            r.scaling = out.scaling;
+            r.in_batch = out.in_batch;
+            r.sum_ktilde = out.sum_ktilde;
+        }
     }
 }
 
@@ -759,14 +790,24 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
 }
 
 int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, long long batch_size,
-                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched, hipStream_t s) {
+                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched,
+                 ResidentResult *out, hipStream_t s) {
     const Shape sh = shape_of(rp.n_i, rp.n_j);
-    int rc = clear(rp, s);
-    if (rc) return rc;
-    Args a = make_args(rp, sh, lambda1, lambda2);
-    a.gap = GapParams{std::exp(-std::log(epsilon) / 5), epsilon0, tolerance, tau, batch_size, max_iter};
-    Segments seg{};
-    return dispatch<true>(a, seg, sh.slots, launched, s);
+    const double factor = std::exp(-std::log(epsilon) / 5);
+    *out = ResidentResult{};
+    out->eps = epsilon0 * factor;
+    do {
+        int rc = clear(rp, s);
+        if (rc) return rc;
+        Args a = make_args(rp, sh, lambda1, lambda2);
+        a.gap = GapParams{factor, tolerance, tau, batch_size, max_iter, kLaunchIters, *out};
+        Segments seg{};
+        rc = dispatch<true>(a, seg, sh.slots, launched, s);
+        if (rc || !*launched) return rc;
+        rc = resident_result(rp, out, s);
+        if (rc) return rc;
+    } while (out->stopped && !out->aborted);
+    return WOTK_OK;
 }
 
 int resident_result(const ResidentProblem &rp, ResidentResult *out, hipStream_t s) {

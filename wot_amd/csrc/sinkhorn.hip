@@ -974,7 +974,8 @@ struct EventPair {
 };
 
 static ResidentProblem resident_problem(const Problem &pb, const Work &w) {
-    return ResidentProblem{pb.C, pb.ldc, pb.CT, pb.ldct, pb.n_i, pb.n_j, pb.G, w.logp, w.misc, w.f, w.g, w.exchange};
+    return ResidentProblem{pb.C, pb.ldc, pb.CT, pb.ldct, pb.n_i, pb.n_j, pb.G, w.logp, w.misc, w.f, w.g, w.u, w.v,
+                           w.exchange};
 }
 
 // the fixed-iteration schedule on a set-up problem (shared by the workspace
@@ -1010,9 +1011,9 @@ static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambd
             rc = resident_result(rp, &r, s);
             if (rc) return rc;
             done = !r.aborted;
-            if (!done) rc = init_state(pb, w, s);
-            if (rc) return rc;
         }
+        if (!done) rc = init_state(pb, w, s);  // an earlier launch of the schedule may have moved it
+        if (rc) return rc;
     }
     if (!done) {
         for (int64_t n = 0; n < scaling_iter; ++n) {
@@ -1373,37 +1374,34 @@ extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const flo
         WOTK_REQUIRE(batch_size > 0, "batch_size must be positive");
         const ResidentProblem rp = resident_problem(pb, w);
         int launched = 0;
-        rc = resident_gap(rp, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, &launched, s);
+        ResidentResult r;
+        rc = resident_gap(rp, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, &launched,
+                          &r, s);
         if (rc) return rc;
-        if (launched) {
-            ResidentResult r;
-            rc = resident_result(rp, &r, s);
-            if (rc) return rc;
-            if (!r.aborted) {
-                if (stats) {
-                    *stats = wotk_stats{};
-                    stats->iterations = r.iterations;
-                    stats->stabilisations = r.stabilisations;
-                    stats->gap_checks = r.checks;
-                    stats->gap = r.gap;
-                    stats->epsilon_final = r.eps;
-                    stats->max_iter_reached = r.max_iter_reached;
-                    if (!r.max_iter_reached) {
-                        stats->primal = r.primal;
-                        stats->dual = r.dual;
-                    }
+        if (launched && !r.aborted) {
+            if (stats) {
+                *stats = wotk_stats{};
+                stats->iterations = r.iterations;
+                stats->stabilisations = r.stabilisations;
+                stats->gap_checks = r.checks;
+                stats->gap = r.gap;
+                stats->epsilon_final = r.eps;
+                stats->max_iter_reached = r.max_iter_reached;
+                if (!r.max_iter_reached) {
+                    stats->primal = r.primal;
+                    stats->dual = r.dual;
                 }
-                if (!r.max_iter_reached && std::isnan(r.gap))
-                    return fail(WOTK_ENAN,
-                                "Overflow encountered in duality gap computation, please report this incident");
-                rc = be.finish(r.eps, r.max_iter_reached ? 1.0 : (double)J, s);
-                if (rc) return rc;
-                WOTK_HIP(hipStreamSynchronize(s));
-                return WOTK_OK;
             }
-            rc = init_state(pb, w, s);
+            if (!r.max_iter_reached && std::isnan(r.gap))
+                return fail(WOTK_ENAN,
+                            "Overflow encountered in duality gap computation, please report this incident");
+            rc = be.finish(r.eps, r.max_iter_reached ? 1.0 : (double)J, s);
             if (rc) return rc;
+            WOTK_HIP(hipStreamSynchronize(s));
+            return WOTK_OK;
         }
+        rc = init_state(pb, w, s);  // an earlier launch of the schedule may have moved it
+        if (rc) return rc;
     }
     return gap_schedule(be, pb, w, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, stats,
                         s);
