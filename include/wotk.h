@@ -155,6 +155,18 @@ int wotk_transport_duality_gap(const float *C, int64_t ldc, const float *CT, int
                                double *g_out, void *workspace, size_t workspace_bytes,
                                wotk_stats *stats, void *stream);
 
+/* How the last wotk_transport_stablev2 / wotk_transport_duality_gap call of an
+ * I x J pair on `workspace` ran (no counterpart in the reference): *route
+ * (HOST) is one of WOTK_ROUTE_*; *launches (HOST) the persistent launches of
+ * the resident solver.  The routes differ in time, and the resident one has
+ * the sweeps' bits.  Waits for the stream. */
+#define WOTK_ROUTE_SWEEPS 0    /* two launched sweeps per iteration                          */
+#define WOTK_ROUTE_ONE_READ 1  /* the iteration over one read of C                           */
+#define WOTK_ROUTE_RESIDENT 2  /* persistent launches                                        */
+#define WOTK_ROUTE_GAVE_UP 3   /* a wait of a persistent launch ran out: repeated by sweeps  */
+int wotk_solver_route(int64_t I, int64_t J, const void *workspace, size_t workspace_bytes, int32_t *route,
+                      int64_t *launches, void *stream);
+
 /* The plan exp((f_i + g_j - C_ij)/eps) / divisor (I x J, ldp, FP64) and/or its
  * row sums from potentials: optimal_transport.py:234-236 (R / J) and :145
  * (divisor 1).  plan or row_sums may be NULL. */

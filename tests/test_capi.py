@@ -96,3 +96,14 @@ def test_emd_is_host_code():
     M = np.array([[0.0, 2.0], [1.0, 0.0]])
     assert emd2(np.array([0.5, 0.5]), np.array([0.5, 0.5]), M) == 0.0
     assert emd2(np.array([1.0, 0.0]), np.array([0.0, 1.0]), M) == 2.0
+
+
+def test_solver_route_checks_its_arguments_on_the_host():
+    import ctypes
+    lib = _native.lib()
+    route, launches = ctypes.c_int32(), ctypes.c_int64()
+    out = ctypes.byref(route), ctypes.byref(launches)
+    assert lib.wotk_solver_route(0, 5, 256, 1 << 20, *out, None) == _native.WOTK_EINVAL
+    assert lib.wotk_solver_route(40, 50, 256, 1 << 20, None, None, None) == _native.WOTK_EINVAL
+    assert lib.wotk_solver_route(40, 50, None, 1 << 20, *out, None) == _native.WOTK_EWORKSPACE
+    assert lib.wotk_solver_route(40, 50, 256, 64, *out, None) == _native.WOTK_EWORKSPACE

@@ -169,3 +169,116 @@ def test_duality_gap_over_several_launches():
     ref = O.optimal_transport_duality_gap(O.default_cost_matrix(x, y), G=g, stats=so, **prm)
     assert st['iterations'] == so['iterations'] == 16390 and st['max_iter_reached'] and so['max_iter_reached']
     assert np.linalg.norm(R - ref) / np.linalg.norm(ref) < 1e-5
+
+
+# ---- the route: a solve that was refused or given up has the same bits, so the tests above cannot see it ----
+def _route(ws, n_i, n_j):
+    import ctypes
+    import torch
+    from wot_amd import _native
+    route, launches = ctypes.c_int32(-1), ctypes.c_int64(-1)
+    _native.check(_native.lib().wotk_solver_route(n_i, n_j, ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+                                                  ctypes.byref(route), ctypes.byref(launches),
+                                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    return route.value, launches.value
+
+
+def _workspace(n_i, n_j):
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    ws = dev.workspace(torch, _native.lib().wotk_solver_workspace_size(n_i, n_j), 'cuda')
+    ws.fill_(255)
+    return ws
+
+
+def _gap(cost, g, ws, fn='wotk_transport_duality_gap', extra=(), **kw):
+    """One duality-gap solve through the C ABI: potentials and statistics."""
+    import ctypes
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, batch_size=5, tolerance=1e-8, tau=1e4, epsilon0=1.0,
+               max_iter=10 ** 7)
+    prm.update(kw)
+    n_i, n_j = cost.shape
+    G = torch.from_numpy(np.ascontiguousarray(g)).cuda()
+    f = torch.empty(n_i, dtype=torch.float64, device='cuda')
+    h = torch.empty(n_j, dtype=torch.float64, device='cuda')
+    st = _native.Stats()
+    p = dev._ptr
+    _native.check(getattr(_native.lib(), fn)(
+        p(cost.C), cost.ldc, p(cost.CT), cost.ldct, n_i, n_j, p(G), prm['lambda1'], prm['lambda2'], prm['epsilon'],
+        prm['batch_size'], prm['tolerance'], prm['tau'], prm['epsilon0'], prm['max_iter'], None, n_j, None, p(f), p(h),
+        p(ws), ws.numel(), ctypes.byref(st), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), *extra))
+    return f, h, st.as_dict()
+
+
+@pytest.mark.parametrize('n_i,n_j', SHAPES)
+def test_route_of_the_fixed_schedule(n_i, n_j):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    x, y, g = _pair(n_i, n_j)
+    cost = (ot.DeviceCost.from_coordinates(x, y) if n_i * n_j > 1
+            else ot.DeviceCost.from_matrix(np.array([[0.7]])))
+    ws = _workspace(n_i, n_j)
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, scaling_iter=23, extra_iter=4, inner_iter_max=5)
+    _run(_native.lib().wotk_transport_stablev2, cost, torch.from_numpy(g).cuda(), prm, ws)
+    assert _route(ws, n_i, n_j) == (_native.ROUTE_RESIDENT, 1)
+
+
+# rows on one side for some workgroups only (wide and tall), several rows per workgroup; the first duality
+# check decides; several launches
+@pytest.mark.parametrize('n_i,n_j,kw,launches', [
+    (120, 150, {}, 1), (300, 400, {}, 1), (400, 300, {}, 1), (300, 360, dict(tolerance=1e-2), 1),
+    (300, 360, dict(batch_size=1000), 1), (900, 8000, dict(tau=3.0), 1), (8000, 900, dict(tau=3.0), 1),
+    (2749, 3001, {}, 1), (60, 50, dict(tolerance=-1.0, max_iter=16384), 1),
+    (60, 50, dict(tolerance=-1.0, max_iter=32769), 3)])
+def test_route_of_the_duality_gap_schedule(n_i, n_j, kw, launches):
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    x, y, g = _pair(n_i, n_j, 1)
+    ws = _workspace(n_i, n_j)
+    _gap(ot.DeviceCost.from_coordinates(x, y), g, ws, **kw)
+    assert _route(ws, n_i, n_j) == (_native.ROUTE_RESIDENT, launches)
+
+
+def test_routes_beyond_the_resident_solver():
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    for n_i, n_j, want in [(2900, 2900, _native.ROUTE_ONE_READ), (40, 9000, _native.ROUTE_SWEEPS)]:
+        x, y, g = _pair(n_i, n_j)
+        ws = _workspace(n_i, n_j)
+        prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, scaling_iter=2, extra_iter=0,
+                   inner_iter_max=5)
+        _run(_native.lib().wotk_transport_stablev2, ot.DeviceCost.from_coordinates(x, y), torch.from_numpy(g).cuda(),
+             prm, ws)
+        assert _route(ws, n_i, n_j) == (want, 0)
+
+
+def test_route_from_threads_and_streams():
+    """Wide and tall pairs from two threads on two streams: both end as resident solves."""
+    import threading
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    shapes = [(300, 400), (1000, 260)]
+    costs = [ot.DeviceCost.from_coordinates(*_pair(i, j, 2)[:2]) for i, j in shapes]
+    torch.cuda.synchronize()
+    routes = [None, None]
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            ws = _workspace(*shapes[k])
+            for _ in range(3):
+                _gap(costs[k], _pair(*shapes[k], 2)[2], ws)
+            routes[k] = _route(ws, *shapes[k])
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in (0, 1)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert routes == [(_native.ROUTE_RESIDENT, 1)] * 2

@@ -26,6 +26,11 @@ KERNEL_BATCH_SHARED = 2
 BATCH_SHARE_EXP = 1
 BATCH_SHARE_EPS = 2
 
+ROUTE_SWEEPS = 0
+ROUTE_ONE_READ = 1
+ROUTE_RESIDENT = 2
+ROUTE_GAVE_UP = 3
+
 DTYPE_F64 = 0
 DTYPE_F32 = 1
 PUSH_FORWARD = 0
@@ -91,6 +96,7 @@ SIGNATURES = {
     'wotk_transport_duality_gap': (ctypes.c_int, [_P, _I64, _P, _I64, _I64, _I64, _P, _D, _D, _D, _I64,
                                                   _D, _D, _D, _I64, _P, _I64, _P, _P, _P, _P, _SZ,
                                                   ctypes.POINTER(Stats), _P]),
+    'wotk_solver_route': (ctypes.c_int, [_I64, _I64, _P, _SZ, ctypes.POINTER(_I32), ctypes.POINTER(_I64), _P]),
     'wotk_plan': (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _P, _D, _D, _P, _I64, _P, _P]),
     'wotk_batch_workspace_size': (_SZ, [_P, _I32, _I32, _I64]),
     'wotk_batch_stablev2': (ctypes.c_int, [_P, _P, _I32, _P, _I32, _P, _P, _D, _I64, _D, _D, _I64, _I64, _P, _P,

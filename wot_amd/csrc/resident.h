@@ -34,6 +34,7 @@ struct ResidentProblem {
 struct ResidentResult {
     int aborted;          // a wait ran out: nothing else is valid, solve again by launches
     int max_iter_reached;
+    long long launches;   // of this solve, all ended but the last when aborted
     long long iterations, stabilisations, checks;
     double gap, primal, dual, eps;
     // duality-gap schedule: the launch has done its iterations and the next one goes on from f, g, u,

@@ -82,6 +82,7 @@ struct Args {
     int n_wg;
     int rf, cf, rg, cg;  // rows per team and chunks per row: C rows, C^T rows
     double lambda1, lambda2, log_ni, log_nj;
+    long long launches;  // this one included
     GapParams gap;
 };
 
@@ -627,6 +628,7 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
     }
     if (so.row_f >= 0) a.rp.f[so.row_f] = sh.f[tid];
     if (so.row_g >= 0) a.rp.g[so.row_g] = sh.g[tid];
+    if (wg == 0 && tid == 0) a.res->launches = a.launches;
     if constexpr (GAP) {
         if (out.stopped) {
             if (so.row_f >= 0) a.rp.u[so.row_f] = sh.u[tid];
@@ -762,6 +764,7 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
     const int64_t total = scaling_iter + extra_iter;
     auto reg = [&](int64_t n) { return (epsilon0 - epsilon) * std::exp(-(double)n) + epsilon; };
     *launched = 0;
+    long long launches = 0;
     for (int64_t at = 0; at < total;) {
         Segments seg{};
         int64_t queued = 0;
@@ -778,6 +781,7 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
         int rc = clear(rp, s);
         if (rc) return rc;
         Args a = make_args(rp, sh, lambda1, lambda2);
+        a.launches = ++launches;
         rc = dispatch<false>(a, seg, sh.slots, launched, s);
         if (rc || !*launched) return rc;
         if (at < total) {  // the next launch clears the flag: look before
@@ -800,6 +804,7 @@ int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, doub
         int rc = clear(rp, s);
         if (rc) return rc;
         Args a = make_args(rp, sh, lambda1, lambda2);
+        a.launches = out->launches + 1;
         a.gap = GapParams{factor, tolerance, tau, batch_size, max_iter, kLaunchIters, *out};
         Segments seg{};
         rc = dispatch<true>(a, seg, sh.slots, launched, s);

@@ -1041,6 +1041,29 @@ static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambd
     return WOTK_OK;
 }
 
+extern "C" int wotk_solver_route(int64_t I, int64_t J, const void *workspace, size_t workspace_bytes, int32_t *route,
+                                 int64_t *launches, void *stream) {
+    WOTK_REQUIRE(I > 0 && J > 0 && I < (1ll << 31) && J < (1ll << 31), "bad shape %lld x %lld", (long long)I,
+                 (long long)J);
+    WOTK_REQUIRE(route && launches, "route and launches are required");
+    Arena ar(const_cast<void *>(workspace), workspace_bytes);
+    Work w;
+    carve(ar, I, J, true, &w);
+    if (!workspace || !ar.ok) return fail(WOTK_EWORKSPACE, "solver workspace too small");
+    *launches = 0;
+    *route = w.col_part ? WOTK_ROUTE_ONE_READ : WOTK_ROUTE_SWEEPS;
+    if (!w.exchange) return WOTK_OK;
+    ResidentProblem rp{};
+    rp.exchange = w.exchange;
+    ResidentResult r;
+    const int rc = resident_result(rp, &r, (hipStream_t)stream);
+    if (rc) return rc;
+    *launches = r.launches;
+    if (r.aborted) *route = WOTK_ROUTE_GAVE_UP;
+    else if (r.launches) *route = WOTK_ROUTE_RESIDENT;
+    return WOTK_OK;
+}
+
 extern "C" int wotk_transport_stablev2(const float *C, int64_t ldc, const float *CT, int64_t ldct,
                                        int64_t I, int64_t J, const double *G, double lambda1,
                                        double lambda2, double epsilon, int64_t scaling_iter,
