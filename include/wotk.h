@@ -495,6 +495,35 @@ int wotk_probe_valu_rates(double *rates_host, int32_t n_rates, void *sink, size_
  * 2, 4 and 8 waves per SIMD: rates_host (HOST, >= 4 entries).  Same sink. */
 int wotk_probe_issue_mix(double *rates_host, int32_t n_rates, void *sink, size_t sink_bytes, void *stream);
 
+/* ---------------------------------------------------------------------------
+ * The solves above with the bounds of their waits and launches set by the
+ * caller (no counterpart in the reference), to run what follows when a bound
+ * is met.  give_up = 1: a workgroup of the resident solver gives up at its
+ * first look at a value that is not there yet, and the solve is repeated by
+ * launched sweeps (wotk_solver_route: WOTK_ROUTE_GAVE_UP).  launch_iters > 0:
+ * iterations per persistent launch.  polls: looks at the sums handed over
+ * between two workgroups of a never-stored sweep before the second one
+ * computes them itself.  Results are those of the unlimited calls, bit for bit.
+ * ------------------------------------------------------------------------- */
+int wotk_probe_stablev2_limits(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
+                               const double *G, double lambda1, double lambda2, double epsilon,
+                               int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
+                               int64_t inner_iter_max, double *plan, int64_t ldp, double *row_sums, double *f_out,
+                               double *g_out, void *workspace, size_t workspace_bytes, wotk_stats *stats,
+                               void *stream, int32_t give_up, int64_t launch_iters);
+int wotk_probe_duality_gap_limits(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
+                                  const double *G, double lambda1, double lambda2, double epsilon,
+                                  int64_t batch_size, double tolerance, double tau, double epsilon0,
+                                  int64_t max_iter, double *plan, int64_t ldp, double *row_sums, double *f_out,
+                                  double *g_out, void *workspace, size_t workspace_bytes, wotk_stats *stats,
+                                  void *stream, int32_t give_up, int64_t launch_iters);
+int wotk_probe_stablev2_coords_limits(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
+                                      const double *G, double lambda1, double lambda2, double epsilon,
+                                      int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
+                                      int64_t inner_iter_max, int32_t terms, double *f_out, double *g_out,
+                                      double *row_sums, double *median_out, void *workspace,
+                                      size_t workspace_bytes, wotk_stats *stats, void *stream, int32_t polls);
+
 #ifdef __cplusplus
 }
 #endif

@@ -79,3 +79,29 @@ def test_gap_schedule_absorptions_match_oracle(n_i, n_j, tau):
     assert abs(st['stabilisations'] - so['stabilisations']) <= abs(st['iterations'] - so['iterations'])
     R = res.dense().cpu().numpy()
     assert np.linalg.norm(R - Ro) / np.linalg.norm(Ro) <= 1e-5
+
+
+# cut units whose sums do not come in time: rows with one and with several splits, both term counts
+@pytest.mark.parametrize('n_i,n_j,d,terms', [(8300, 8450, 20, 6), (8300, 8450, 17, 3), (16500, 900, 70, 6)])
+def test_sums_that_do_not_come_are_computed_again(n_i, n_j, d, terms):
+    import ctypes
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    gen = torch.Generator(device='cuda').manual_seed(n_i + d)
+    x = torch.randn(n_i, d, dtype=torch.float64, device='cuda', generator=gen)
+    y = torch.randn(n_j, d, dtype=torch.float64, device='cuda', generator=gen) + 0.2
+    G = torch.exp(0.3 * torch.randn(n_i, dtype=torch.float64, device='cuda', generator=gen))
+    L, p = _native.lib(), dev._ptr
+    ws = dev.workspace(torch, L.wotk_fused_workspace_size(n_i, n_j, d), 'cuda')
+
+    def solve(fn, *extra):
+        out = [torch.empty(n, dtype=torch.float64, device='cuda') for n in (n_i, n_j, n_i, 1)]
+        st = _native.Stats()
+        _native.check(fn(p(x), p(y), n_i, n_j, d, p(G), 1.0, 50.0, 0.5, 3, 1e4, 0.5, 0, 50, terms,
+                         *(p(t) for t in out), p(ws), ws.numel(), ctypes.byref(st),
+                         ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), *extra))
+        return out
+
+    for a, b in zip(solve(L.wotk_transport_stablev2_coords), solve(L.wotk_probe_stablev2_coords_limits, 0)):
+        assert torch.equal(a, b)

@@ -282,3 +282,66 @@ def test_route_from_threads_and_streams():
     for t in ts:
         t.join()
     assert routes == [(_native.ROUTE_RESIDENT, 1)] * 2
+
+
+# ---- what follows when a bound is met: the same bits by another route ----
+def _fixed(fn, cost, g, ws, extra=()):
+    import ctypes
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    n_i, n_j = cost.shape
+    G = torch.from_numpy(np.ascontiguousarray(g)).cuda()
+    f = torch.empty(n_i, dtype=torch.float64, device='cuda')
+    h = torch.empty(n_j, dtype=torch.float64, device='cuda')
+    st = _native.Stats()
+    p = dev._ptr
+    _native.check(getattr(_native.lib(), fn)(
+        p(cost.C), cost.ldc, p(cost.CT), cost.ldct, n_i, n_j, p(G), 1.0, 50.0, 0.05, 43, 1e4, 1.0, 4, 11, None, n_j,
+        None, p(f), p(h), p(ws), ws.numel(), ctypes.byref(st),
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), *extra))
+    return f, h, st.as_dict()
+
+
+# pairs of several workgroups, with rows on one side only for some of them
+@pytest.mark.parametrize('n_i,n_j', [(30, 20), (300, 400), (1000, 260), (2049, 2047)])
+def test_a_wait_that_is_given_up(n_i, n_j):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    x, y, g = _pair(n_i, n_j, 4)
+    cost = ot.DeviceCost.from_coordinates(x, y)
+    ws = _workspace(n_i, n_j)
+    a = _fixed('wotk_transport_stablev2', cost, g, ws)
+    assert _route(ws, n_i, n_j)[0] == _native.ROUTE_RESIDENT
+    b = _fixed('wotk_probe_stablev2_limits', cost, g, ws, (1, 0))
+    assert _route(ws, n_i, n_j)[0] == _native.ROUTE_GAVE_UP
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    a = _gap(cost, g, ws, tau=3.0)
+    assert _route(ws, n_i, n_j)[0] == _native.ROUTE_RESIDENT
+    b = _gap(cost, g, ws, 'wotk_probe_duality_gap_limits', (1, 0), tau=3.0)
+    assert _route(ws, n_i, n_j)[0] == _native.ROUTE_GAVE_UP
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    for key in ('iterations', 'stabilisations', 'gap_checks', 'epsilon_final'):
+        assert a[2][key] == b[2][key]
+
+
+# one iteration per launch, cuts inside and at the ends of batches
+@pytest.mark.parametrize('n_i,n_j', [(30, 20), (300, 400), (1000, 260)])
+@pytest.mark.parametrize('launch_iters', [1, 5, 7])
+def test_launches_that_stop(n_i, n_j, launch_iters):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    x, y, g = _pair(n_i, n_j, 4)
+    cost = ot.DeviceCost.from_coordinates(x, y)
+    ws = _workspace(n_i, n_j)
+    a = _fixed('wotk_transport_stablev2', cost, g, ws)
+    b = _fixed('wotk_probe_stablev2_limits', cost, g, ws, (0, launch_iters))
+    assert _route(ws, n_i, n_j) == (_native.ROUTE_RESIDENT, -(-47 // launch_iters))
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    for kw in (dict(tau=3.0), dict(tau=3.0, batch_size=3, max_iter=311)):
+        a = _gap(cost, g, ws, **kw)
+        b = _gap(cost, g, ws, 'wotk_probe_duality_gap_limits', (0, launch_iters), **kw)
+        assert _route(ws, n_i, n_j) == (_native.ROUTE_RESIDENT, -(-a[2]['iterations'] // launch_iters))
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and a[2] == b[2]

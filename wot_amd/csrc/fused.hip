@@ -104,6 +104,7 @@ struct FusedArgs {
     int whole;                   // one unit per workgroup; else an equal run of tiles each
     unsigned long long *box;     // [workgroup][word][thread]: partial sums handed to the next workgroup
     unsigned tag;                // this launch's mark on them
+    int polls;                   // looks at them
     TauTrack tau;                // growth of the potentials (prev null: not tracked)
     double *base;                // what they grow from: u or v
     int opens;                   // the iteration's first sweep
@@ -129,10 +130,9 @@ __device__ __forceinline__ FusedUnit fused_unit(const FusedArgs &fa, int64_t pos
 
 // Partial sums passed between workgroups: 32 bits of value and the launch's mark
 // in one 8-byte word, so a word is either whole or not yet there and no fence is
-// needed.  The wait is bounded: after kFusedPolls looks (about 0.2 ms) the caller
-// computes the missing part itself, so progress never depends on which workgroups
-// the chip holds at once.
-constexpr int kFusedPolls = 128;
+// needed.  The wait is bounded: after so many looks (FusedProblem::polls, 128: about
+// 0.2 ms) the caller computes the missing part itself, so progress never depends on
+// which workgroups the chip holds at once.
 __device__ __forceinline__ unsigned long long fused_word(unsigned v, unsigned tag) {
     return (unsigned long long)tag << 32 | v;
 }
@@ -154,9 +154,9 @@ __device__ __forceinline__ void fused_send(unsigned long long *box, unsigned tag
     }
 }
 template <typename T>
-__device__ __forceinline__ bool fused_take(unsigned long long *box, unsigned tag, T (&s)[16]) {
+__device__ __forceinline__ bool fused_take(unsigned long long *box, unsigned tag, int polls, T (&s)[16]) {
     constexpr int W = sizeof(T) / 4;
-    for (int q = 0; q < kFusedPolls; ++q) {
+    for (int q = 0; q < polls; ++q) {
         bool there = true;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kFThreads, fused_waves(TERMS, NKS)) void fused_lse_
         if (begin > un.first) {
             int64_t at = (int64_t)blockIdx.x * kWords + tid;
             asm volatile("" : "+v"(at));  // the words' 16 addresses are not kept in registers over the tiles
-            taken = fused_take(fa.box + at, fa.tag, s);
+            taken = fused_take(fa.box + at, fa.tag, fa.polls, s);
             if (!taken) ta = un.t0;
         }
         if (!taken) {
@@ -710,7 +710,7 @@ static FusedArgs problem_args(const FusedProblem &fp, bool target_rows, const do
     return FusedArgs{target_rows ? fp.yp : fp.xp, target_rows ? fp.xp : fp.yp, target_rows ? fp.ny : fp.nx,
                      target_rows ? fp.nx : fp.ny, nr, nc, fp.kp, h, pot, logw, logw_dev, std::log((double)nc), alpha,
                      eps, kLog2E / eps, row_sums, second_set ? fp.part2 : fp.part, rs_div, 0, 0, 0, 0, 0,
-                     second_set ? fp.box2 : fp.box, ++fp.tag, TauTrack{}, nullptr, 0, nullptr};
+                     second_set ? fp.box2 : fp.box, ++fp.tag, fp.polls, TauTrack{}, nullptr, 0, nullptr};
 }
 
 template <bool EXACT>
@@ -770,18 +770,17 @@ extern "C" size_t wotk_fused_workspace_size(int64_t I, int64_t J, int64_t d) {
     return fused_problem_bytes(I, J, d) + 256 + fz_state_carve(ar, I, J, &st);
 }
 
-extern "C" int wotk_transport_stablev2_coords(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
-                                              const double *G, double lambda1, double lambda2, double epsilon,
-                                              int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
-                                              int64_t inner_iter_max, int32_t terms, double *f_out, double *g_out,
-                                              double *row_sums, double *median_out, void *workspace,
-                                              size_t workspace_bytes, wotk_stats *stats, void *stream) {
-    hipStream_t s = (hipStream_t)stream;
+static int stablev2_coords_call(const double *X, const double *Y, int64_t I, int64_t J, int64_t d, const double *G,
+                                double lambda1, double lambda2, double epsilon, int64_t scaling_iter,
+                                double epsilon0, int64_t extra_iter, int64_t inner_iter_max, int32_t terms,
+                                double *f_out, double *g_out, double *row_sums, double *median_out,
+                                void *workspace, size_t workspace_bytes, int32_t polls, wotk_stats *stats,
+                                hipStream_t s) {
     WOTK_REQUIRE(scaling_iter >= 0 && extra_iter >= 0 && scaling_iter + extra_iter > 0 && inner_iter_max > 0,
                  "bad iteration counts");
     WOTK_REQUIRE(G != nullptr, "G is required");
-    (void)tau;
     FusedProblem fp;
+    if (polls >= 0) fp.polls = polls;
     size_t used = 0;
     int rc = fused_problem_setup(X, Y, I, J, d, terms, workspace, workspace_bytes, &fp, &used, s);
     if (rc) return rc;
@@ -834,4 +833,29 @@ extern "C" int wotk_transport_stablev2_coords(const double *X, const double *Y, 
         stats->epsilon_final = e_end;
     }
     return WOTK_OK;
+}
+
+extern "C" int wotk_transport_stablev2_coords(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
+                                              const double *G, double lambda1, double lambda2, double epsilon,
+                                              int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
+                                              int64_t inner_iter_max, int32_t terms, double *f_out, double *g_out,
+                                              double *row_sums, double *median_out, void *workspace,
+                                              size_t workspace_bytes, wotk_stats *stats, void *stream) {
+    (void)tau;
+    return stablev2_coords_call(X, Y, I, J, d, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
+                                inner_iter_max, terms, f_out, g_out, row_sums, median_out, workspace,
+                                workspace_bytes, -1, stats, (hipStream_t)stream);
+}
+
+extern "C" int wotk_probe_stablev2_coords_limits(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
+                                                 const double *G, double lambda1, double lambda2, double epsilon,
+                                                 int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
+                                                 int64_t inner_iter_max, int32_t terms, double *f_out, double *g_out,
+                                                 double *row_sums, double *median_out, void *workspace,
+                                                 size_t workspace_bytes, wotk_stats *stats, void *stream,
+                                                 int32_t polls) {
+    (void)tau;
+    return stablev2_coords_call(X, Y, I, J, d, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
+                                inner_iter_max, terms, f_out, g_out, row_sums, median_out, workspace,
+                                workspace_bytes, polls, stats, (hipStream_t)stream);
 }

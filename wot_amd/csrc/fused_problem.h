@@ -23,6 +23,7 @@ struct FusedProblem {
     double *part = nullptr, *part2 = nullptr;
     unsigned long long *box = nullptr, *box2 = nullptr;  // sums handed between workgroups
     int box_words = 0;
+    int polls = 128;                                     // looks at them before a part is computed again
     mutable unsigned tag = 0;                            // the last launch's mark on them
     void *median_ws = nullptr;
     const double *median = nullptr;  // device: the exact median of the FP64 distances

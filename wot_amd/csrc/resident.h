@@ -10,6 +10,14 @@
 
 namespace wotk {
 
+// how long a workgroup waits for a value and how much one launch does
+struct ResidentLimits {
+    long long wait_ticks = 20ll * 100000000ll;  // 20 s of the 100 MHz clock, looked at ...
+    unsigned look_mask = 255;                   // ... every 256 polls
+    // 0.08 to 0.25 s, so that no launch holds the chip for long however many iterations a schedule takes
+    long long launch_iters = 16384;
+};
+
 // whether pairs of this shape take the resident solver
 bool resident_fits(int64_t I, int64_t J);
 
@@ -47,13 +55,14 @@ struct ResidentResult {
 // The fixed-iteration schedule (optimal_transport.py:167-236).  *launched is 0 when the
 // device cannot hold all workgroups at once: nothing ran.
 int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, double epsilon0,
-                   int64_t scaling_iter, int64_t inner_iter_max, int64_t extra_iter, int *launched, hipStream_t s);
+                   int64_t scaling_iter, int64_t inner_iter_max, int64_t extra_iter, const ResidentLimits &lim,
+                   int *launched, hipStream_t s);
 
 // the duality-gap schedule (optimal_transport.py:67-164) up to its last iteration; *out is its
 // outcome when *launched (waits for it)
 int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, long long batch_size,
-                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched,
-                 ResidentResult *out, hipStream_t s);
+                 double tolerance, double tau, double epsilon0, long long max_iter, const ResidentLimits &lim,
+                 int *launched, ResidentResult *out, hipStream_t s);
 
 // the result of the last resident launch on rp (waits for it)
 int resident_result(const ResidentProblem &rp, ResidentResult *out, hipStream_t s);

@@ -30,7 +30,7 @@
 // tests/test_resident_exchange.py holds a model of this that delays workgroups at will.
 //
 // Progress.  The launch is cooperative: all workgroups are resident or none runs, and
-// two such launches do not share the device.  Every wait is bounded (kWaitSeconds): a
+// two such launches do not share the device.  Every wait is bounded (ResidentLimits): a
 // workgroup that gives up raises a flag that ends all others' waits, and the caller solves
 // again by launches.
 #include <algorithm>
@@ -53,12 +53,8 @@ constexpr int kMaxSide = 8704;           // potentials of one side in LDS (two s
 constexpr int kMaxLds = 2 * 8 * 1024 * ((kMaxSide + 1023) / 1024);  // bytes of both sides' potentials
 constexpr int kSums = 8;                 // values a workgroup contributes to a check
 constexpr int kSegments = 96;            // eps segments per launch
-// iterations per launch: 0.08 to 0.25 s, so that no launch holds the chip for long however many
-// iterations a schedule takes
-constexpr int64_t kLaunchIters = 16384;
 constexpr u64 kEmpty = 0x7ffddeadc0ffee01ull;
 constexpr u64 kPlainNan = 0x7ff8000000000000ull;
-constexpr long long kWaitTicks = 20ll * 100000000ll;  // 20 s of the 100 MHz clock
 constexpr double kSigInit = -1.0e6;      // "no term yet", as in the sweep
 
 struct Segments {
@@ -69,7 +65,7 @@ struct Segments {
 
 struct GapParams {
     double factor, tolerance, tau;
-    long long batch, max_iter, launch_iters;
+    long long batch, max_iter;
     ResidentResult from;  // the state at the launch: all zero but eps, or where the last launch stopped
 };
 
@@ -83,6 +79,7 @@ struct Args {
     int rf, cf, rg, cg;  // rows per team and chunks per row: C rows, C^T rows
     double lambda1, lambda2, log_ni, log_nj;
     long long launches;  // this one included
+    ResidentLimits lim;
     GapParams gap;
 };
 
@@ -199,9 +196,9 @@ struct Solver {
         for (int n = 1; x == kEmpty; ++n) {
             __builtin_amdgcn_s_sleep(1);
             x = load_x(p);
-            if ((n & 255) == 0 && x == kEmpty) {
+            if ((n & a.lim.look_mask) == 0 && x == kEmpty) {
                 if (__hip_atomic_load(&a.res->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
-                    wall_clock64() - start > kWaitTicks) {
+                    wall_clock64() - start > a.lim.wait_ticks) {
                     __hip_atomic_store(&a.res->aborted, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     sh.aborted[phase] = 1;
                     return false;
@@ -531,7 +528,7 @@ struct Solver {
         out = gp_.from;
         out.stopped = 0;
         bool resumed = gp_.from.stopped, first = true;
-        const long long stop_at = out.iterations + gp_.launch_iters;
+        const long long stop_at = out.iterations + a.lim.launch_iters;
         long long t = out.in_batch;
         for (int e = out.scaling; e <= n_scal; ++e) {
             if (!resumed) {
@@ -716,7 +713,8 @@ int dispatch(Args &a, Segments &seg, int slots, int *launched, hipStream_t s) {
     return launch<kMaxSlots, GAP>(a, seg, launched, s);
 }
 
-Args make_args(const ResidentProblem &rp, const Shape &sh, double lambda1, double lambda2) {
+Args make_args(const ResidentProblem &rp, const Shape &sh, double lambda1, double lambda2,
+               const ResidentLimits &lim) {
     const Exchange e = carve(rp.exchange, rp.n_i, rp.n_j);
     Args a{};
     a.rp = rp;
@@ -734,6 +732,7 @@ Args make_args(const ResidentProblem &rp, const Shape &sh, double lambda1, doubl
     a.lambda2 = lambda2;
     a.log_ni = std::log((double)rp.n_i);
     a.log_nj = std::log((double)rp.n_j);
+    a.lim = lim;
     return a;
 }
 
@@ -759,7 +758,8 @@ bool resident_fits(int64_t I, int64_t J) {
 size_t resident_bytes(int64_t I, int64_t J) { return 256 + sizeof(u64) * (size_t)carve(nullptr, I, J).n; }
 
 int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, double epsilon0,
-                   int64_t scaling_iter, int64_t inner_iter_max, int64_t extra_iter, int *launched, hipStream_t s) {
+                   int64_t scaling_iter, int64_t inner_iter_max, int64_t extra_iter, const ResidentLimits &lim,
+                   int *launched, hipStream_t s) {
     const Shape sh = shape_of(rp.n_i, rp.n_j);
     const int64_t total = scaling_iter + extra_iter;
     auto reg = [&](int64_t n) { return (epsilon0 - epsilon) * std::exp(-(double)n) + epsilon; };
@@ -768,11 +768,11 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
     for (int64_t at = 0; at < total;) {
         Segments seg{};
         int64_t queued = 0;
-        while (at < total && seg.count < kSegments && queued < kLaunchIters) {
+        while (at < total && seg.count < kSegments && queued < lim.launch_iters) {
             // up to the next change of eps
             const int64_t block = at < scaling_iter ? at / inner_iter_max : scaling_iter / inner_iter_max;
             const int64_t end = at < scaling_iter ? std::min(scaling_iter, (block + 1) * inner_iter_max) : total;
-            const int64_t n = std::min(end - at, kLaunchIters - queued);
+            const int64_t n = std::min<int64_t>(end - at, lim.launch_iters - queued);
             seg.eps[seg.count] = reg(block);
             seg.iters[seg.count++] = n;
             queued += n;
@@ -780,7 +780,7 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
         }
         int rc = clear(rp, s);
         if (rc) return rc;
-        Args a = make_args(rp, sh, lambda1, lambda2);
+        Args a = make_args(rp, sh, lambda1, lambda2, lim);
         a.launches = ++launches;
         rc = dispatch<false>(a, seg, sh.slots, launched, s);
         if (rc || !*launched) return rc;
@@ -794,8 +794,8 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
 }
 
 int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, long long batch_size,
-                 double tolerance, double tau, double epsilon0, long long max_iter, int *launched,
-                 ResidentResult *out, hipStream_t s) {
+                 double tolerance, double tau, double epsilon0, long long max_iter, const ResidentLimits &lim,
+                 int *launched, ResidentResult *out, hipStream_t s) {
     const Shape sh = shape_of(rp.n_i, rp.n_j);
     const double factor = std::exp(-std::log(epsilon) / 5);
     *out = ResidentResult{};
@@ -803,9 +803,9 @@ int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, doub
     do {
         int rc = clear(rp, s);
         if (rc) return rc;
-        Args a = make_args(rp, sh, lambda1, lambda2);
+        Args a = make_args(rp, sh, lambda1, lambda2, lim);
         a.launches = out->launches + 1;
-        a.gap = GapParams{factor, tolerance, tau, batch_size, max_iter, kLaunchIters, *out};
+        a.gap = GapParams{factor, tolerance, tau, batch_size, max_iter, *out};
         Segments seg{};
         rc = dispatch<true>(a, seg, sh.slots, launched, s);
         if (rc || !*launched) return rc;

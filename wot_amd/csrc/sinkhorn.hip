@@ -983,7 +983,7 @@ static ResidentProblem resident_problem(const Problem &pb, const Work &w) {
 static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambda2, double epsilon,
                         int64_t scaling_iter, double epsilon0, int64_t extra_iter, int64_t inner_iter_max,
                         double *plan, int64_t ldp, double *row_sums, double *f_out, double *g_out, bool timed,
-                        wotk_stats *stats, hipStream_t s) {
+                        const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
     WOTK_REQUIRE(scaling_iter >= 0 && extra_iter >= 0 && scaling_iter + extra_iter > 0,
                  "at least one scaling iteration is required");
     WOTK_REQUIRE(inner_iter_max > 0, "inner_iter_max must be positive");
@@ -1004,7 +1004,7 @@ static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambd
         const ResidentProblem rp = resident_problem(pb, w);
         int launched = 0;
         rc = resident_fixed(rp, lambda1, lambda2, epsilon, epsilon0, scaling_iter, inner_iter_max, extra_iter,
-                            &launched, s);
+                            lim, &launched, s);
         if (rc) return rc;
         if (launched) {
             ResidentResult r;
@@ -1064,6 +1064,19 @@ extern "C" int wotk_solver_route(int64_t I, int64_t J, const void *workspace, si
     return WOTK_OK;
 }
 
+static int stablev2_call(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
+                         const double *G, double lambda1, double lambda2, double epsilon, int64_t scaling_iter,
+                         double epsilon0, int64_t extra_iter, int64_t inner_iter_max, double *plan, int64_t ldp,
+                         double *row_sums, double *f_out, double *g_out, void *workspace, size_t workspace_bytes,
+                         const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
+    Problem pb;
+    Work w;
+    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    if (rc) return rc;
+    return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
+                        ldp, row_sums, f_out, g_out, true, lim, stats, s);
+}
+
 extern "C" int wotk_transport_stablev2(const float *C, int64_t ldc, const float *CT, int64_t ldct,
                                        int64_t I, int64_t J, const double *G, double lambda1,
                                        double lambda2, double epsilon, int64_t scaling_iter,
@@ -1072,14 +1085,36 @@ extern "C" int wotk_transport_stablev2(const float *C, int64_t ldc, const float 
                                        double *row_sums, double *f_out, double *g_out,
                                        void *workspace, size_t workspace_bytes, wotk_stats *stats,
                                        void *stream) {
-    hipStream_t s = (hipStream_t)stream;
-    Problem pb;
-    Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
-    if (rc) return rc;
     (void)tau;  // absorption is exact in the log domain; tau only changes the FP64 reference's rounding
-    return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
-                        ldp, row_sums, f_out, g_out, true, stats, s);
+    return stablev2_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
+                         inner_iter_max, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
+                         ResidentLimits{}, stats, (hipStream_t)stream);
+}
+
+// limits of a probe: waits that end at their first look, launches of so many iterations (0: as ever)
+static ResidentLimits probe_limits(int32_t give_up, int64_t launch_iters) {
+    ResidentLimits lim;
+    if (give_up) {
+        lim.wait_ticks = -1;
+        lim.look_mask = 0;
+    }
+    if (launch_iters > 0) lim.launch_iters = launch_iters;
+    return lim;
+}
+
+extern "C" int wotk_probe_stablev2_limits(const float *C, int64_t ldc, const float *CT, int64_t ldct,
+                                          int64_t I, int64_t J, const double *G, double lambda1,
+                                          double lambda2, double epsilon, int64_t scaling_iter,
+                                          double tau, double epsilon0, int64_t extra_iter,
+                                          int64_t inner_iter_max, double *plan, int64_t ldp,
+                                          double *row_sums, double *f_out, double *g_out,
+                                          void *workspace, size_t workspace_bytes, wotk_stats *stats,
+                                          void *stream,
+                                          int32_t give_up, int64_t launch_iters) {
+    (void)tau;
+    return stablev2_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
+                         inner_iter_max, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
+                         probe_limits(give_up, launch_iters), stats, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1139,7 +1174,7 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
     if (rc) return rc;
     (void)tau;
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
-                        ldp, row_sums, f_out, g_out, false, stats, s);
+                        ldp, row_sums, f_out, g_out, false, ResidentLimits{}, stats, s);
 }
 
 // second stream and event of the duality-gap solver's last scaling; drained
@@ -1378,15 +1413,11 @@ struct StoredBackend {
     }
 };
 
-extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const float *CT,
-                                          int64_t ldct, int64_t I, int64_t J, const double *G,
-                                          double lambda1, double lambda2, double epsilon,
-                                          int64_t batch_size, double tolerance, double tau,
-                                          double epsilon0, int64_t max_iter, double *plan,
-                                          int64_t ldp, double *row_sums, double *f_out,
-                                          double *g_out, void *workspace, size_t workspace_bytes,
-                                          wotk_stats *stats, void *stream) {
-    hipStream_t s = (hipStream_t)stream;
+static int duality_gap_call(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
+                            const double *G, double lambda1, double lambda2, double epsilon, int64_t batch_size,
+                            double tolerance, double tau, double epsilon0, int64_t max_iter, double *plan,
+                            int64_t ldp, double *row_sums, double *f_out, double *g_out, void *workspace,
+                            size_t workspace_bytes, const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
     Problem pb;
     Work w;
     int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
@@ -1398,8 +1429,8 @@ extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const flo
         const ResidentProblem rp = resident_problem(pb, w);
         int launched = 0;
         ResidentResult r;
-        rc = resident_gap(rp, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, &launched,
-                          &r, s);
+        rc = resident_gap(rp, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, lim,
+                          &launched, &r, s);
         if (rc) return rc;
         if (launched && !r.aborted) {
             if (stats) {
@@ -1428,6 +1459,33 @@ extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const flo
     }
     return gap_schedule(be, pb, w, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0, max_iter, stats,
                         s);
+}
+
+extern "C" int wotk_transport_duality_gap(const float *C, int64_t ldc, const float *CT,
+                                          int64_t ldct, int64_t I, int64_t J, const double *G,
+                                          double lambda1, double lambda2, double epsilon,
+                                          int64_t batch_size, double tolerance, double tau,
+                                          double epsilon0, int64_t max_iter, double *plan,
+                                          int64_t ldp, double *row_sums, double *f_out,
+                                          double *g_out, void *workspace, size_t workspace_bytes,
+                                          wotk_stats *stats, void *stream) {
+    return duality_gap_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0,
+                            max_iter, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes, ResidentLimits{},
+                            stats, (hipStream_t)stream);
+}
+
+extern "C" int wotk_probe_duality_gap_limits(const float *C, int64_t ldc, const float *CT,
+                                             int64_t ldct, int64_t I, int64_t J, const double *G,
+                                             double lambda1, double lambda2, double epsilon,
+                                             int64_t batch_size, double tolerance, double tau,
+                                             double epsilon0, int64_t max_iter, double *plan,
+                                             int64_t ldp, double *row_sums, double *f_out,
+                                             double *g_out, void *workspace, size_t workspace_bytes,
+                                             wotk_stats *stats, void *stream,
+                                             int32_t give_up, int64_t launch_iters) {
+    return duality_gap_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, batch_size, tolerance, tau, epsilon0,
+                            max_iter, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
+                            probe_limits(give_up, launch_iters), stats, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
