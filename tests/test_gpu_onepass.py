@@ -125,3 +125,50 @@ def test_duality_gap_schedule_matches_fp64(n_i, n_j, kw):
     if 'stabilisations' in so:
         assert st['stabilisations'] == so['stabilisations']
     assert float((R - ref).norm() / ref.norm()) < 1e-6
+
+
+def _both_of_matrix(C, G, **kw):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, scaling_iter=150, extra_iter=20,
+               inner_iter_max=50)
+    prm.update(kw)
+    cost = ot.DeviceCost.from_matrix(C)
+    Gd = torch.from_numpy(np.ascontiguousarray(G)).cuda()
+    L = _native.lib()
+    ws = dev.workspace(torch, L.wotk_solver_workspace_size(*cost.shape), 'cuda')
+    return (_run(L.wotk_transport_stablev2, cost, Gd, prm, ws),
+            _run(L.wotk_transport_stablev2_noalloc, cost, Gd, prm))
+
+
+# forbidden pairs (infinite) and costs beyond 2^31 / k, in the first, a middle and the last row and column and
+# strewn; every width of the columns' chunks; some in the first eps already
+@pytest.mark.parametrize('n_i,n_j', [(2201, 3839), (2100, 4101), (1021, 8221), (701, 12289), (517, 16389)])
+@pytest.mark.parametrize('big', [np.inf, 1e9, 3e38])
+def test_forbidden_pairs_are_terms_of_zero(n_i, n_j, big):
+    import torch
+    rng = np.random.default_rng(n_j)
+    C = rng.gamma(6.0, 1 / 6.0, (n_i, n_j))
+    C[rng.random((n_i, n_j)) < 0.01] = big
+    for r in (0, n_i // 2, n_i - 1):
+        C[r, :: 2] = big
+    for c in (0, n_j // 2, n_j - 1):
+        C[1:: 2, c] = big
+    one, two = _both_of_matrix(C, np.exp(0.3 * rng.standard_normal(n_i)))
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.isfinite(b).all()
+        # exponents of a few times max C / eps = 100 rounded at 2^-24 by the sweeps, averaged over the terms,
+        # times eps, over 340 half-iterations that do not expand: 340 * 0.05 * 100 * 2^-24 * ln 2
+        assert float((a - b).abs().max()) < 7e-5
+
+
+def test_nan_costs_stay_nan():
+    import torch
+    rng = np.random.default_rng(3)
+    C = rng.gamma(6.0, 1 / 6.0, (2100, 4100))
+    C[77, 1234] = np.nan
+    one, two = _both_of_matrix(C, np.ones(2100), scaling_iter=0, extra_iter=1)
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))

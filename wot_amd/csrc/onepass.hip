@@ -196,9 +196,17 @@ struct RowPass {
                 for (int q = 0; q < 4; ++q) {
                     const double y = fma(-ra.k, (double)cur.v[r][c][q], hk[q]);
                     const double n = rint(y);
-                    e[q] = ldexpf(__builtin_amdgcn_exp2f((float)(y - n)), (int)n - N[r]);
+                    // saturating: a cost far above 2^31 / k is a term of 0, not a wrapped exponent
+                    e[q] = ldexpf(__builtin_amdgcn_exp2f((float)(y - n)), __builtin_elementwise_sub_sat((int)n, N[r]));
                 }
-                s[r] += (double)((e[0] + e[1]) + (e[2] + e[3]));
+                float t = (e[0] + e[1]) + (e[2] + e[3]);
+                if (__builtin_expect(t != t, 0)) {  // an infinite cost (y - n is no number) is a term of 0
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (fma(-ra.k, (double)cur.v[r][c][q], hk[q]) == -INFINITY) e[q] = 0.f;
+                    t = (e[0] + e[1]) + (e[2] + e[3]);
+                }
+                s[r] += (double)t;
                 cur.v[r][c] = e;
             }
             // keep the next chunk's shifts and exponents out of this one's registers
