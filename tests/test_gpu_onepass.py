@@ -172,3 +172,40 @@ def test_nan_costs_stay_nan():
     one, two = _both_of_matrix(C, np.ones(2100), scaling_iter=0, extra_iter=1)
     for a, b in zip(one[:2], two[:2]):
         assert torch.equal(torch.isnan(a), torch.isnan(b))
+
+
+@pytest.mark.parametrize('eps,lam1', [(0.05, 1.0), (0.003, 5.0), (0.003, 50.0)])
+def test_rows_whose_terms_overflow(eps, lam1):
+    """Zero growth: such a row has no shift, and its terms pass 2^128 where it lies on a target that only far
+    cells serve."""
+    import torch
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(2100, 4100, dim=30, n_components=5, seed=2100)
+    x, y, G = dp.x.copy(), dp.y.copy(), dp.growth.copy()
+    zero = [0, 17, 900, 2099]
+    y[[3, 1024, 2047, 4099]] *= 4.0
+    x[zero] = y[[3, 1024, 2047, 4099]]
+    G[zero] = 0.0
+    cost, one, two = _both(x, y, G, epsilon=eps, epsilon0=1.0, lambda1=lam1, scaling_iter=300, extra_iter=20,
+                           inner_iter_max=50)
+    # the terms of such rows leave FP32: the case is the one that it is meant to be
+    top = (two[1][None, :] - cost.dense()[zero].double()).max() / eps / np.log(2.0)
+    assert float(top) > 128
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.equal(torch.isinf(a), torch.isinf(b)) and not torch.isnan(a).any()
+        fin = torch.isfinite(b)
+        # exponents up to max |C| / eps rounded at 2^-24, times eps, over 640 half-iterations
+        assert float((a - b)[fin].abs().max()) < 640 * 2.0 ** -24 * float(cost.dense().max())
+
+
+@pytest.mark.parametrize('lam1,lam2', [(0.1, 50.0), (0.01, 0.1), (0.002, 0.002)])
+def test_small_penalties(lam1, lam2):
+    """Rows and columns that the plan hardly serves: their sums are far from 1 at every iteration."""
+    import torch
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(2100, 4100, dim=30, n_components=5, seed=4)
+    cost, one, two = _both(dp.x, dp.y, dp.growth, lambda1=lam1, lambda2=lam2)
+    for a, b in zip(one[:2], two[:2]):
+        assert torch.isfinite(a).all()
+        # exponents up to max |C| / eps rounded at 2^-24, times eps, over 340 half-iterations
+        assert float((a - b).abs().max()) < 340 * 2.0 ** -24 * float(cost.dense().max())

@@ -27,11 +27,13 @@
 // terms at a time): a convert and an FP64 multiply-add per entry beside the 11
 // instructions of the term.
 //
-// Range.  A row whose sum leaves [2^-40, 2^40] (its potential moved far: a large
-// change of eps, an outlier cell) is redone at the end of the workgroup with its
-// true maximum.  Terms below 2^-126 are lost: at most I 2^-126 w_i, so a column sum
-// of at least 2^-30 has lost less than 2^-28 of itself; smaller (or overflowed)
-// columns are redone from C^T with an online maximum.
+// Range.  A row whose sum leaves [2^-40, 2^40] or whose weight exceeds 2^40 (its
+// potential moved far: a large change of eps, an outlier cell) is left out of the
+// column sums (its terms may be infinite) and redone at the end of the workgroup
+// with its true maximum.  Terms below 2^-126 are lost: at most I 2^-126 w_i, so a
+// column sum of at least 2^-30 has lost less than 2^-28 of itself; smaller (or
+// overflowed) columns are redone from C^T with an online maximum.  A sum that is no
+// number comes from a NaN in the inputs and stays one.
 #include <algorithm>
 #include <cmath>
 
@@ -46,6 +48,7 @@ constexpr int kCT = kT - 64;       // most threads that own columns; LDS stride 
 constexpr int kMaxRows = 8192;     // rows per workgroup (bad-row bits in LDS)
 constexpr int kMaxChunks = 5;      // groups of four columns per thread (registers; LDS 30 KB each)
 constexpr double kRowLo = 9.094947017729282e-13, kRowHi = 1.099511627776e12;  // 2^-40, 2^40
+constexpr double kWeightHi = 1.099511627776e12;  // 2^40
 constexpr double kColLo = 9.313225746154785e-10, kColHi = 1.2379400392853803e27;  // 2^-30, 2^90
 
 struct RowArgs {
@@ -224,6 +227,9 @@ struct RowPass {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const double w = sh.wrow[it & 1][r];
+            // a row to redo has weight 0, and its terms may be infinite
+            if ((__builtin_amdgcn_readfirstlane(__double2hiint(w)) | __builtin_amdgcn_readfirstlane(__double2loint(w))) == 0)
+                continue;
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -312,7 +318,7 @@ __device__ void finish_rows(const RowArgs &ra, RowShared<R> &sh, int n) {
         const double fn = ra.alpha * ra.eps * (lp + ra.log_nj - lse2 * kLn2);
         const double w = exp2(ra.k * fn + (double)N);
         if ((lane & 15) == 15 && r < R) {
-            const bool out = S < kRowLo || S > kRowHi;
+            const bool out = S < kRowLo || S > kRowHi || w > kWeightHi;
             if (mine && absorb) ra.tau.u[row] = fo;
             if (mine && out) atomicOr(&sh.bad[(it * R + r) >> 5], 1u << ((it * R + r) & 31));
             if (mine && !out) ra.f[row] = fn;
