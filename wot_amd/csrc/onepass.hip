@@ -29,7 +29,7 @@
 //
 // Range.  A row whose sum leaves [2^-40, 2^40] or whose weight exceeds 2^40 (its
 // potential moved far: a large change of eps, an outlier cell) is left out of the
-// column sums (its terms may be infinite) and redone at the end of the workgroup
+// column sums (weight 0, terms kept finite) and redone at the end of the workgroup
 // with its true maximum.  Terms below 2^-126 are lost: at most I 2^-126 w_i, so a
 // column sum of at least 2^-30 has lost less than 2^-28 of itself; smaller (or
 // overflowed) columns are redone from C^T with an online maximum.  A sum that is no
@@ -203,10 +203,14 @@ struct RowPass {
                     e[q] = ldexpf(__builtin_amdgcn_exp2f((float)(y - n)), __builtin_elementwise_sub_sat((int)n, N[r]));
                 }
                 float t = (e[0] + e[1]) + (e[2] + e[3]);
-                if (__builtin_expect(t != t, 0)) {  // an infinite cost (y - n is no number) is a term of 0
+                // An infinite cost (y - n is no number) is a term of 0; a term that overflows stays finite:
+                // its row's sum tells that it has to be redone, and its weight in the columns is 0.
+                if (__builtin_expect(!(t < INFINITY), 0)) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < 4; ++q) {
                         if (fma(-ra.k, (double)cur.v[r][c][q], hk[q]) == -INFINITY) e[q] = 0.f;
+                        if (e[q] == INFINITY) e[q] = 3.0e38f;
+                    }
                     t = (e[0] + e[1]) + (e[2] + e[3]);
                 }
                 s[r] += (double)t;
@@ -227,9 +231,6 @@ struct RowPass {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const double w = sh.wrow[it & 1][r];
-            // a row to redo has weight 0, and its terms may be infinite
-            if ((__builtin_amdgcn_readfirstlane(__double2hiint(w)) | __builtin_amdgcn_readfirstlane(__double2loint(w))) == 0)
-                continue;
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
