@@ -163,11 +163,11 @@ def test_duality_gap_over_several_launches():
     import wot_amd.ot as ot
     x, y, g = _pair(60, 50, 1)
     prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, batch_size=7, tolerance=-1.0, tau=1.0, epsilon0=1.0,
-               max_iter=16390)
+               max_iter=4100)
     st, so = {}, {}
     R = ot.optimal_transport_duality_gap(ot.DeviceCost.from_coordinates(x, y), g, stats=st, **prm)
     ref = O.optimal_transport_duality_gap(O.default_cost_matrix(x, y), G=g, stats=so, **prm)
-    assert st['iterations'] == so['iterations'] == 16390 and st['max_iter_reached'] and so['max_iter_reached']
+    assert st['iterations'] == so['iterations'] == 4100 and st['max_iter_reached'] and so['max_iter_reached']
     assert np.linalg.norm(R - ref) / np.linalg.norm(ref) < 1e-5
 
 
@@ -233,8 +233,8 @@ def test_route_of_the_fixed_schedule(n_i, n_j):
 @pytest.mark.parametrize('n_i,n_j,kw,launches', [
     (120, 150, {}, 1), (300, 400, {}, 1), (400, 300, {}, 1), (300, 360, dict(tolerance=1e-2), 1),
     (300, 360, dict(batch_size=1000), 1), (900, 8000, dict(tau=3.0), 1), (8000, 900, dict(tau=3.0), 1),
-    (2749, 3001, {}, 1), (60, 50, dict(tolerance=-1.0, max_iter=16384), 1),
-    (60, 50, dict(tolerance=-1.0, max_iter=32769), 3)])
+    (2749, 3001, {}, 1), (60, 50, dict(tolerance=-1.0, max_iter=2048), 1),
+    (60, 50, dict(tolerance=-1.0, max_iter=4097), 3)])
 def test_route_of_the_duality_gap_schedule(n_i, n_j, kw, launches):
     import wot_amd.ot as ot
     from wot_amd import _native
@@ -258,30 +258,65 @@ def test_routes_beyond_the_resident_solver():
         assert _route(ws, n_i, n_j) == (want, 0)
 
 
-def test_route_from_threads_and_streams():
-    """Wide and tall pairs from two threads on two streams: both end as resident solves."""
+def test_route_beside_another_solve():
+    """A solve that starts while another is under way takes the sweeps, and neither gives up."""
+    import threading
+    import time
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    shapes = [(300, 400), (1000, 260), (2000, 2500)]
+    pairs = [_pair(i, j, 2) for i, j in shapes]
+    costs = [ot.DeviceCost.from_coordinates(x, y) for x, y, _ in pairs]
+    refs = [_fixed('wotk_transport_stablev2', c, p[2], _workspace(*s)) for c, p, s in zip(costs, pairs, shapes)]
+    long_ws = _workspace(60, 50)
+    x, y, g = _pair(60, 50, 1)
+    long_cost = ot.DeviceCost.from_coordinates(x, y)
+    torch.cuda.synchronize()
+    seen = []
+
+    def long_solve():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            _gap(long_cost, g, long_ws, tolerance=-1.0, max_iter=300000)  # more than 1 s
+
+    t = threading.Thread(target=long_solve)
+    t.start()
+    time.sleep(0.2)
+    for c, p, s, ref in zip(costs, pairs, shapes, refs):
+        ws = _workspace(*s)
+        out = _fixed('wotk_transport_stablev2', c, p[2], ws)
+        seen.append(_route(ws, *s)[0])
+        assert torch.equal(out[0], ref[0]) and torch.equal(out[1], ref[1])
+    assert t.is_alive()
+    t.join()
+    assert seen == [_native.ROUTE_SWEEPS] * 3
+    assert _route(long_ws, 60, 50) == (_native.ROUTE_RESIDENT, 147)
+
+
+def test_routes_of_several_threads():
+    """Wide and tall pairs from four threads: resident or by sweeps, never given up."""
     import threading
     import torch
     import wot_amd.ot as ot
     from wot_amd import _native
-    shapes = [(300, 400), (1000, 260)]
+    shapes = [(300, 400), (1000, 260), (2000, 2500), (30, 20)]
     costs = [ot.DeviceCost.from_coordinates(*_pair(i, j, 2)[:2]) for i, j in shapes]
     torch.cuda.synchronize()
-    routes = [None, None]
+    routes = [[] for _ in shapes]
 
     def work(k):
         with torch.cuda.stream(torch.cuda.Stream()):
             ws = _workspace(*shapes[k])
-            for _ in range(3):
+            for _ in range(4):
                 _gap(costs[k], _pair(*shapes[k], 2)[2], ws)
-            routes[k] = _route(ws, *shapes[k])
+                routes[k].append(_route(ws, *shapes[k])[0])
 
-    ts = [threading.Thread(target=work, args=(k,)) for k in (0, 1)]
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
     for t in ts:
         t.start()
     for t in ts:
         t.join()
-    assert routes == [(_native.ROUTE_RESIDENT, 1)] * 2
+    assert all(r in (_native.ROUTE_RESIDENT, _native.ROUTE_SWEEPS) for rs in routes for r in rs)
 
 
 # ---- what follows when a bound is met: the same bits by another route ----

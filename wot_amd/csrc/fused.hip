@@ -24,6 +24,7 @@
 #include "common.h"
 #include "distance.h"
 #include "fused_problem.h"
+#include "underway.h"
 
 namespace wotk {
 
@@ -776,6 +777,7 @@ static int stablev2_coords_call(const double *X, const double *Y, int64_t I, int
                                 double *f_out, double *g_out, double *row_sums, double *median_out,
                                 void *workspace, size_t workspace_bytes, int32_t polls, wotk_stats *stats,
                                 hipStream_t s) {
+    const UnderWay here;
     WOTK_REQUIRE(scaling_iter >= 0 && extra_iter >= 0 && scaling_iter + extra_iter > 0 && inner_iter_max > 0,
                  "bad iteration counts");
     WOTK_REQUIRE(G != nullptr, "G is required");

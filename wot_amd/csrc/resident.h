@@ -12,10 +12,13 @@ namespace wotk {
 
 // how long a workgroup waits for a value and how much one launch does
 struct ResidentLimits {
-    long long wait_ticks = 20ll * 100000000ll;  // 20 s of the 100 MHz clock, looked at ...
-    unsigned look_mask = 255;                   // ... every 256 polls
-    // 0.08 to 0.25 s, so that no launch holds the chip for long however many iterations a schedule takes
-    long long launch_iters = 16384;
+    // 0.1 s of the 100 MHz clock, looked at every 256 polls: a value takes some us, so a longer wait is
+    // for workgroups without CUs, and sweeps get on beside whatever has them
+    long long wait_ticks = 10000000ll;
+    unsigned look_mask = 255;
+    // 10 to 30 ms, so that no launch holds the chip, or a hardware queue that other streams share, for
+    // long; the next launch costs about 40 us
+    long long launch_iters = 2048;
 };
 
 // whether pairs of this shape take the resident solver
@@ -63,6 +66,9 @@ int resident_fixed(const ResidentProblem &rp, double lambda1, double lambda2, do
 int resident_gap(const ResidentProblem &rp, double lambda1, double lambda2, double epsilon, long long batch_size,
                  double tolerance, double tau, double epsilon0, long long max_iter, const ResidentLimits &lim,
                  int *launched, ResidentResult *out, hipStream_t s);
+
+// leaves the result of no launch on rp, for a solve that does not take the resident solver
+int resident_pass_by(const ResidentProblem &rp, hipStream_t s);
 
 // the result of the last resident launch on rp (waits for it)
 int resident_result(const ResidentProblem &rp, ResidentResult *out, hipStream_t s);

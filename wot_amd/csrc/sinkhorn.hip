@@ -25,6 +25,7 @@
 #include "fused_problem.h"
 #include "onepass.h"
 #include "resident.h"
+#include "underway.h"
 
 namespace wotk {
 
@@ -978,6 +979,14 @@ static ResidentProblem resident_problem(const Problem &pb, const Work &w) {
                            w.exchange};
 }
 
+// w.exchange stays only where the solve takes the resident route; the route is left in the workspace
+static int resident_or_not(const Problem &pb, Work &w, const UnderWay &here, hipStream_t s) {
+    if (!w.exchange || here.alone()) return WOTK_OK;
+    const int rc = resident_pass_by(resident_problem(pb, w), s);
+    w.exchange = nullptr;
+    return rc;
+}
+
 // the fixed-iteration schedule on a set-up problem (shared by the workspace
 // and the scratch entry points); `timed` brackets the sweeps with events
 static int stablev2_run(const Problem &pb, Work &w, double lambda1, double lambda2, double epsilon,
@@ -1069,9 +1078,12 @@ static int stablev2_call(const float *C, int64_t ldc, const float *CT, int64_t l
                          double epsilon0, int64_t extra_iter, int64_t inner_iter_max, double *plan, int64_t ldp,
                          double *row_sums, double *f_out, double *g_out, void *workspace, size_t workspace_bytes,
                          const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
+    const UnderWay here;
     Problem pb;
     Work w;
     int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    if (rc) return rc;
+    rc = resident_or_not(pb, w, here, s);
     if (rc) return rc;
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
                         ldp, row_sums, f_out, g_out, true, lim, stats, s);
@@ -1124,7 +1136,6 @@ extern "C" int wotk_probe_stablev2_limits(const float *C, int64_t ldc, const flo
 // (calls that overlap on one GPU race); the solver initialises every part of
 // the state it reads, so the previous call's contents do not matter.
 constexpr size_t kScratchBytes = (size_t)16 << 20;  // 16 MiB: I, J up to ~95,000
-constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static void *g_scratch_ptr[kMaxDevices];  // device address of `scratch` on each GPU (host-side)
 static std::mutex g_scratch_mutex;
@@ -1164,6 +1175,7 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
                  "%lld x %lld needs %zu bytes of solver state; the no-allocation entry point holds %zu "
                  "(use wotk_transport_stablev2 with a workspace)",
                  (long long)I, (long long)J, need, kScratchBytes);
+    const UnderWay here;
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
     int rc = scratch_ptr(&ws);
@@ -1418,9 +1430,12 @@ static int duality_gap_call(const float *C, int64_t ldc, const float *CT, int64_
                             double tolerance, double tau, double epsilon0, int64_t max_iter, double *plan,
                             int64_t ldp, double *row_sums, double *f_out, double *g_out, void *workspace,
                             size_t workspace_bytes, const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
+    const UnderWay here;
     Problem pb;
     Work w;
     int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    if (rc) return rc;
+    rc = resident_or_not(pb, w, here, s);
     if (rc) return rc;
     WOTK_REQUIRE(!plan || ldp >= J, "ldp < J");
     StoredBackend be{pb, w, plan, ldp, row_sums, f_out, g_out};
@@ -1586,6 +1601,7 @@ extern "C" int wotk_transport_duality_gap_coords(const double *X, const double *
                                                  int64_t max_iter, int32_t terms, double *f_out, double *g_out,
                                                  double *row_sums, double *median_out, void *workspace,
                                                  size_t workspace_bytes, wotk_stats *stats, void *stream) {
+    const UnderWay here;
     hipStream_t s = (hipStream_t)stream;
     WOTK_REQUIRE(G != nullptr, "G is required");
     FusedProblem fp;
