@@ -87,3 +87,34 @@ def test_median_of_the_never_stored_pair():
         r = large.transport_stablev2_coords(x, y, np.ones(n_i), scaling_iter=1, extra_iter=0)
         cost = ot.DeviceCost.from_coordinates(x, y)
         assert float(r.median.cpu()[0]) == float(cost.median.cpu()[0])
+
+
+# more equal distances than the middle bins' list holds: one value, the two middle ranks in two values, a few
+# values, one value among unequal ones; with the candidate lists and without (never stored)
+@pytest.mark.parametrize('kind', ['one', 'halves', 'few', 'spike'])
+@pytest.mark.parametrize('n_i,n_j', [(520, 514), (2100, 2003)])
+def test_heavy_ties(kind, n_i, n_j):
+    import wot_amd.ot as ot
+    from wot_amd.ot import large
+    rng = np.random.default_rng(n_i)
+    x, y = np.zeros((n_i, 3)), np.ones((n_j, 3))
+    if kind == 'halves':
+        x[n_i // 2:] = 3.0
+    elif kind == 'few':
+        x, y = rng.integers(0, 3, (n_i, 3)).astype(float), rng.integers(0, 3, (n_j, 3)).astype(float)
+    elif kind == 'spike':
+        x[: 2 * n_i // 5] = rng.random((2 * n_i // 5, 3))
+        y[: n_j // 5] = 4.0 + rng.random((n_j // 5, 3))
+    cost = ot.DeviceCost.from_coordinates(x, y)
+    D = np.zeros((n_i, n_j))
+    for k in range(3):
+        D += (x[:, k, None] - y[None, :, k]) ** 2
+    # sums of three squares in another order of rounding than the device's: only the exact kinds compare by bits
+    flat = np.sort(D.ravel())
+    lo, hi = flat[(flat.size - 1) // 2], flat[flat.size // 2]
+    med, idx = float(cost.median.cpu()[0]), cost.median_index.cpu().numpy()
+    assert med == pytest.approx((lo + hi) / 2, rel=1e-15 if kind != 'spike' else 1e-14)
+    if kind != 'spike':
+        assert idx[0] == np.flatnonzero(D.ravel() == lo)[0] and idx[1] == np.flatnonzero(D.ravel() == hi)[0]
+    r = large.transport_stablev2_coords(x, y, np.ones(n_i), scaling_iter=1, extra_iter=0)
+    assert float(r.median.cpu()[0]) == med

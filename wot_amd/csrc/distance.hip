@@ -14,7 +14,8 @@
 //              holding the one or two middle ranks in one workgroup)
 // When the bracket misses the rank or heavy ties overflow the kept list, a device
 // flag starts a six-digit radix select that regenerates the distances per digit;
-// otherwise its launches exit at once.  Bound: FP64 issue (2 d operations per entry
+// otherwise its launches exit at once.  (Coordinates of 4 integers, d = 30: 6.8 ms for
+// 15000 x 15000, 0.70 ms for 4000 x 3500; read from a stored matrix 68.8 and 4.7 ms.)  Bound: FP64 issue (2 d operations per entry
 // and pass at 3.4e13 / s).  15000 x 15000, d = 30, cost and median: 1.57 ms (0.75 ms
 // collect, 0.7 ms write, 0.08 ms selection) against 4.73 ms with a stored FP64 matrix
 // read by six digit passes, a next-above, an index and a normalise pass (88 bytes
@@ -252,7 +253,7 @@ struct MedianBuffers {
     unsigned *key32;          // samples
     unsigned *seg_count;      // per segment, 64 unsigneds apart
     u64 *seg_below;           // per segment, 32 u64 apart
-    unsigned *hist;           // candidate bins
+    u64 *hist;                // candidate bins
     u64 *fhist;               // fallback digit bins
     u64 *cand_key, *cand_idx;
     u64 *list_key, *list_idx;
@@ -275,7 +276,7 @@ static size_t median_carve(Arena &ar, int64_t I, int64_t J, bool lean, MedianBuf
     b->key32 = ar.take<unsigned>(kSamplesLarge);
     b->seg_count = ar.take<unsigned>(kSegments * 64);
     b->seg_below = ar.take<u64>(kSegments * 32);
-    b->hist = ar.take<unsigned>(kCandBins);
+    b->hist = ar.take<u64>(kCandBins);
     b->fhist = ar.take<u64>(kRadixBins);
     b->cand_key = ar.take<u64>((size_t)b->seg_cap * b->n_seg);
     b->cand_idx = ar.take<u64>((size_t)b->seg_cap * b->n_seg);
@@ -290,9 +291,9 @@ size_t distance_median_bytes(int64_t I, int64_t J, bool lean) {
     return median_carve(ar, I, J, lean, &b) + 256;
 }
 
-// inclusive scan over a 1024-thread workgroup (16 waves); red: 16 entries
+// inclusive scan over a workgroup; red: one entry per wave
 template <typename T>
-__device__ inline T block_scan_1024(T x, T *red) {
+__device__ inline T block_scan(T x, T *red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -307,14 +308,14 @@ __device__ inline T block_scan_1024(T x, T *red) {
     return x + before;
 }
 
-// true in the workgroup that finishes last; its loads after this see the other
-// workgroups' stores (every thread fences before the ticket and after it)
+// true in the workgroup that finishes last, which reads with load_dev what the others added up with
+// atomics: each wave has waited for its own by then.  (A fence per thread instead, whose release
+// writes back the L2, made a pass over 3000 x 3000 take 130 us, now 50.)
 __device__ inline bool last_block(unsigned *ticket, int *flag) {
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) *flag = atomicAdd(ticket, 1u) == gridDim.x - 1;
     __syncthreads();
-    __threadfence();
     return *flag != 0;
 }
 
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(1024) void dist_bracket_kernel(const unsigned *__re
     MedianState *st = b.st;
     for (int k = t; k < kSegments * 64; k += 1024) b.seg_count[k] = 0u;
     for (int k = t; k < kSegments * 32; k += 1024) b.seg_below[k] = 0ull;
-    for (int k = t; k < kCandBins; k += 1024) b.hist[k] = 0u;
+    for (int k = t; k < kCandBins; k += 1024) b.hist[k] = 0ull;
     for (int k = t; k < kRadixBins; k += 1024) b.fhist[k] = 0ull;
     if (t == 0) {
         st->fallback = 0;
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(1024) void dist_bracket_kernel(const unsigned *__re
             c[q] = h[4 * t + q];
             mine += c[q];
         }
-        unsigned before = block_scan_1024(mine, red) - mine;
+        unsigned before = block_scan(mine, red) - mine;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(1024) void dist_bracket_kernel(const unsigned *__re
     for (int w = 0; w < 2; ++w) {
         if (want[w] < 0 || want[w] >= m) continue;  // uniform
         const unsigned c0 = h[w * 2048 + 2 * t], c1 = h[w * 2048 + 2 * t + 1];
-        const unsigned before = block_scan_1024(c0 + c1, red) - (c0 + c1);
+        const unsigned before = block_scan(c0 + c1, red) - (c0 + c1);
         const long long r = want[w] - (long long)base_rank[w];
         if (r >= (long long)before && r < (long long)before + c0) res[w] = 2 * t;
         else if (r >= (long long)before + c0 && r < (long long)before + c0 + c1) res[w] = 2 * t + 1;
@@ -496,7 +497,19 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
     u64 below_all = 0;
     const u64 prefix = st->prefix, mask = st->mask;
     const u64 lo_key = st->lo_key, hi_key = st->hi_key;
-    u64 best = ~0ull;
+    u64 best = ~0ull, best_hi = ~0ull;
+    // Equal bins one after the other go to LDS as one add: where distances are tied, all lanes of a
+    // wave meet in one bin, entry after entry.
+    int run_bin = -1;
+    unsigned run = 0;
+    auto count_bin = [&](int bin) {
+        if (bin != run_bin) {
+            if (run) atomicAdd(&h[run_bin], run);
+            run_bin = bin;
+            run = 0;
+        }
+        ++run;
+    };
     const int64_t n_tiles = (int64_t)pa.tiles_i * pa.tiles_j;
     for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
         Tile tile;
@@ -562,57 +575,74 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
                 const u64 k = (u64)__double_as_longlong(tile.v[e]);
                 if (MODE == kBins) {
                     below_all += k < lo;
-                    if (k >= lo && k <= hi) atomicAdd(&h[(k - lo) >> bin_shift], 1u);
+                    if (k >= lo && k <= hi) count_bin((int)((k - lo) >> bin_shift));
                 } else if (MODE == kGather) {
                     if (k >= lo && k <= hi) {
                         const unsigned at = atomicAdd(&st->n_list, 1u);
-                        if (at < (unsigned)kListCap) {
+                        if (at < (unsigned)kListCap) {  // place_rank_kernel has seen to it
                             pa.b.list_key[at] = k;
                             pa.b.list_idx[at] = (u64)tile.row(e) * (u64)pa.pb.n_j + (u64)tile.col(e);
                         }
                     }
                 } else if (MODE == kDigit) {
-                    if ((k & mask) == prefix) atomicAdd(&h[(k >> pa.shift) & ((1ull << pa.width) - 1ull)], 1u);
+                    if ((k & mask) == prefix) count_bin((int)((k >> pa.shift) & ((1ull << pa.width) - 1ull)));
                 } else if (MODE == kNextAbove) {
                     if (k > prefix && k < best) best = k;
                 } else {
                     const u64 idx = (u64)tile.row(e) * (u64)pa.pb.n_j + (u64)tile.col(e);
-                    if (k == lo_key) atomicMin(&pa.index_out[0], idx);
-                    if (k == hi_key) atomicMin(&pa.index_out[1], idx);
+                    if (k == lo_key && idx < best) best = idx;
+                    if (k == hi_key && idx < best_hi) best_hi = idx;
                 }
             }
         }
     }
-    if constexpr (MODE == kBins) {
+    if constexpr (NH > 1) {
+        if (run) atomicAdd(&h[run_bin], run);
         __syncthreads();
+    }
+    if constexpr (MODE == kBins) {
         for (int q = tid; q < kCandBins; q += 256)
-            if (h[q]) atomicAdd(&pa.b.hist[q], h[q]);
+            if (h[q]) atomicAdd(&pa.b.hist[q], (u64)h[q]);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) below_all += __shfl_xor(below_all, off);
         if (lane == 0) atomicAdd(&pa.b.seg_below[(blockIdx.x % kSegments) * 32], below_all);
     }
     if constexpr (MODE == kDigit) {
-        __syncthreads();
         for (int q = tid; q < kRadixBins; q += 256)
             if (h[q]) atomicAdd(&pa.b.fhist[q], (u64)h[q]);
         if (!last_block(&st->ticket[0], &is_last)) return;
-        if (tid == 0) {
-            st->ticket[0] = 0u;
-            const int nb = 1 << pa.width;
-            u64 cum = 0;
-            int q = 0;
-            u64 c = load_dev(&pa.b.fhist[0]);
-            while (q < nb - 1 && cum + c <= (u64)st->frank) {
-                cum += c;
-                c = load_dev(&pa.b.fhist[++q]);
-            }
-            st->prefix |= (u64)q << pa.shift;
-            st->mask |= ((1ull << pa.width) - 1ull) << pa.shift;
-            st->frank -= (long long)cum;
-            if (pa.last) st->eq = c;
+        // the digit's bin that holds the rank: eight bins per thread
+        constexpr int PER = kRadixBins / 256;
+        const u64 want = (u64)st->frank;
+        u64 c[PER], mine = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            c[q] = load_dev(&pa.b.fhist[PER * tid + q]);
+            mine += c[q];
         }
-        __syncthreads();
+        u64 before = block_scan(mine, wbelow) - mine;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            if (want >= before && want < before + c[q]) {  // one thread, one bin
+                st->prefix |= (u64)(PER * tid + q) << pa.shift;
+                st->mask |= ((1ull << pa.width) - 1ull) << pa.shift;
+                st->frank -= (long long)before;
+                if (pa.last) st->eq = c[q];
+            }
+            before += c[q];
+        }
+        if (tid == 0) st->ticket[0] = 0u;
         for (int q = tid; q < kRadixBins; q += 256) pa.b.fhist[q] = 0ull;
+    }
+    if constexpr (MODE == kIndex) {  // one atomic per wave: tied keys are many
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const u64 o = __shfl_xor(best, off), p = __shfl_xor(best_hi, off);
+            best = o < best ? o : best;
+            best_hi = p < best_hi ? p : best_hi;
+        }
+        if (lane == 0 && best != ~0ull) atomicMin(&pa.index_out[0], best);
+        if (lane == 0 && best_hi != ~0ull) atomicMin(&pa.index_out[1], best_hi);
     }
     if constexpr (MODE == kNextAbove) {
 #pragma unroll
@@ -640,7 +670,7 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
 __global__ __launch_bounds__(1024) void place_rank_kernel(MedianBuffers b, int odd) {
     __shared__ u64 red[16];
     __shared__ int over, bin[2];
-    __shared__ u64 start[2];
+    __shared__ u64 start[2], end[2];
     const int t = threadIdx.x;
     MedianState *st = b.st;
     if (t == 0) over = 0;
@@ -651,7 +681,7 @@ __global__ __launch_bounds__(1024) void place_rank_kernel(MedianBuffers b, int o
         below = load_dev(&b.seg_below[t * 32]);
         if (load_dev(&b.seg_count[t * 64]) > b.seg_cap) over = 1;
     }
-    const u64 below_all = block_scan_1024(below, red);
+    const u64 below_all = block_scan(below, red);
     if (t == 1023) start[0] = below_all;
     __syncthreads();
     const long long r = st->rank - (long long)start[0];  // rank of the lower middle among the candidates
@@ -662,7 +692,7 @@ __global__ __launch_bounds__(1024) void place_rank_kernel(MedianBuffers b, int o
         c[q] = load_dev(&b.hist[4 * t + q]);
         mine += c[q];
     }
-    u64 before = block_scan_1024(mine, red) - mine;
+    u64 before = block_scan(mine, red) - mine;
     const long long want[2] = {r, odd ? r : r + 1};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -671,12 +701,14 @@ __global__ __launch_bounds__(1024) void place_rank_kernel(MedianBuffers b, int o
             if (want[w] >= (long long)before && want[w] < (long long)(before + c[q])) {
                 bin[w] = 4 * t + q;
                 start[w] = before;
+                end[w] = before + c[q];
             }
         before += c[q];
     }
     __syncthreads();
     if (t == 0) {
-        if (over || bin[0] < 0 || bin[1] < 0) {
+        // heavy ties in the middle bins: no list holds them
+        if (over || bin[0] < 0 || bin[1] < 0 || end[1] - start[0] > (u64)kListCap) {
             st->fallback = 1;
         } else {
             const u64 lo = st->lo;
@@ -703,7 +735,7 @@ __global__ __launch_bounds__(1024) void cand_hist_kernel(MedianBuffers b) {
     }
     __syncthreads();
     for (int q = t; q < kCandBins; q += 1024)
-        if (h[q]) atomicAdd(&b.hist[q], h[q]);
+        if (h[q]) atomicAdd(&b.hist[q], (u64)h[q]);
 }
 
 // Exact order statistics of n (key, index) pairs, n >= 1, by one 1024-thread
@@ -749,7 +781,7 @@ __device__ void list_select(const u64 *keys, const u64 *idx, unsigned n, long lo
         }
         __syncthreads();
         const unsigned c0 = h[2 * t], c1 = h[2 * t + 1];
-        const unsigned before = block_scan_1024(c0 + c1, red) - (c0 + c1);
+        const unsigned before = block_scan(c0 + c1, red) - (c0 + c1);
         if (r >= before && r < before + c0) {
             sel_bin = 2 * t;
             sel_cum = before;
@@ -833,11 +865,6 @@ __global__ __launch_bounds__(1024) void cand_gather_kernel(MedianBuffers b) {
 __global__ __launch_bounds__(1024) void list_select_kernel(MedianBuffers b, int odd, u64 *index_out) {
     MedianState *st = b.st;
     if (st->fallback) return;
-    if (st->n_list > (unsigned)kListCap) {  // heavy ties in the middle bins
-        __syncthreads();
-        if (threadIdx.x == 0) st->fallback = 1;
-        return;
-    }
     list_select(b.list_key, b.list_idx, st->n_list, st->rank, odd, st, index_out);
 }
 
