@@ -118,3 +118,11 @@ def test_heavy_ties(kind, n_i, n_j):
         assert idx[0] == np.flatnonzero(D.ravel() == lo)[0] and idx[1] == np.flatnonzero(D.ravel() == hi)[0]
     r = large.transport_stablev2_coords(x, y, np.ones(n_i), scaling_iter=1, extra_iter=0)
     assert float(r.median.cpu()[0]) == med
+
+
+# either side of the bounds of one list (24576 entries) and of 16 lists (2^22)
+@pytest.mark.parametrize('n_i,n_j', [(128, 192), (157, 157), (2047, 2048), (2048, 2048)])
+@pytest.mark.parametrize('kind', ['normal', 'sorted_clusters'])
+def test_number_of_candidate_lists(kind, n_i, n_j):
+    for mode in ('f64', 'bf16x6'):
+        test_cost_and_median(kind, n_i, n_j, 30, mode)

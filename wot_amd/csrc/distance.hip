@@ -15,11 +15,11 @@
 // When the bracket misses the rank or heavy ties overflow the kept list, a device
 // flag starts a six-digit radix select that regenerates the distances per digit;
 // otherwise its launches exit at once.  (Coordinates of 4 integers, d = 30: 6.8 ms for
-// 15000 x 15000, 0.70 ms for 4000 x 3500; read from a stored matrix 68.8 and 4.7 ms.)  Bound: FP64 issue (2 d operations per entry
-// and pass at 3.4e13 / s).  15000 x 15000, d = 30, cost and median: 1.57 ms (0.75 ms
-// collect, 0.7 ms write, 0.08 ms selection) against 4.73 ms with a stored FP64 matrix
-// read by six digit passes, a next-above, an index and a normalise pass (88 bytes
-// per entry); 1215 x 1163: 0.11 ms against 0.38 ms.
+// 15000 x 15000, 0.70 ms for 4000 x 3500; read from a stored matrix 68.8 and 4.7 ms.)
+// Bound: FP64 issue (2 d operations per entry and pass at 3.4e13 / s).  15000 x 15000,
+// d = 30, cost and median: 1.57 ms (0.75 ms collect, 0.7 ms write, 0.08 ms selection)
+// against 4.73 ms with a stored FP64 matrix read by six digit passes, a next-above, an
+// index and a normalise pass (88 bytes per entry); 1215 x 1163: 0.11 ms against 0.38 ms.
 #include <algorithm>
 
 #include "distance.h"
@@ -222,11 +222,16 @@ struct Bf16Tile {
 // ---------------------------------------------------------------------------
 // median state and buffers
 // ---------------------------------------------------------------------------
-constexpr int kSegments = 256;        // candidate lists (one append counter each, spread over the tiles)
+// candidate lists (one append counter each, spread over the tiles), at most; 16 below 2^22 entries, where
+// a tile's worth of slack in each would be most of the workspace
+constexpr int kSegments = 256;
 constexpr int kCandBins = 4096;
 constexpr int kListCap = 1 << 16;     // entries of the middle bins
 constexpr int kRadixBins = 2048;
-constexpr int64_t kCollectAll = 1 << 18;   // pairs up to this many entries: every entry is a candidate
+// Pairs up to this many entries: every entry is a candidate, and one workgroup selects among all of
+// them (us for cost and median, so / with the bracket; normal, then integer coordinates: 120 x 127
+// 95 / 120, 99 / 118; 150 x 157 107 / 121, 115 / 116; 180 x 187 120 / 122, 135 / 118; 300 x 307 197 / 123).
+constexpr int64_t kCollectAll = 3 << 13;
 // Above this many entries the candidate lists (2 bytes per entry) are not worth their
 // memory: one more regeneration (0.4 ms per 2^28 entries) takes their place.
 constexpr int64_t kLeanEntries = 1ll << 28;
@@ -258,7 +263,7 @@ struct MedianBuffers {
     u64 *cand_key, *cand_idx;
     u64 *list_key, *list_idx;
     unsigned seg_cap;
-    int n_seg;
+    int n_seg, seg_shift;     // 2^(32 - seg_shift) lists
     int n_samples;
     int lean;                 // no candidate lists: a counting pass and a gathering pass
 };
@@ -268,9 +273,10 @@ static size_t median_carve(Arena &ar, int64_t I, int64_t J, bool lean, MedianBuf
     const bool all = n <= kCollectAll;
     b->lean = !all && (lean || n > kLeanEntries);
     b->n_samples = all ? 0 : (n < (1ll << 22) ? kSamplesSmall : kSamplesLarge);
-    b->n_seg = all ? 1 : kSegments;
-    // 12.5 % of the entries (the bracket holds 2.3-4.7 %), spread over the segments
-    const int64_t cap = all ? n : b->lean ? 0 : n / 8 + kSegments * 16384;
+    b->n_seg = all ? 1 : n < (1ll << 22) ? 16 : kSegments;
+    b->seg_shift = b->n_seg == kSegments ? 24 : 28;
+    // 12.5 % of the entries (the bracket holds 2.3-4.7 %), spread over the segments, and a tile each
+    const int64_t cap = all ? n : b->lean ? 0 : n / 8 + b->n_seg * 16384;
     b->seg_cap = (unsigned)((cap + b->n_seg - 1) / b->n_seg);
     b->st = ar.take<MedianState>(1);
     b->key32 = ar.take<unsigned>(kSamplesLarge);
@@ -541,7 +547,7 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
             __syncthreads();
             // lists spread over the tiles by a multiplicative hash, so that runs of similar tiles
             // (cells sorted by cluster) do not fill one segment
-            const int seg = pa.b.n_seg == 1 ? 0 : (int)(((unsigned)t * 2654435761u) >> 24);
+            const int seg = pa.b.n_seg == 1 ? 0 : (int)(((unsigned)t * 2654435761u) >> pa.b.seg_shift);
             if (tid == 0) {
                 wbase = atomicAdd(&pa.b.seg_count[seg * 64], wsum[0] + wsum[1] + wsum[2] + wsum[3]);
                 atomicAdd(&pa.b.seg_below[seg * 32], wbelow[0] + wbelow[1] + wbelow[2] + wbelow[3]);
@@ -899,9 +905,9 @@ static int median_passes(const DistanceProblem &pb, const MedianBuffers &b, int6
     } else {
         dist_pass_kernel<Tile, kCollect><<<(unsigned)std::min<int64_t>(tiles, 1 << 20), 256, 0, s>>>(pa);
         if (b.n_samples) {
-            cand_hist_kernel<<<kSegments, 1024, 0, s>>>(b);
+            cand_hist_kernel<<<b.n_seg, 1024, 0, s>>>(b);
             place_rank_kernel<<<1, 1024, 0, s>>>(b, odd);
-            cand_gather_kernel<<<kSegments, 1024, 0, s>>>(b);
+            cand_gather_kernel<<<b.n_seg, 1024, 0, s>>>(b);
             list_select_kernel<<<1, 1024, 0, s>>>(b, odd, idx);
         }
     }
