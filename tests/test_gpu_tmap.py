@@ -386,3 +386,24 @@ def test_propagate_at_the_edges_of_its_splits(sizes, k, dtype):
                         tol = 2 * (2 * sum(sizes) + 8 * len(maps)) * 2.0 ** -53
                         assert float(((outs[s] - ref) / ref).abs().max()) < tol
                 assert got is outs[-1]
+
+
+# numbers of workgroups per split on either side of the split rule's bounds (push: cells out / 64, 4 or 2
+# population groups per layer; pull: cells out / 256), long and short reductions
+@pytest.mark.parametrize('rows,cols,k', [(8300, 16512, 3), (8300, 13000, 5), (900, 16512, 3), (8200, 33000, 3),
+                                         (300, 70000, 40), (16600, 8300, 40), (70000, 300, 20), (10100, 8210, 3)])
+def test_split_rule(tm, rows, cols, k):
+    import torch
+    gen = torch.Generator(device='cuda').manual_seed(rows)
+    M = torch.rand(rows, cols, dtype=torch.float32, device='cuda', generator=gen)
+    dm = tm.DeviceMap.upload(M, 'float32')
+    D = M.double()
+    for direction, T in ((tm.PUSH_FORWARD, D.T), (tm.PULL_BACK, D)):
+        P = torch.rand(T.shape[1], k, dtype=torch.float64, device='cuda', generator=gen)
+        ref = T @ P
+        for normalize in (False, True):
+            out = tm.propagate([dm], P, direction, normalize=normalize)
+            want = ref / ref.sum(0) if normalize else ref
+            # positive FP64 sums of at most 70000 products in another order
+            assert float(((out - want) / want).abs().max()) < 70000 * 2.0 ** -53 * 4
+    del M, D

@@ -569,10 +569,20 @@ StepShape step_shape(const wotk_tmap &m, int direction, int n_groups) {
     s.n_tiles = (int)tiles;
     // push: a workgroup's waves share the split's rows, four row trips at least for each wave
     const int64_t quantum = push ? 16 * kWaves : pull_step_cols(m.dtype);
-    const int64_t waves = push ? kWaves : 1, least = push ? 4 : 8;
+    const int64_t least = push ? 4 : 8;
     // as many splits as kTargetWaves waves hold, each reduction chunk >= `least` quanta
+    constexpr int64_t places = kTargetWaves / kWaves;
     const int64_t layers = push ? (n_groups + 1) / 2 : n_groups;  // a push wave takes two groups
-    int64_t want = kTargetWaves / (waves * tiles * layers);
+    const int64_t wgs = (push ? tiles : (tiles + kWaves - 1) / kWaves) * layers;
+    int64_t want = places / wgs;
+    // One or two splits can leave much of the one round of workgroups empty (20000 cells, push: 313 of
+    // 512).  Then more and shorter ones, which the chip balances, as long as their partial sums stay
+    // small beside the map: us at 1 / 2 / 4 / 8 splits, push, 10 populations, FP32, 12000 x 12000
+    // 231 / 171 / 133 / 132, 20000 x 20000 493 / 353 / 324 / 317, 4000 x 24576 112 / 97 / 102 / 111; pull,
+    // 40 populations, at 1 / 2 / 5 / 8, 24000 x 24000 2620 / 2025 / 1710 / 1670.  Above two rounds one
+    // split: 130000 x 2000, pull, at 1 / 2 / 5 / 8 376 / 394 / 420 / 430.
+    const bool filled = want > 2 || (want == 2 && 10 * wgs >= 4 * places) || (want == 1 && 8 * wgs >= 7 * places);
+    if (!filled) want = wgs > 2 * places ? 1 : s.reduce_len < 8192 ? 2 : push ? 4 : 5;
     int64_t most = std::max<int64_t>(1, s.reduce_len / (least * quantum));
     int64_t splits = std::max<int64_t>(1, std::min(want, most));
     s.split_len = round_up((s.reduce_len + splits - 1) / splits, quantum);
