@@ -407,3 +407,25 @@ def test_split_rule(tm, rows, cols, k):
             # positive FP64 sums of at most 70000 products in another order
             assert float(((out - want) / want).abs().max()) < 70000 * 2.0 ** -53 * 4
     del M, D
+
+
+# cells on either side of 512 blocks of 64, where the blocks' sums are folded before their use
+@pytest.mark.parametrize('wide', [32768, 32769, 50001])
+@pytest.mark.parametrize('k', [3, 20])
+def test_totals_of_many_cells(tm, wide, k):
+    import torch
+    gen = torch.Generator(device='cuda').manual_seed(wide + k)
+    maps = [torch.rand(s, dtype=torch.float64, device='cuda', generator=gen)
+            for s in ((150, wide), (wide, 130), (130, wide))]
+    dms = [tm.DeviceMap.upload(m) for m in maps]
+    P = torch.rand(150, k, dtype=torch.float64, device='cuda', generator=gen)
+    outs = [torch.empty(m.shape[1], k, dtype=torch.float64, device='cuda') for m in maps]
+    tm.propagate(dms, P, tm.PUSH_FORWARD, outs=outs)
+    p = P
+    for m, o in zip(maps, outs):
+        p = m.T @ p
+        p /= p.sum(0)
+        # three maps' positive FP64 sums of at most 50001 products each, and their totals
+        assert float(((o - p) / p).abs().max()) < 6 * 50001 * 2.0 ** -53
+    back = tm.propagate(dms[:1], torch.rand(wide, k, dtype=torch.float64, device='cuda', generator=gen), tm.PULL_BACK)
+    assert float((back.sum(0) - 1.0).abs().max()) < 1e-12

@@ -58,6 +58,8 @@ struct PopSums {
     int n_blocks, n_pops;
 };
 
+constexpr int kFoldBlocks = 512;
+
 // total of population group * 16 + l % 16 in every lane l (1 where there is none); all WAVES
 // waves of the workgroup
 template <int WAVES>
@@ -496,6 +498,12 @@ __global__ __launch_bounds__(kReduceThreads) void pops_reduce_kernel(const doubl
     }
 }
 
+// many blocks' sums as one: what every workgroup of the next product and of the output would add up itself
+__global__ __launch_bounds__(1024) void pops_fold_kernel(PopSums ps, double *__restrict__ out) {
+    const double t = pop_total<16>(ps, blockIdx.x);
+    if (threadIdx.x < kPopTile) out[blockIdx.x * kPopTile + threadIdx.x] = t;
+}
+
 __global__ __launch_bounds__(kReduceThreads) void pops_export_kernel(PopExport ex) {
     export_cells(ex, blockIdx.y, blockIdx.x);
 }
@@ -592,7 +600,8 @@ StepShape step_shape(const wotk_tmap &m, int direction, int n_groups) {
 }
 
 struct Layout {
-    double *part = nullptr, *pop_a = nullptr, *pop_b = nullptr, *block_sums[2] = {nullptr, nullptr};
+    double *part = nullptr, *pop_a = nullptr, *pop_b = nullptr, *block_sums[2] = {nullptr, nullptr},
+           *totals[2] = {nullptr, nullptr};
 };
 
 int check_chain(const wotk_tmap *maps, int32_t n_maps, int32_t direction, int32_t n_pops) {
@@ -634,6 +643,7 @@ Layout carve(Arena &ar, const wotk_tmap *maps, int32_t n_maps, int32_t direction
     L.pop_a = ar.take<double>((size_t)max_cells * n_groups * kPopTile);
     L.pop_b = ar.take<double>((size_t)max_cells * n_groups * kPopTile);
     for (double *&sums : L.block_sums) sums = ar.take<double>((size_t)max_blocks * n_groups * kPopTile);
+    for (double *&sums : L.totals) sums = ar.take<double>((size_t)n_groups * kPopTile);
     return L;
 }
 
@@ -738,6 +748,11 @@ extern "C" int wotk_tmap_propagate(const wotk_tmap *maps, int32_t n_maps, int32_
             L.part, sh.n_split, sh.n_out, n_blocks, nxt, sums, ex);
         WOTK_LAUNCH_CHECK();
         scale = PopSums{normalize ? sums : nullptr, n_blocks, n_pops};
+        if (normalize && n_blocks > kFoldBlocks) {
+            pops_fold_kernel<<<n_groups, 1024, 0, st>>>(scale, L.totals[s & 1]);
+            WOTK_LAUNCH_CHECK();
+            scale = PopSums{L.totals[s & 1], 1, n_pops};
+        }
         ex = PopExport{nxt, sh.n_out, n_pops, scale, outs[s], ldo};
         std::swap(cur, nxt);
     }
