@@ -130,10 +130,10 @@ int wotk_transport_stablev2(const float *C, int64_t ldc, const float *CT, int64_
  * serving loops, harnesses that forbid hipMalloc).  Arguments and outputs are
  * those of wotk_transport_stablev2 without the workspace: the solver state
  * lives in one static device array per GPU of wotk_scratch_capacity() bytes
- * (16 MiB: wotk_solver_workspace_size(I, J) must fit, i.e. I, J up to about
- * 95,000; larger problems are rejected with WOTK_EINVAL).  The call allocates
- * nothing (no hipMalloc / hipFree, no events: stats->sweep_ms is 0); calls that
- * overlap on one GPU share the array and race. */
+ * (16 MiB: I, J up to 133,120; larger problems are rejected with
+ * WOTK_EINVAL).  The call allocates nothing (no hipMalloc / hipFree, no
+ * events: stats->sweep_ms is 0); calls that overlap on one GPU share the
+ * array and race. */
 size_t wotk_scratch_capacity(void);
 int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I,
                                     int64_t J, const double *G, double lambda1, double lambda2,

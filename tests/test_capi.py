@@ -107,3 +107,17 @@ def test_solver_route_checks_its_arguments_on_the_host():
     assert lib.wotk_solver_route(40, 50, 256, 1 << 20, None, None, None) == _native.WOTK_EINVAL
     assert lib.wotk_solver_route(40, 50, None, 1 << 20, *out, None) == _native.WOTK_EWORKSPACE
     assert lib.wotk_solver_route(40, 50, 256, 64, *out, None) == _native.WOTK_EWORKSPACE
+
+
+def test_no_allocation_entry_point_takes_the_largest_pairs():
+    """The static array holds the sweeps' state only: pairs up to its 16 MiB, not less for other solvers' sake."""
+    lib = _native.lib()
+
+    def refused(n_i, n_j):  # without G no pair is solved: the size is looked at first
+        rc = lib.wotk_transport_stablev2_noalloc(None, 1 << 20, None, 1 << 20, n_i, n_j, None, 1.0, 50.0, 0.05, 10, 1e4,
+                                                 1.0, 0, 50, None, n_j, None, None, None, None, None)
+        assert rc != _native.WOTK_OK
+        return 'bytes of solver state' in lib.wotk_last_error().decode()
+
+    assert not refused(100000, 167360) and not refused(133120, 133120)
+    assert refused(100000, 167392) and refused(133152, 133152) and refused(16 << 20, 16 << 20)

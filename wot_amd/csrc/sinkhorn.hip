@@ -764,8 +764,12 @@ struct Work {
 
 constexpr int kEvoBlocks = 64;
 
-// extras: with the buffers of the resident solver or the one-read iteration where the shape takes them
-static size_t carve(Arena &ar, int64_t I, int64_t J, bool extras, Work *w) {
+// what a workspace is for: sweeps only (the no-allocation entry point), the duality-gap schedule over any
+// backend, or also the buffers of the resident solver or the one-read iteration where the shape takes them
+enum class Buffers { kSweeps, kSchedule, kRoutes };
+
+static size_t carve(Arena &ar, int64_t I, int64_t J, Buffers what, Work *w) {
+    const bool extras = what == Buffers::kRoutes;
     const int64_t I4 = round_up(I, 4), J4 = round_up(J, 4);
     w->f = ar.take<double>(I4);
     w->g = ar.take<double>(J4);
@@ -787,9 +791,9 @@ static size_t carve(Arena &ar, int64_t I, int64_t J, bool extras, Work *w) {
     w->us = ar.take<double>(I4);
     w->vs = ar.take<double>(J4);
     w->counter = ar.take<long long>(4);
-    w->slot = ar.take<unsigned long long>(4);
-    w->skip = ar.take<int>(4);
-    w->evo = ar.take<double>(4 * kEvoBlocks);
+    w->slot = reinterpret_cast<unsigned long long *>(w->misc + 8);  // misc: 0, 1 and 4 are others
+    w->skip = reinterpret_cast<int *>(w->misc + 12);
+    w->evo = what == Buffers::kSweeps ? nullptr : ar.take<double>(4 * kEvoBlocks);
     w->col_part = nullptr;
     if (extras && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
     w->gap_rows = w->gap_cols = w->gap_margins = nullptr;
@@ -948,11 +952,11 @@ using namespace wotk;
 extern "C" size_t wotk_solver_workspace_size(int64_t I, int64_t J) {
     Arena ar(nullptr, 0);
     Work w;
-    return carve(ar, I, J, true, &w);
+    return carve(ar, I, J, Buffers::kRoutes, &w);
 }
 
 static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
-                 const double *G, bool extras, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
+                 const double *G, Buffers what, void *workspace, size_t ws_bytes, Problem *pb, Work *w,
                  hipStream_t s) {
     WOTK_REQUIRE(I > 0 && J > 0 && I < (1ll << 31) && J < (1ll << 31), "bad shape %lld x %lld",
                  (long long)I, (long long)J);
@@ -960,7 +964,7 @@ static int setup(const float *C, int64_t ldc, const float *CT, int64_t ldct, int
     int rc = check_problem(*pb);
     if (rc) return rc;
     Arena ar(workspace, ws_bytes);
-    carve(ar, I, J, extras, w);
+    carve(ar, I, J, what, w);
     if (!workspace || !ar.ok) return fail(WOTK_EWORKSPACE, "solver workspace too small");
     return init_state(*pb, *w, s);
 }
@@ -1057,7 +1061,7 @@ extern "C" int wotk_solver_route(int64_t I, int64_t J, const void *workspace, si
     WOTK_REQUIRE(route && launches, "route and launches are required");
     Arena ar(const_cast<void *>(workspace), workspace_bytes);
     Work w;
-    carve(ar, I, J, true, &w);
+    carve(ar, I, J, Buffers::kRoutes, &w);
     if (!workspace || !ar.ok) return fail(WOTK_EWORKSPACE, "solver workspace too small");
     *launches = 0;
     *route = w.col_part ? WOTK_ROUTE_ONE_READ : WOTK_ROUTE_SWEEPS;
@@ -1081,7 +1085,7 @@ static int stablev2_call(const float *C, int64_t ldc, const float *CT, int64_t l
     const UnderWay here;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     rc = resident_or_not(pb, w, here, s);
     if (rc) return rc;
@@ -1135,7 +1139,7 @@ extern "C" int wotk_probe_stablev2_limits(const float *C, int64_t ldc, const flo
 // instead of a caller workspace.  Every call on a GPU shares that GPU's array
 // (calls that overlap on one GPU race); the solver initialises every part of
 // the state it reads, so the previous call's contents do not matter.
-constexpr size_t kScratchBytes = (size_t)16 << 20;  // 16 MiB: I, J up to ~95,000
+constexpr size_t kScratchBytes = (size_t)16 << 20;  // 16 MiB: I, J up to 133,120
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static void *g_scratch_ptr[kMaxDevices];  // device address of `scratch` on each GPU (host-side)
 static std::mutex g_scratch_mutex;
@@ -1170,7 +1174,7 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
                  (long long)J);
     Arena count(nullptr, 0);
     Work counted;
-    const size_t need = carve(count, I, J, false, &counted);
+    const size_t need = carve(count, I, J, Buffers::kSweeps, &counted);
     WOTK_REQUIRE(need <= kScratchBytes,
                  "%lld x %lld needs %zu bytes of solver state; the no-allocation entry point holds %zu "
                  "(use wotk_transport_stablev2 with a workspace)",
@@ -1182,7 +1186,7 @@ extern "C" int wotk_transport_stablev2_noalloc(const float *C, int64_t ldc, cons
     if (rc) return rc;
     Problem pb;
     Work w;
-    rc = setup(C, ldc, CT, ldct, I, J, G, false, ws, kScratchBytes, &pb, &w, s);
+    rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kSweeps, ws, kScratchBytes, &pb, &w, s);
     if (rc) return rc;
     (void)tau;
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
@@ -1433,7 +1437,7 @@ static int duality_gap_call(const float *C, int64_t ldc, const float *CT, int64_
     const UnderWay here;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     rc = resident_or_not(pb, w, here, s);
     if (rc) return rc;
@@ -1592,7 +1596,7 @@ struct FusedBackend {
 extern "C" size_t wotk_duality_gap_coords_workspace_size(int64_t I, int64_t J, int64_t d) {
     Arena ar(nullptr, 0);
     Work w;
-    return fused_problem_bytes(I, J, d) + 256 + carve(ar, I, J, false, &w);
+    return fused_problem_bytes(I, J, d) + 256 + carve(ar, I, J, Buffers::kSchedule, &w);
 }
 
 extern "C" int wotk_transport_duality_gap_coords(const double *X, const double *Y, int64_t I, int64_t J, int64_t d,
@@ -1611,7 +1615,7 @@ extern "C" int wotk_transport_duality_gap_coords(const double *X, const double *
     used = (used + 255) & ~size_t(255);
     Arena ar(static_cast<char *>(workspace) + used, workspace_bytes > used ? workspace_bytes - used : 0);
     Work w;
-    carve(ar, I, J, false, &w);
+    carve(ar, I, J, Buffers::kSchedule, &w);
     if (!ar.ok) return fail(WOTK_EWORKSPACE, "workspace too small");
     const Problem pb{nullptr, 0, nullptr, 0, (int)I, (int)J, G};
     rc = init_state(pb, w, s);
@@ -1640,7 +1644,7 @@ extern "C" int wotk_primal_dual(const float *C, int64_t ldc, const float *CT, in
     hipStream_t s = (hipStream_t)stream;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, true, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     WOTK_REQUIRE(out_host != nullptr, "out_host is required");
     copy2_kernel<<<64, 256, 0, s>>>(w.f, f, pb.n_i, w.g, g, pb.n_j);
