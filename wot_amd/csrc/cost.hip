@@ -186,21 +186,25 @@ static int median_run(const double *values, int64_t n, double *out, int64_t *ind
 }
 
 // ---------------------------------------------------------------------------
-// FP64 (I x J) -> FP32 C (I x J) and C^T (J x I), each entry value*scale.  Padding
+// FP64 (I x J) -> FP32 C (I x J) and C^T (J x I), each entry value / *divisor (the
+// median, on the device) or value * scale.  Padding
 // columns up to the next multiple of 4 are written as 0 so the float4 sweeps
 // read finite values there.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void normalise_transpose_kernel(
-    const double *__restrict__ C64, int64_t ld64, int n_i, int n_j, double scale, float *__restrict__ C, int64_t ldc, float *__restrict__ CT, int64_t ldct) {
+    const double *__restrict__ C64, int64_t ld64, int n_i, int n_j, const double *__restrict__ divisor, double scale,
+    float *__restrict__ C, int64_t ldc, float *__restrict__ CT, int64_t ldct) {
     __shared__ float tile[64][65];
     const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
+    const double dv = divisor ? *divisor : 0.0;
     const int pad_j = (n_j + 3) & ~3, pad_i = (n_i + 3) & ~3;
     for (int r = ty; r < 64; r += 4) {
         const int i = i0 + r, j = j0 + tx;
         float v = 0.f;
         if (i < n_i && j < n_j) {
-            v = (float)(C64[(int64_t)i * ld64 + j] * scale);
+            const double c = C64[(int64_t)i * ld64 + j];
+            v = (float)(divisor ? c / dv : c * scale);
         }
         tile[r][tx] = v;
         if (i < n_i && j < pad_j) C[(int64_t)i * ldc + j] = v;
@@ -212,10 +216,10 @@ __global__ __launch_bounds__(256) void normalise_transpose_kernel(
     }
 }
 
-static int launch_normalise_transpose(const double *C64, int64_t ld64, int64_t I, int64_t J, double scale, float *C,
-                                      int64_t ldc, float *CT, int64_t ldct, hipStream_t s) {
+static int launch_normalise_transpose(const double *C64, int64_t ld64, int64_t I, int64_t J, const double *divisor,
+                                      double scale, float *C, int64_t ldc, float *CT, int64_t ldct, hipStream_t s) {
     dim3 grid((unsigned)((round_up(J, 4) + 63) / 64), (unsigned)((round_up(I, 4) + 63) / 64));
-    normalise_transpose_kernel<<<grid, 256, 0, s>>>(C64, ld64, (int)I, (int)J, scale, C, ldc, CT, ldct);
+    normalise_transpose_kernel<<<grid, 256, 0, s>>>(C64, ld64, (int)I, (int)J, divisor, scale, C, ldc, CT, ldct);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
 }
@@ -253,10 +257,15 @@ extern "C" int wotk_median_f64(const double *values, int64_t n, double *median_o
     return median_run(values, n, median_out, median_index_out, st, h, (hipStream_t)stream);
 }
 
+static int mode_terms(int32_t mode) { return mode == WOTK_COST_BF16X3 ? 3 : mode == WOTK_COST_BF16X6 ? 6 : 0; }
+
 extern "C" size_t wotk_cost_workspace_size(int64_t I, int64_t J, int64_t d, int32_t mode) {
     Arena ar(nullptr, 0);
+    const int terms = mode_terms(mode);
     ar.take<char>(distance_median_bytes(I, J, false));
-    if (mode == WOTK_COST_BF16X3 || mode == WOTK_COST_BF16X6) ar.take<char>(cost_bf16_scratch(I, J, d));
+    if (distances_stored(DistanceProblem{nullptr, nullptr, (int)I, (int)J, (int)d, terms, 0, {}, {}}))
+        ar.take<double>((size_t)I * J);
+    if (terms) ar.take<char>(cost_bf16_scratch(I, J, d));
     return ar.off;
 }
 
@@ -278,17 +287,24 @@ extern "C" int wotk_cost_sqeuclid(const double *X, const double *Y, int64_t I, i
     hipStream_t s = (hipStream_t)stream;
     Arena ar(workspace, workspace_bytes);
     void *med_ws = ar.take<char>(distance_median_bytes(I, J, false));
+    DistanceProblem pb{X, Y, (int)I, (int)J, (int)d, mode_terms(mode), 0, {}, {}};
+    const bool stored = distances_stored(pb);
+    double *D = stored ? ar.take<double>((size_t)I * J) : nullptr;
     void *scratch = nullptr;
-    if (mode != WOTK_COST_F64) scratch = ar.take<char>(cost_bf16_scratch(I, J, d));
+    if (pb.terms) scratch = ar.take<char>(cost_bf16_scratch(I, J, d));
     if (!ar.ok || !workspace) return fail(WOTK_EWORKSPACE, "cost workspace too small");
-    DistanceProblem pb{X, Y, (int)I, (int)J, (int)d,
-                       mode == WOTK_COST_F64 ? 0 : mode == WOTK_COST_BF16X3 ? 3 : 6, 0, {}, {}};
     if (pb.terms) rc = prepare_split(&pb, scratch, s);
     if (rc) return rc;
+    if (stored) {
+        rc = launch_distances(pb, D, J, s);
+        if (rc) return rc;
+        pb.D = D;
+    }
     const double *median = nullptr;
     rc = distance_median(pb, false, med_ws, median_index_out, &median, s);
     if (rc) return rc;
-    rc = launch_cost_write(pb, median, C, ldc, CT, ldct, s);
+    rc = stored ? launch_normalise_transpose(D, J, I, J, median, 1.0, C, ldc, CT, ldct, s)
+                : launch_cost_write(pb, median, C, ldc, CT, ldct, s);
     if (rc) return rc;
     if (median_out) WOTK_HIP(hipMemcpyAsync(median_out, median, sizeof(double), hipMemcpyDeviceToDevice, s));
     return WOTK_OK;
@@ -299,5 +315,5 @@ extern "C" int wotk_cost_import(const double *C64, int64_t I, int64_t J, int64_t
     int rc = check_cost_layout(I, J, 1, C, ldc, CT, ldct);
     if (rc) return rc;
     WOTK_REQUIRE(ld64 >= J, "ld64 < J");
-    return launch_normalise_transpose(C64, ld64, I, J, scale, C, ldc, CT, ldct, (hipStream_t)stream);
+    return launch_normalise_transpose(C64, ld64, I, J, nullptr, scale, C, ldc, CT, ldct, (hipStream_t)stream);
 }

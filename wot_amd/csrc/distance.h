@@ -27,6 +27,7 @@ struct DistanceProblem {
     int terms;
     int kp;
     SplitCoords xs, ys;
+    const double *D = nullptr;  // stored (I x J, contiguous): read instead of formed
 };
 
 // split-BF16 preparation of pb (terms 3 or 6) into scratch (cost_mfma.hip)
@@ -46,7 +47,11 @@ int distance_median(const DistanceProblem &pb, bool lean, void *workspace, int64
 int launch_cost_write(const DistanceProblem &pb, const double *median, float *C, int64_t ldc, float *CT,
                       int64_t ldct, hipStream_t s);
 
-// the FP64 distances themselves (terms = 0 problems)
+// whether pb's distances are formed once and stored in FP64 for the median and the cost
+bool distances_stored(const DistanceProblem &pb);
+
+// the FP64 distances themselves to D (I x J, ld)
+int launch_distances(const DistanceProblem &pb, double *D, int64_t ld, hipStream_t s);
 int launch_sqeuclid_f64(const double *X, const double *Y, int64_t I, int64_t J, int64_t d, double *C64, int64_t ld,
                         hipStream_t s);
 

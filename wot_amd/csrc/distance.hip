@@ -42,15 +42,18 @@ typedef unsigned long long u64;
 // load in flight at once; the row pitch is twice an odd number, which puts the 16
 // rows a quarter wave reads on distinct banks.  (A transposing, 8-byte staging of the
 // same tile cost 0.2 ms per pass of 15000 x 15000.)
-struct F64Tile {
-    static constexpr int ROWS = 128, COLS = 64, NE = 32, WAVES = 3;
+// TR x TC entries per thread.  Where 8 x 4 leaves CUs without a tile, 4 x 2 (a fourth of the entries in a
+// third of the time; sums and bits the same).
+template <int TR, int TC>
+struct F64TileOf {
+    static constexpr int ROWS = 16 * TR, COLS = 16 * TC, NE = TR * TC, WAVES = 3;
     static constexpr int P = 34;  // row pitch and largest k chunk: 2 * 17
     static constexpr size_t LDS = sizeof(double) * (ROWS + COLS) * P;
     double v[NE];
     int i0, j0, tx, ty;
 
-    __device__ int row(int e) const { return i0 + ty + 16 * (e >> 2); }
-    __device__ int col(int e) const { return j0 + tx + 16 * (e & 3); }
+    __device__ int row(int e) const { return i0 + ty + 16 * (e / TC); }
+    __device__ int col(int e) const { return j0 + tx + 16 * (e % TC); }
 
     // coordinates [k0, k0 + km) of N points from p0, zeros past the last point and past an odd km;
     // B 16-byte pieces per thread in flight
@@ -88,19 +91,19 @@ struct F64Tile {
     }
 
     struct Operands {
-        double x[8], y[4];
+        double x[TR], y[TC];
         __device__ void load(const double *xk, const double *yk) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) x[q] = xk[q * 16 * P];
+            for (int q = 0; q < TR; ++q) x[q] = xk[q * 16 * P];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) y[q] = yk[q * 16 * P];
+            for (int q = 0; q < TC; ++q) y[q] = yk[q * 16 * P];
         }
     };
 
     __device__ void step(const Operands &o) {
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-            const double t = o.x[e >> 2] - o.y[e & 3];
+            const double t = o.x[e / TC] - o.y[e % TC];
             v[e] = fma(t, t, v[e]);
         }
     }
@@ -116,8 +119,8 @@ struct F64Tile {
         const int kc = ((pb.d + chunks - 1) / chunks + 1) & ~1;
         double *xs = reinterpret_cast<double *>(lds);
         double *ys = xs + ROWS * P;
-        stage<ROWS, 9>(pb.X, pb.n_i, i0, pb.d, 0, min(kc, pb.d), xs);
-        stage<COLS, 5>(pb.Y, pb.n_j, j0, pb.d, 0, min(kc, pb.d), ys);
+        stage<ROWS, (ROWS * P / 2 + 255) / 256>(pb.X, pb.n_i, i0, pb.d, 0, min(kc, pb.d), xs);
+        stage<COLS, (COLS * P / 2 + 255) / 256>(pb.Y, pb.n_j, j0, pb.d, 0, min(kc, pb.d), ys);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < NE; ++e) v[e] = 0.0;
@@ -140,6 +143,27 @@ struct F64Tile {
             stage<COLS, 3>(pb.Y, pb.n_j, j0, pb.d, k0, min(kc, pb.d - k0), ys);
             __syncthreads();
         }
+    }
+};
+using F64Tile = F64TileOf<8, 4>;
+using F64SmallTile = F64TileOf<4, 2>;
+
+// Distances that lie in memory, a wave's lanes along the columns.
+struct StoredTile {
+    static constexpr int ROWS = 128, COLS = 64, NE = 32, WAVES = 4;
+    static constexpr size_t LDS = 0;
+    double v[NE];
+    int i0, j0;
+
+    __device__ int row(int e) const { return i0 + ((int)threadIdx.x >> 6) * NE + e; }
+    __device__ int col(int) const { return j0 + ((int)threadIdx.x & 63); }
+
+    __device__ void compute(const DistanceProblem &pb, int ti, int tj, unsigned char *) {
+        i0 = ti * ROWS;
+        j0 = tj * COLS;
+        const double *p = pb.D + min(col(0), pb.n_j - 1);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) v[e] = p[(int64_t)min(row(e), pb.n_i - 1) * pb.n_j];
     }
 };
 
@@ -333,7 +357,8 @@ __device__ inline unsigned load_dev(const unsigned *p) {
 // sampled pairs: high words of their FP64 distances (the BF16 modes' distances
 // differ by about 1e-5 of the value, far inside the margin)
 __global__ __launch_bounds__(256) void dist_sample_kernel(const double *__restrict__ X, const double *__restrict__ Y,
-                                                          int n_i, int n_j, int d, unsigned *__restrict__ key32) {
+                                                          const double *__restrict__ D, int n_i, int n_j, int d,
+                                                          unsigned *__restrict__ key32) {
     const unsigned t = blockIdx.x * 256 + threadIdx.x;
     // two rounds of a 64-bit mixer (splitmix64's constants): independent row and column draws
     u64 z = (u64)(t + 1) * 0x9E3779B97F4A7C15ull;
@@ -343,9 +368,13 @@ __global__ __launch_bounds__(256) void dist_sample_kernel(const double *__restri
     const int64_t i = (int64_t)(((z & 0xffffffffull) * (u64)n_i) >> 32);
     const int64_t j = (int64_t)(((z >> 32) * (u64)n_j) >> 32);
     double acc = 0.0;
-    for (int k = 0; k < d; ++k) {
-        const double q = X[i * d + k] - Y[j * d + k];
-        acc = fma(q, q, acc);
+    if (D) {
+        acc = D[i * n_j + j];
+    } else {
+        for (int k = 0; k < d; ++k) {
+            const double q = X[i * d + k] - Y[j * d + k];
+            acc = fma(q, q, acc);
+        }
     }
     key32[t] = (unsigned)((u64)__double_as_longlong(acc) >> 32);
 }
@@ -886,7 +915,7 @@ static int median_passes(const DistanceProblem &pb, const MedianBuffers &b, int6
     const int odd = (int)(n % 2);
     u64 *idx = reinterpret_cast<u64 *>(index_out);
     if (b.n_samples)
-        dist_sample_kernel<<<b.n_samples / 256, 256, 0, s>>>(pb.X, pb.Y, pb.n_i, pb.n_j, pb.d, b.key32);
+        dist_sample_kernel<<<b.n_samples / 256, 256, 0, s>>>(pb.X, pb.Y, pb.D, pb.n_i, pb.n_j, pb.d, b.key32);
     if (b.n_samples == kSamplesLarge)
         dist_bracket_kernel<kSamplesLarge / 1024><<<1, 1024, 0, s>>>(b.key32, rank, (double)n, b);
     else if (b.n_samples == kSamplesSmall)
@@ -935,6 +964,7 @@ int distance_median(const DistanceProblem &pb, bool lean, void *workspace, int64
     MedianBuffers b;
     median_carve(ar, pb.n_i, pb.n_j, lean, &b);
     *median = &b.st->median;
+    if (pb.D) return median_passes<StoredTile>(pb, b, index_out, s);
     if (pb.terms == 0) return median_passes<F64Tile>(pb, b, index_out, s);
     if (pb.terms == 3) return median_passes<Bf16Tile<3>>(pb, b, index_out, s);
     return median_passes<Bf16Tile<6>>(pb, b, index_out, s);
@@ -1060,24 +1090,54 @@ int launch_cost_write(const DistanceProblem &pb, const double *median, float *C,
 }
 
 // the FP64 distances as they are
-__global__ __launch_bounds__(256, F64Tile::WAVES) void sqeuclid_f64_kernel(DistanceProblem pb, int tiles_j, double *__restrict__ D,
-                                                           int64_t ld) {
-    __shared__ __align__(16) unsigned char lds[F64Tile::LDS];
-    F64Tile t;
+template <class Tile>
+__global__ __launch_bounds__(256, Tile::WAVES) void dist_store_kernel(DistanceProblem pb, int tiles_j,
+                                                                      double *__restrict__ D, int64_t ld) {
+    __shared__ __align__(16) unsigned char lds[Tile::LDS ? Tile::LDS : 16];
+    Tile t;
     t.compute(pb, (int)(blockIdx.x / tiles_j), (int)(blockIdx.x % tiles_j), lds);
 #pragma unroll
-    for (int e = 0; e < F64Tile::NE; ++e)
+    for (int e = 0; e < Tile::NE; ++e)
         if (t.row(e) < pb.n_i && t.col(e) < pb.n_j) D[(int64_t)t.row(e) * ld + t.col(e)] = t.v[e];
+}
+
+template <class Tile>
+static int64_t tiles_of(const DistanceProblem &pb) {
+    return (((int64_t)pb.n_i + Tile::ROWS - 1) / Tile::ROWS) * (((int64_t)pb.n_j + Tile::COLS - 1) / Tile::COLS);
+}
+
+template <class Tile>
+static int launch_store(const DistanceProblem &pb, double *D, int64_t ld, hipStream_t s) {
+    const int64_t tiles = tiles_of<Tile>(pb);
+    WOTK_REQUIRE(tiles < (1ll << 31), "cost matrix too large");
+    dist_store_kernel<Tile><<<(unsigned)tiles, 256, 0, s>>>(pb, (pb.n_j + Tile::COLS - 1) / Tile::COLS, D, ld);
+    WOTK_LAUNCH_CHECK();
+    return WOTK_OK;
+}
+
+// one tile per CU at most: a fourth of the tile (us, 128 x 64 / 64 x 32: 300 x 303, d = 200 71 / 46; 1000 x
+// 1003, d = 30 31 / 28, d = 1000 288 / 179; at 512 tiles, 2000 x 2003, 38 / 39, 430 / 455)
+constexpr int64_t kSmallTiles = 256;
+
+int launch_distances(const DistanceProblem &pb, double *D, int64_t ld, hipStream_t s) {
+    if (pb.terms == 3) return launch_store<Bf16Tile<3>>(pb, D, ld, s);
+    if (pb.terms == 6) return launch_store<Bf16Tile<6>>(pb, D, ld, s);
+    if (tiles_of<F64Tile>(pb) <= kSmallTiles) return launch_store<F64SmallTile>(pb, D, ld, s);
+    return launch_store<F64Tile>(pb, D, ld, s);
 }
 
 int launch_sqeuclid_f64(const double *X, const double *Y, int64_t I, int64_t J, int64_t d, double *C64, int64_t ld,
                         hipStream_t s) {
-    const DistanceProblem pb{X, Y, (int)I, (int)J, (int)d, 0, 0, {}, {}};
-    const int64_t tj = (J + F64Tile::COLS - 1) / F64Tile::COLS, ti = (I + F64Tile::ROWS - 1) / F64Tile::ROWS;
-    WOTK_REQUIRE(ti * tj < (1ll << 31), "cost matrix too large");
-    sqeuclid_f64_kernel<<<(unsigned)(ti * tj), 256, 0, s>>>(pb, (int)tj, C64, ld);
-    WOTK_LAUNCH_CHECK();
-    return WOTK_OK;
+    return launch_distances(DistanceProblem{X, Y, (int)I, (int)J, (int)d, 0, 0, {}, {}}, C64, ld, s);
+}
+
+// Regenerated or stored once and read twice: 2 d operations per entry against 24 bytes (us for cost and
+// median, regenerated / stored).  FP64: d = 50 at 5000 x 5003 424 / 393, at 15000 x 15003 2475 / 2503; d = 64 482 /
+// 418 and 3060 / 2793; d = 200 1203 / 726 and 8018 / 5405.  Split bf16, whose products cost less: 1000 x 1003 d = 64
+// 234 / 223, 3000 x 3003 d = 100 415 / 375; 15000 x 15003 d = 160 2634 / 2974, d = 200 3294 / 3303, d = 300 4516 / 3920.
+bool distances_stored(const DistanceProblem &pb) {
+    const bool small = (int64_t)pb.n_i * pb.n_j <= 1 << 24;
+    return pb.d > (pb.terms == 0 || small ? 64 : 256);
 }
 
 }  // namespace wotk
