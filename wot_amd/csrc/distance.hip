@@ -250,7 +250,7 @@ struct Bf16Tile {
 // a tile's worth of slack in each would be most of the workspace
 constexpr int kSegments = 256;
 constexpr int kCandBins = 4096;
-constexpr int kListCap = 1 << 16;     // entries of the middle bins
+constexpr int kListCap = 1 << 18, kListMost = 1 << 20;  // entries of the middle bins, at least and at most
 constexpr int kRadixBins = 2048;
 // Pairs up to this many entries: every entry is a candidate, and one workgroup selects among all of
 // them (us for cost and median, so / with the bracket; normal, then integer coordinates: 120 x 127
@@ -286,7 +286,7 @@ struct MedianBuffers {
     u64 *fhist;               // fallback digit bins
     u64 *cand_key, *cand_idx;
     u64 *list_key, *list_idx;
-    unsigned seg_cap;
+    unsigned seg_cap, list_cap;
     int n_seg, seg_shift;     // 2^(32 - seg_shift) lists
     int n_samples;
     int lean;                 // no candidate lists: a counting pass and a gathering pass
@@ -310,8 +310,12 @@ static size_t median_carve(Arena &ar, int64_t I, int64_t J, bool lean, MedianBuf
     b->fhist = ar.take<u64>(kRadixBins);
     b->cand_key = ar.take<u64>((size_t)b->seg_cap * b->n_seg);
     b->cand_idx = ar.take<u64>((size_t)b->seg_cap * b->n_seg);
-    b->list_key = ar.take<u64>(kListCap);
-    b->list_idx = ar.take<u64>(kListCap);
+    // One distance in 64 may lie in the middle bins: tied ones (integer coordinates: about 1 % each)
+    // are then still selected from the list, one workgroup's work, instead of by eight more passes
+    // (split bf16, 8000 x 8003, d = 200: 1.7 ms against 4.3).  2.2 million took it 3.5 ms, the passes 1.9.
+    b->list_cap = (unsigned)std::max<int64_t>(kListCap, b->lean ? 0 : std::min<int64_t>(n / 64, kListMost));
+    b->list_key = ar.take<u64>(b->list_cap);
+    b->list_idx = ar.take<u64>(b->list_cap);
     return ar.off;
 }
 
@@ -549,7 +553,7 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
     for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
         Tile tile;
         tile.compute(pa.pb, (int)(t / pa.tiles_j), (int)(t % pa.tiles_j), lds);
-        if constexpr (MODE == kCollect) {
+        if constexpr (MODE == kCollect || MODE == kGather) {
             unsigned below = 0;
             u64 keep = 0;  // bit e: entry e is a candidate
 #pragma unroll
@@ -559,6 +563,7 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
                 below += in && k < lo;
                 keep |= (u64)(in && k >= lo && k <= hi) << e;
             }
+            if (MODE == kGather && !__syncthreads_or(keep != 0)) continue;  // most tiles hold none
             const unsigned mine = (unsigned)__popcll(keep);
             unsigned incl = mine;
 #pragma unroll
@@ -578,22 +583,29 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
             // (cells sorted by cluster) do not fill one segment
             const int seg = pa.b.n_seg == 1 ? 0 : (int)(((unsigned)t * 2654435761u) >> pa.b.seg_shift);
             if (tid == 0) {
-                wbase = atomicAdd(&pa.b.seg_count[seg * 64], wsum[0] + wsum[1] + wsum[2] + wsum[3]);
-                atomicAdd(&pa.b.seg_below[seg * 32], wbelow[0] + wbelow[1] + wbelow[2] + wbelow[3]);
+                const unsigned all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+                if (MODE == kCollect) {
+                    wbase = atomicAdd(&pa.b.seg_count[seg * 64], all);
+                    atomicAdd(&pa.b.seg_below[seg * 32], wbelow[0] + wbelow[1] + wbelow[2] + wbelow[3]);
+                } else if (all) {  // one add per tile: an add per entry took 11 ns, one after the other
+                    wbase = atomicAdd(&st->n_list, all);
+                }
             }
             __syncthreads();
             unsigned at = wbase + incl - mine;
             for (int w = 0; w < wave; ++w) at += wsum[w];
-            const int64_t seg0 = (int64_t)seg * pa.b.seg_cap;
             if (mine) {
-                u64 *ck = pa.b.cand_key + seg0, *ci = pa.b.cand_idx + seg0;
+                const int64_t seg0 = (int64_t)seg * pa.b.seg_cap;
+                const unsigned cap = MODE == kCollect ? pa.b.seg_cap : pa.b.list_cap;
+                u64 *ck = MODE == kCollect ? pa.b.cand_key + seg0 : pa.b.list_key;
+                u64 *ci = MODE == kCollect ? pa.b.cand_idx + seg0 : pa.b.list_idx;
 #pragma unroll
                 for (int g = 0; g < Tile::NE; g += 8) {
                     if (((keep >> g) & 255ull) == 0) continue;
 #pragma unroll
                     for (int e = g; e < g + 8; ++e) {
                         if ((keep >> e) & 1ull) {
-                            if (at < pa.b.seg_cap) {
+                            if (at < cap) {
                                 ck[at] = (u64)__double_as_longlong(tile.v[e]);
                                 ci[at] = (u64)tile.row(e) * (u64)pa.pb.n_j + (u64)tile.col(e);
                             }
@@ -611,14 +623,6 @@ __global__ __launch_bounds__(256, MODE == kBins || MODE == kDigit ? 2 : Tile::WA
                 if (MODE == kBins) {
                     below_all += k < lo;
                     if (k >= lo && k <= hi) count_bin((int)((k - lo) >> bin_shift));
-                } else if (MODE == kGather) {
-                    if (k >= lo && k <= hi) {
-                        const unsigned at = atomicAdd(&st->n_list, 1u);
-                        if (at < (unsigned)kListCap) {  // place_rank_kernel has seen to it
-                            pa.b.list_key[at] = k;
-                            pa.b.list_idx[at] = (u64)tile.row(e) * (u64)pa.pb.n_j + (u64)tile.col(e);
-                        }
-                    }
                 } else if (MODE == kDigit) {
                     if ((k & mask) == prefix) count_bin((int)((k >> pa.shift) & ((1ull << pa.width) - 1ull)));
                 } else if (MODE == kNextAbove) {
@@ -743,7 +747,7 @@ __global__ __launch_bounds__(1024) void place_rank_kernel(MedianBuffers b, int o
     __syncthreads();
     if (t == 0) {
         // heavy ties in the middle bins: no list holds them
-        if (over || bin[0] < 0 || bin[1] < 0 || end[1] - start[0] > (u64)kListCap) {
+        if (over || bin[0] < 0 || bin[1] < 0 || end[1] - start[0] > (u64)b.list_cap) {
             st->fallback = 1;
         } else {
             const u64 lo = st->lo;
@@ -773,6 +777,20 @@ __global__ __launch_bounds__(1024) void cand_hist_kernel(MedianBuffers b) {
         if (h[q]) atomicAdd(&b.hist[q], (u64)h[q]);
 }
 
+// f(e, keys[e]) for the thread's entries, eight loads in flight (one at a time, a list of 600000 tied
+// distances took 2 ms)
+template <class F>
+__device__ inline void each_key(const u64 *keys, unsigned n, F f) {
+    for (unsigned e0 = threadIdx.x; e0 < n; e0 += 8 * 1024) {
+        u64 x[8];
+#pragma unroll
+        for (unsigned u = 0; u < 8; ++u) x[u] = e0 + u * 1024 < n ? keys[e0 + u * 1024] : 0ull;
+#pragma unroll
+        for (unsigned u = 0; u < 8; ++u)
+            if (e0 + u * 1024 < n) f(e0 + u * 1024, x[u]);
+    }
+}
+
 // Exact order statistics of n (key, index) pairs, n >= 1, by one 1024-thread
 // workgroup: radix select on key - min, 11 bits a time, then the smallest key
 // above and the smallest indices.
@@ -790,10 +808,10 @@ __device__ void list_select(const u64 *keys, const u64 *idx, unsigned n, long lo
     }
     __syncthreads();
     u64 a = ~0ull, z = 0ull;
-    for (unsigned e = t; e < n; e += 1024) {
-        a = keys[e] < a ? keys[e] : a;
-        z = keys[e] > z ? keys[e] : z;
-    }
+    each_key(keys, n, [&](unsigned, u64 k) {
+        a = k < a ? k : a;
+        z = k > z ? k : z;
+    });
     for (int off = 32; off > 0; off >>= 1) {
         const u64 p = __shfl_xor(a, off), q = __shfl_xor(z, off);
         a = p < a ? p : a;
@@ -810,10 +828,9 @@ __device__ void list_select(const u64 *keys, const u64 *idx, unsigned n, long lo
     while (span) {  // uniform
         for (int q = t; q < kRadixBins; q += 1024) h[q] = 0u;
         __syncthreads();
-        for (unsigned e = t; e < n; e += 1024) {
-            const u64 x = keys[e] - base;
-            if (keys[e] >= base && x <= span) atomicAdd(&h[x >> shift], 1u);
-        }
+        each_key(keys, n, [&](unsigned, u64 k) {
+            if (k >= base && k - base <= span) atomicAdd(&h[(k - base) >> shift], 1u);
+        });
         __syncthreads();
         const unsigned c0 = h[2 * t], c1 = h[2 * t + 1];
         const unsigned before = block_scan(c0 + c1, red) - (c0 + c1);
@@ -837,8 +854,9 @@ __device__ void list_select(const u64 *keys, const u64 *idx, unsigned n, long lo
     // base is the lower middle key, held by eq entries, r of them before the rank
     u64 above = ~0ull;
     if (!odd && r + 1 >= eq) {
-        for (unsigned e = t; e < n; e += 1024)
-            if (keys[e] > base && keys[e] < above) above = keys[e];
+        each_key(keys, n, [&](unsigned, u64 k) {
+            if (k > base && k < above) above = k;
+        });
         for (int off = 32; off > 0; off >>= 1) {
             const u64 p = __shfl_xor(above, off);
             above = p < above ? p : above;
@@ -851,10 +869,10 @@ __device__ void list_select(const u64 *keys, const u64 *idx, unsigned n, long lo
     }
     if (index_out) {
         u64 i0 = ~0ull, i1 = ~0ull;
-        for (unsigned e = t; e < n; e += 1024) {
-            if (keys[e] == base && idx[e] < i0) i0 = idx[e];
-            if (keys[e] == above && idx[e] < i1) i1 = idx[e];
-        }
+        each_key(keys, n, [&](unsigned e, u64 k) {
+            if (k == base && idx[e] < i0) i0 = idx[e];
+            if (k == above && idx[e] < i1) i1 = idx[e];
+        });
         for (int off = 32; off > 0; off >>= 1) {
             const u64 p = __shfl_xor(i0, off), q = __shfl_xor(i1, off);
             i0 = p < i0 ? p : i0;
@@ -887,7 +905,7 @@ __global__ __launch_bounds__(1024) void cand_gather_kernel(MedianBuffers b) {
             const u64 k = b.cand_key[s0 + e];
             if (k >= lo && k <= hi) {
                 const unsigned at = atomicAdd(&st->n_list, 1u);
-                if (at < (unsigned)kListCap) {
+                if (at < b.list_cap) {
                     b.list_key[at] = k;
                     b.list_idx[at] = b.cand_idx[s0 + e];
                 }
