@@ -86,6 +86,12 @@ def test_gemm_tiles_exact(tm, m, k, n):
     assert bool((C[:, n:] == -7.0).all())
 
 
+# one chunk of K, one buffer: products of more than 256 small tiles
+@pytest.mark.parametrize('m,k,n', [(1100, 1, 1030), (1025, 16, 1999), (1100, 32, 1300), (1100, 33, 1300)])
+def test_gemm_one_chunk_exact(tm, m, k, n):
+    test_gemm_tiles_exact(tm, m, k, n)
+
+
 def test_gemm_nonfinite(tm):
     import torch
     A, B = torch.ones((70, 40), device='cuda'), torch.ones((40, 70), device='cuda')

@@ -57,14 +57,15 @@ __device__ inline bool gemm_tile(const GemmArgs &ga, int &tm, int &tn) {
 // MFMA 32x32x2 operand layout (lane l of a wave64): A element (row l%32, k l/32),
 // B element (k l/32, column l%32); accumulator register r holds row
 // 8*(r/4) + 4*(l/32) + r%4, column l%32.
-// TM: tile rows and columns; KS: groups of four waves that share the tile's K.
-template <int TM, int KS>
+// TM: tile rows and columns; KS: groups of four waves that share the tile's K; BUFS: 1 where K is one
+// chunk (half the LDS: twice the workgroups per CU).
+template <int TM, int KS, int BUFS>
 __global__ __launch_bounds__(256 * KS) void gemm_f32_mfma_kernel(GemmArgs ga) {
     constexpr int NB = TM / 64;          // 32-wide blocks per wave and side
     constexpr int AP = kGK + 4, BP = TM + 8;
     constexpr int BUF = TM * AP + kGK * BP;
     constexpr int U = TM * kGK / 1024;   // 16-byte pieces per thread and operand
-    __shared__ __align__(16) float lds[KS][2][BUF];
+    __shared__ __align__(16) float lds[KS][BUFS][BUF];
     int tm, tn;
     if (!gemm_tile(ga, tm, tn)) return;
     const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, ks = threadIdx.x >> 8;
@@ -130,11 +131,11 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_mfma_kernel(GemmArgs ga) {
     }
     __syncthreads();
     for (int i = 0; i < rounds; ++i) {
-        const bool more = i + 1 < (KS == 1 ? rounds : mine);
+        const bool more = BUFS > 1 && i + 1 < (KS == 1 ? rounds : mine);
         if (more) fetch(ks + (i + 1) * KS);
         if (KS == 1 || i < mine) {
-            const float *as = lds[ks][i & 1] + (wm + lr) * AP + 4 * lk;
-            const float *bs = lds[ks][i & 1] + TM * AP + 4 * lk * BP + wn + lr;
+            const float *as = lds[ks][i & (BUFS - 1)] + (wm + lr) * AP + 4 * lk;
+            const float *bs = lds[ks][i & (BUFS - 1)] + TM * AP + 4 * lk * BP + wn + lr;
 #pragma unroll
             for (int kk = 0; kk < kGK; kk += 8) {
                 f4 av[NB];
@@ -191,13 +192,13 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_mfma_kernel(GemmArgs ga) {
             }
 }
 
-template <int TM, int KS>
+template <int TM, int KS, int BUFS = 2>
 static int launch_gemm(GemmArgs ga, hipStream_t s) {
     ga.tiles_m = (ga.M + TM - 1) / TM;
     ga.tiles_n = (ga.N + TM - 1) / TM;
     const int64_t total = (int64_t)ga.tiles_m * ga.tiles_n;
     WOTK_REQUIRE(total < (1ll << 28), "GEMM output too large");
-    gemm_f32_mfma_kernel<TM, KS><<<(unsigned)(8 * ((total + 7) / 8)), 256 * KS, 0, s>>>(ga);
+    gemm_f32_mfma_kernel<TM, KS, BUFS><<<(unsigned)(8 * ((total + 7) / 8)), 256 * KS, 0, s>>>(ga);
     WOTK_LAUNCH_CHECK();
     return WOTK_OK;
 }
@@ -218,6 +219,9 @@ extern "C" int wotk_gemm_f32(const float *A, int64_t lda, const float *B, int64_
     // 128 x 128 tile's (97 against 130 TFLOP/s on full rounds).  Up to one round of 64 x 64
     // tiles, 16 waves on each instead of 4 (700 x 5000 x 700: 103 against 134 us).
     if (t64 <= 256) return launch_gemm<64, 4>(ga, s);
+    // one chunk of K: bound by the product's own bytes, small tiles in flight on them (us, 128 x 128 with
+    // two buffers / this: 5000 x 5000 x 16 52 / 46, 12000 x 12000 x 1 159 / 145)
+    if (K <= kGK) return launch_gemm<64, 1, 1>(ga, s);
     const double c128 = 4.0 * (double)((t128 + 255) / 256), c64 = 1.3 * (double)((t64 + 255) / 256);
     return c128 <= c64 ? launch_gemm<128, 1>(ga, s) : launch_gemm<64, 1>(ga, s);
 }
