@@ -319,6 +319,25 @@ def test_routes_of_several_threads():
     assert all(r in (_native.ROUTE_RESIDENT, _native.ROUTE_SWEEPS) for rs in routes for r in rs)
 
 
+@pytest.mark.parametrize('n_i,n_j', [(30, 20), (300, 400), (2049, 2047)])
+def test_few_iterations_take_the_sweeps(n_i, n_j):
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    x, y, g = _pair(n_i, n_j)
+    cost = ot.DeviceCost.from_coordinates(x, y)
+    ws = _workspace(n_i, n_j)
+    prm = dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, epsilon0=1.0, inner_iter_max=5)
+    for its, extra, route in ((1, 0, _native.ROUTE_SWEEPS), (10, 5, _native.ROUTE_SWEEPS),
+                              (10, 6, _native.ROUTE_RESIDENT)):
+        a = _run(_native.lib().wotk_transport_stablev2, cost, torch.from_numpy(g).cuda(),
+                 dict(prm, scaling_iter=its, extra_iter=extra), ws)
+        assert _route(ws, n_i, n_j) == (route, int(route == _native.ROUTE_RESIDENT))
+        b = _run(_native.lib().wotk_transport_stablev2_noalloc, cost, torch.from_numpy(g).cuda(),
+                 dict(prm, scaling_iter=its, extra_iter=extra))
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
 # ---- what follows when a bound is met: the same bits by another route ----
 def _fixed(fn, cost, g, ws, extra=()):
     import ctypes

@@ -983,9 +983,14 @@ static ResidentProblem resident_problem(const Problem &pb, const Work &w) {
                            w.exchange};
 }
 
-// w.exchange stays only where the solve takes the resident route; the route is left in the workspace
-static int resident_or_not(const Problem &pb, Work &w, const UnderWay &here, hipStream_t s) {
-    if (!w.exchange || here.alone()) return WOTK_OK;
+// A persistent launch is set up (30 us) before it gains: us for 1 / 11 / 20 iterations, launched and
+// resident, 120 x 150 80 / 147 / 223 and 111 / 150 / 196, 1500 x 1500 81 / 196 / 299 and 112 / 205 / 287.
+constexpr int64_t kResidentIters = 16;
+
+// w.exchange stays only where a solve of so many iterations takes the resident route; the route is
+// left in the workspace
+static int resident_or_not(const Problem &pb, Work &w, const UnderWay &here, int64_t iterations, hipStream_t s) {
+    if (!w.exchange || (here.alone() && iterations >= kResidentIters)) return WOTK_OK;
     const int rc = resident_pass_by(resident_problem(pb, w), s);
     w.exchange = nullptr;
     return rc;
@@ -1087,7 +1092,7 @@ static int stablev2_call(const float *C, int64_t ldc, const float *CT, int64_t l
     Work w;
     int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
-    rc = resident_or_not(pb, w, here, s);
+    rc = resident_or_not(pb, w, here, scaling_iter + extra_iter, s);
     if (rc) return rc;
     return stablev2_run(pb, w, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter, inner_iter_max, plan,
                         ldp, row_sums, f_out, g_out, true, lim, stats, s);
@@ -1439,7 +1444,7 @@ static int duality_gap_call(const float *C, int64_t ldc, const float *CT, int64_
     Work w;
     int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
-    rc = resident_or_not(pb, w, here, s);
+    rc = resident_or_not(pb, w, here, kResidentIters, s);
     if (rc) return rc;
     WOTK_REQUIRE(!plan || ldp >= J, "ldp < J");
     StoredBackend be{pb, w, plan, ldp, row_sums, f_out, g_out};
