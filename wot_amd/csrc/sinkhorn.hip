@@ -1325,16 +1325,18 @@ static int gap_schedule(B &be, const Problem &pb, Work &w, double lambda1, doubl
                 it += 5;
                 ++checks;
                 cur_queued = cur;
-                WOTK_HIP(hipEventRecord(side.snap, s));
-                WOTK_HIP(hipStreamWaitEvent(side.s, side.snap, 0));
                 const double *result = w.gapout + out;
+                hipStream_t reader = s;  // nothing runs ahead of the check: it is read in line
                 if (w.run_ahead && it + 5 < max_iter) {
+                    reader = side.s;
+                    WOTK_HIP(hipEventRecord(side.snap, s));
+                    WOTK_HIP(hipStreamWaitEvent(side.s, side.snap, 0));
                     rc = batch();
                     if (rc) return rc;
                     queued = true;
                 }
-                WOTK_HIP(hipMemcpyAsync(host_out, result, sizeof(double), hipMemcpyDeviceToHost, side.s));
-                WOTK_HIP(hipStreamSynchronize(side.s));
+                WOTK_HIP(hipMemcpyAsync(host_out, result, sizeof(double), hipMemcpyDeviceToHost, reader));
+                WOTK_HIP(hipStreamSynchronize(reader));
                 gap = host_out[0];
             }
             if (queued) cur = cur_queued;  // the batch ahead did nothing
