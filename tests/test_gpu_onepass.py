@@ -209,3 +209,36 @@ def test_small_penalties(lam1, lam2):
         assert torch.isfinite(a).all()
         # exponents up to max |C| / eps rounded at 2^-24, times eps, over 340 half-iterations
         assert float((a - b).abs().max()) < 340 * 2.0 ** -24 * float(cost.dense().max())
+
+
+# the one-read gap pass: pairs with a short side, and from 2^24 entries on, in whole and ragged tiles
+@pytest.mark.parametrize('n_i,n_j,kw', [(1500, 6001, {}), (6017, 1500, dict(tau=2.0)), (4200, 4100, {}),
+                                        (5003, 3401, dict(batch_size=3))])
+def test_one_read_gap_pass_matches_fp64(n_i, n_j, kw):
+    test_duality_gap_schedule_matches_fp64(n_i, n_j, kw)
+
+
+def test_objectives_on_either_side_of_the_gap_pass_rule():
+    """2900 x 2900 takes two passes, 4200 x 4100 and 1500 x 6001 one: both against FP64."""
+    import torch
+    import wot_amd.ot as ot
+    from wot_amd.ot import device as dev
+    from wot_amd.synthetic import day_pair
+    for n_i, n_j in ((2900, 2900), (4200, 4100), (1500, 6001)):
+        dp = day_pair(n_i, n_j, dim=30, n_components=5, seed=n_j)
+        cost = ot.DeviceCost.from_coordinates(dp.x, dp.y)
+        G = torch.from_numpy(dp.growth).cuda()
+        r = dev.solve(cost, G, 'fixed_iters', dict(lambda1=1.0, lambda2=50.0, epsilon=0.05, scaling_iter=60, tau=1e4,
+                                                   epsilon0=1.0, extra_iter=0, inner_iter_max=20),
+                      want_potentials=True)
+        pri, dua = dev.primal_dual(cost, G, r['f'], r['g'], 1.0, 50.0, 0.05)
+        C, f, g = cost.dense().double(), r['f'], r['g']
+        y = (f[:, None] + g[None, :] - C) / 0.05
+        R, K = torch.exp(y), torch.exp(-C / 0.05)
+        q, n, m = G.mean(), n_i, n_j
+        x1, x2 = R.sum(1) / m, R.sum(0) / n
+        want_p = float((x1 * torch.log(x1 / G) - x1 + G).sum() / n + 50.0 * (x2 * torch.log(x2 / q) - x2 + q).sum() / m
+                       + (0.05 * ((R * y).sum() - R.sum() + K.sum()) + (R * C).sum()) / (n * m))
+        want_d = float(-(G * (torch.exp(-f) - 1)).sum() / n - 50.0 * (q * (torch.exp(-g / 50.0) - 1)).sum() / m
+                       - 0.05 * (R.sum() - K.sum()) / (n * m))
+        assert pri == pytest.approx(want_p, rel=1e-10) and dua == pytest.approx(want_d, rel=1e-10)

@@ -759,10 +759,18 @@ struct Work {
     int *skip;                 // set when a batch that runs ahead must not run
     bool run_ahead = false;    // the iteration's launches look at *skip
     double *evo;               // partial sums of the evolution check
-    double *gap_rows, *gap_cols, *gap_margins;  // one-read gap pass: partials per tile (with col_part)
+    double *gap_rows, *gap_cols, *gap_margins;  // one-read gap pass: partials per tile, or nullptr: two passes
 };
 
 constexpr int kEvoBlocks = 64;
+
+// Below 2^24 entries C and C^T come from the Infinity Cache, and two passes with their rows over all
+// CUs take less than one read (us for the objectives alone, two passes / one read: 2900 x 2900 143 / 171,
+// 3500 x 3500 170 / 188, 4300 x 4200 218 / 207; duality-gap solves 11850 / 12600, 13790 / 14590, 16170 / 15990);
+// with one short side one of the two has few rows (20000 x 600 243 / 212, 16520 / 15960).
+static bool one_read_gap(int64_t I, int64_t J) {
+    return one_pass_fits(I, J) && (I * J >= 1ll << 24 || std::min(I, J) < 2048);
+}
 
 // what a workspace is for: sweeps only (the no-allocation entry point), the duality-gap schedule over any
 // backend, or also the buffers of the resident solver or the one-read iteration where the shape takes them
@@ -797,7 +805,7 @@ static size_t carve(Arena &ar, int64_t I, int64_t J, Buffers what, Work *w) {
     w->col_part = nullptr;
     if (extras && one_pass_fits(I, J)) w->col_part = ar.take<float>(one_pass_partials(I, J));
     w->gap_rows = w->gap_cols = w->gap_margins = nullptr;
-    if (w->col_part || (!ar.base && extras && one_pass_fits(I, J))) {
+    if (extras && one_read_gap(I, J)) {
         const int64_t ti = (I + kGapRows - 1) / kGapRows, tj = (J + kGapCols - 1) / kGapCols;
         w->gap_rows = ar.take<double>((size_t)tj * I);
         w->gap_cols = ar.take<double>((size_t)ti * J);
