@@ -59,22 +59,42 @@ __device__ __forceinline__ double exp2_f64(double x) {
     return ldexp(p, (int)n);
 }
 
-// sums over a wave by DPP, no LDS permutes: row_shr 1, 2, 4, 8, then row_bcast 15 (lanes 31 and
-// 63 hold the sums of their 32 lanes), then row_bcast 31 (lane 63 holds the sum of all)
+// sums over a wave by DPP, no LDS permutes: row_shr 1, 2, 4, 8 (the last lane of each 16 holds
+// their sum), then row_bcast 15 (lanes 31 and 63 hold the sums of their 32 lanes), then row_bcast 31
+// (lane 63 holds the sum of all)
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp_add(double v) {
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
     return v + __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double half_wave_sum_dpp(double v) {
+__device__ __forceinline__ double row_sum_dpp(double v) {
     v = dpp_add<0x111, 0xf>(v);
     v = dpp_add<0x112, 0xf>(v);
     v = dpp_add<0x114, 0xf>(v);
-    v = dpp_add<0x118, 0xf>(v);
-    return dpp_add<0x142, 0xa>(v);
+    return dpp_add<0x118, 0xf>(v);
 }
+__device__ __forceinline__ double half_wave_sum_dpp(double v) { return dpp_add<0x142, 0xa>(row_sum_dpp(v)); }
 __device__ __forceinline__ double wave_sum_dpp(double v) { return dpp_add<0x143, 0xc>(half_wave_sum_dpp(v)); }
+
+// sum and maximum over a wave in every lane
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
+    return v;
+}
+
+// two partial sums sum_k 2^(y_k - sg) put together
+__device__ __forceinline__ void lse_merge(double &sg, double &sd, double og, double os) {
+    const double ng = fmax(sg, og);
+    sd = ldexp(sd, (int)(sg - ng)) + ldexp(os, (int)(og - ng));
+    sg = ng;
+}
 #endif
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }

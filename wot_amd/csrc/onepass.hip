@@ -74,46 +74,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// v + v moved by a DPP control; lanes without a source add 0
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
-    return v + __hiloint2double(hi, lo);
-}
-
-// sums over 16-lane rows, in the last lane of each row
-__device__ __forceinline__ double row_sum16(double v) {
-    v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
-    v = dpp_add<0x112, 0xf>(v);
-    v = dpp_add<0x114, 0xf>(v);
-    return dpp_add<0x118, 0xf>(v);
-}
-
-// sum over the wave, in lane 63 (no LDS permutes: their latency would stand in every step)
-__device__ __forceinline__ double wave_sum_last(double v) {
-    v = row_sum16(v);
-    v = dpp_add<0x142, 0xa>(v);         // row_bcast 15
-    return dpp_add<0x143, 0xc>(v);      // row_bcast 31
-}
-
-__device__ __forceinline__ double read_lane(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-
-__device__ __forceinline__ double wave_sum64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
-__device__ __forceinline__ double wave_max64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
-    return v;
-}
-
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -222,7 +182,7 @@ struct RowPass {
         load_f(it + 1);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const double t = wave_sum_last(s[r]);
+            const double t = wave_sum_dpp(s[r]);
             if (lane == 63) sh.wsum[it & 1][r][wave] = t;
         }
     }
@@ -313,7 +273,7 @@ __device__ void finish_rows(const RowArgs &ra, RowShared<R> &sh, int n) {
         const int rw = mine ? row : 0;
         const double fo = ra.f[rw], lp = ra.logp[rw];
         lds_barrier();
-        const double S = row_sum16(sh.wsum[it & 1][r][lane & 15]);  // in the last lane of each 16
+        const double S = row_sum_dpp(sh.wsum[it & 1][r][lane & 15]);  // in the last lane of each 16
         const int N = shift_of(ra.k * fo);
         const double lse2 = log2(S) + (double)N;
         const double fn = ra.alpha * ra.eps * (lp + ra.log_nj - lse2 * kLn2);
@@ -348,7 +308,7 @@ __device__ void redo_bad(const RowArgs &ra, RowShared<R> &sh, const double2 *h, 
         double m = -1.0e300;
         for (int c = 0; c < chunks; ++c)
             for (int q = 0; q < 4; ++q) m = fmax(m, exponent(c, q));
-        m = wave_max64(m);
+        m = wave_max(m);
         __syncthreads();
         if (lane == 0) sh.red[wave] = m;
         __syncthreads();
@@ -357,7 +317,7 @@ __device__ void redo_bad(const RowArgs &ra, RowShared<R> &sh, const double2 *h, 
         double s = 0.0;
         for (int c = 0; c < chunks; ++c)
             for (int q = 0; q < 4; ++q) s += (double)__builtin_amdgcn_exp2f((float)(exponent(c, q) - top));
-        s = wave_sum64(s);
+        s = wave_sum(s);
         __syncthreads();
         if (lane == 0) sh.red[wave] = s;
         __syncthreads();
@@ -469,7 +429,7 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
         const float *row = ca.CT + (int64_t)col * ca.ldct;
         double m = -1.0e300;
         for (int i = threadIdx.x; i < ca.n_i; i += kT) m = fmax(m, (ca.f[i] - (double)row[i]) * ca.k);
-        m = wave_max64(m);
+        m = wave_max(m);
         if (c == 0) wred[p] = m;
         __syncthreads();
         for (int w = 0; w < kW; ++w) m = fmax(m, wred[w]);
@@ -478,7 +438,7 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
         double t = 0.0;
         for (int i = threadIdx.x; i < ca.n_i; i += kT)
             t += (double)__builtin_amdgcn_exp2f((float)((ca.f[i] - (double)row[i]) * ca.k - sh));
-        t = wave_sum64(t);
+        t = wave_sum(t);
         if (c == 0) wred[p] = t;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -493,7 +453,7 @@ __global__ __launch_bounds__(kT) void one_pass_cols_kernel(ColArgs ca) {
         if (p == 0 && j < ca.n_j) m = (ca.g[j] - ca.tau.v[j]) * ca.tau.inv_eps;
         for (int i = blockIdx.x * kT + threadIdx.x; i < ca.n_i; i += (int)gridDim.x * kT)
             m = fmax(m, (ca.f[i] - ca.tau.u[i]) * ca.tau.inv_eps);
-        m = wave_max64(m);
+        m = wave_max(m);
         __syncthreads();
         if (c == 0) wred[p] = m;
         __syncthreads();
@@ -539,11 +499,12 @@ int launch_rows(const RowArgs &ra, int grid, hipStream_t s) {
 }  // namespace
 
 // Where one read of C beats two sweeps over C and C^T (us per iteration, two sweeps against one
-// read): 2900 x 2900 19.2 / 17.9, 9000 x 1001 24.8 / 22.6, 600 x 19000 42.4 / 30.5, 6000 x 5000
-// 43.7 / 33.1, 10000 x 8001 105 / 64.9, 15000 x 15000 275 / 154, 19000 x 19000 (the widest rows whose
-// sums fit in registers) 439 / 236.  Pairs under 2^23 entries go to the resident solver instead
-// (14.4 us at 2749 x 3001); the ones of them that it does not take keep the two sweeps, whose FP32
-// sums their FP64 maps are held to.
+// read): 2900 x 2900 19.2 / 17.7, 9000 x 1001 24.8 / 22.6, 600 x 19000 42.4 / 30.5, 6000 x 5000
+// 43.7 / 33.1, 10000 x 8001 105 / 65.5, 15000 x 15000 275 / 155, 19000 x 19000 (the widest rows whose
+// sums fit in registers) 439 / 236.  The line at 2^23 entries is not a crossing of times: it is
+// where results change.  Up to it a pair's potentials have the two sweeps' bits, by the resident
+// solver or, with a side it does not take, by the sweeps themselves (9000 x 800: 24.9); above it
+// columns are summed in FP64.
 bool one_pass_fits(int64_t I, int64_t J) {
     if (chunks_of(J) > kMaxChunks || I > (int64_t)kCus * kMaxRows) return false;
     return I * J >= (1ll << 23);

@@ -134,19 +134,6 @@ __device__ __forceinline__ int xor_max(int v) {
     return max(v, dpp_mov<0x121>(v));
 }
 
-__device__ __forceinline__ double wave_max64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
-    return v;
-}
-
-// two partial sums sum_k 2^(y_k - sg), merged as the sweep merges them
-__device__ __forceinline__ void lse_merge(double &sg, double &sd, double og, double os) {
-    const double ng = fmax(sg, og);
-    sd = ldexp(sd, (int)(sg - ng)) + ldexp(os, (int)(og - ng));
-    sg = ng;
-}
-
 struct Shared {
     double2 red[kMaxOwn][4];      // per owned row and wave: (shift, sum); or row sums
     double wsum[16][kSums];       // per wave, for the checks
@@ -336,7 +323,7 @@ struct Solver {
             if (row_f >= 0) grown = fmax(grown, (sh.f[tid] - sh.u[tid]) * inv_eps);
             const int q = pt == 2 ? 0 : pt + 1, after = q == 2 ? 0 : q + 1;
             if (tid < 64) {
-                grown = wave_max64(grown);
+                grown = wave_max(grown);
                 if (tid == 0) {
                     // the next iteration's buffer held the maxima before the last ones
                     store_x(a.flags + (int64_t)after * kMaxWg + wg, kEmpty);
@@ -359,7 +346,7 @@ struct Solver {
             u64 x = load_x(a.flags + (int64_t)pt * kMaxWg + tid);
             if (wait_value(a.flags + (int64_t)pt * kMaxWg + tid, x)) m = unpack(x);
         }
-        m = wave_max64(m);
+        m = wave_max(m);
         if (lane == 0) sh.wsum[tid >> 6][0] = m;
         if (!sync_ok()) return false;
         m = sh.wsum[0][0];
@@ -748,9 +735,11 @@ int clear(const ResidentProblem &rp, hipStream_t s) {
 }  // namespace
 
 // Where the resident solver beats launched sweeps: everywhere its registers hold the pair (us per
-// iteration, launched / resident): 50 x 60 8.0 / 4.5, 300 x 400 8.3 / 5.2, 1000 x 1000 8.9 / 6.2,
-// 2000 x 2500 15.8 / 10.9, 2890 x 2890 19.8 / 14.5, 900 x 8000 23.1 / 15.4.  From 2^23 entries on
-// the one-read iteration is the other side: 17.9 us at 2900 x 2900.
+// iteration, launched / resident): 50 x 60 8.0 / 4.4, 300 x 400 8.3 / 4.9, 1000 x 1000 8.9 / 6.0,
+// 2000 x 2500 15.8 / 11.0, 2890 x 2890 19.8 / 14.5, 900 x 8000 23.1 / 15.8; solves of a few iterations
+// aside (sinkhorn.hip).  Nine pieces a thread would reach 3072 x 3072, where the one-read iteration
+// takes 18; the line stands at 2^23 entries, from which on results come from that one's FP64 column
+// sums.
 bool resident_fits(int64_t I, int64_t J) {
     if (I > kMaxSide || J > kMaxSide || I * J > (1ll << 23)) return false;
     const Shape s = shape_of(I, J);

@@ -48,27 +48,6 @@ __device__ __forceinline__ float4 load_stream4(const float *p) {
 }
 
 // ---------------------------------------------------------------------------
-// block reductions (256 threads = 4 wave64)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void lse_merge(double &sg, double &sd, double og, double os) {
-    const double ng = fmax(sg, og);
-    sd = ldexp(sd, (int)(sg - ng)) + ldexp(os, (int)(og - ng));
-    sg = ng;
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
-    return v;
-}
-
-// ---------------------------------------------------------------------------
 // Row log-sum-exp sweep with the potential update fused in the epilogue.
 //   lse_i = ln sum_j exp((h_j - A_ij)/eps)            (natural log)
 //   pot_i = alpha * eps * (logw_i + log_n_other - lse_i)

@@ -27,7 +27,7 @@ namespace wotk {
 namespace {
 
 constexpr int kPopTile = 16;          // populations per MFMA tile
-constexpr int kWaves = 4;             // waves per workgroup (no LDS, no barriers)
+constexpr int kWaves = 4;             // waves per workgroup (LDS for the push's sums over them and the totals only)
 // Waves of a product: two per SIMD, all resident at once.  Splits are rounded down, so that no
 // second round of a few waves follows (seven maps of 3900 to 12001 cells, 10 populations: 596 us;
 // 607 at three per SIMD, 669 at one and a half; 684 at three and 708 at four rounded up)
