@@ -153,7 +153,8 @@ struct Solver {
     f4 c[S], ct[S];               // this thread's pieces of its team's C and C^T rows
     // owner threads (tid < kMaxOwn): the workgroup's rows tid
     int row_f, row_g;             // or -1
-    bool has_f, has_g;            // whether the workgroup owns rows of C / of C^T
+    // potentials that the workgroup reads: all, or none where it owns no row of C (need_g) or of C^T
+    int need_f, need_g;
     int pf;                       // parity of the last published f and g
     int pt;                       // buffer of the last published maxima
     int pc;                       // buffer of the last published sums
@@ -279,45 +280,39 @@ struct Solver {
         const double k = kLog2E / eps, inv_eps = 1.0 / eps;
         const double al1 = a.lambda1 / (a.lambda1 + eps), al2 = a.lambda2 / (a.lambda2 + eps);
         const int n_i = a.rp.n_i, n_j = a.rp.n_j;
-        if (has_f) {
-            if (first) {
-                for (int j = tid; j < n_j; j += kT) hg[place(j)] = a.rp.g[j] * k;
-            } else {
-                take(a.gx + (int64_t)pf * n_j, n_j, hg, k);
-            }
+        if (first) {
+            for (int j = tid; j < n_j; j += kT) hg[place(j)] = a.rp.g[j] * k;
+        } else {
+            take(a.gx + (int64_t)pf * n_j, need_g, hg, k);
         }
         if (!sync_ok()) return false;
         if (checks && flag_open && !absorb()) return false;
         const int p = pf ^ 1;  // this iteration's buffers; the other ones hold what their readers have read
-        if (has_f) {
-            if (row_f >= 0 && !first) store_x(a.fx + (int64_t)pf * n_i + row_f, kEmpty);
-            sweep(c, a.rf, a.cf, hg, k);
-            __syncthreads();
-            if (row_f >= 0) {
-                sh.fp[tid] = sh.f[tid];
-                sh.up[tid] = sh.u[tid];
-                const double f = potential(sh.lw[tid], a.log_nj, al1, eps);
-                sh.f[tid] = f;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied buffer first
-                store_x(a.fx + (int64_t)p * n_i + row_f, pack(f));
-            }
+        if (row_f >= 0 && !first) store_x(a.fx + (int64_t)pf * n_i + row_f, kEmpty);
+        sweep(c, a.rf, a.cf, hg, k);
+        __syncthreads();
+        if (row_f >= 0) {
+            sh.fp[tid] = sh.f[tid];
+            sh.up[tid] = sh.u[tid];
+            const double f = potential(sh.lw[tid], a.log_nj, al1, eps);
+            sh.f[tid] = f;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied buffer first
+            store_x(a.fx + (int64_t)p * n_i + row_f, pack(f));
         }
-        if (has_g) take(a.fx + (int64_t)p * n_i, n_i, hf, k);
+        take(a.fx + (int64_t)p * n_i, need_f, hf, k);
         if (!sync_ok()) return false;
+        if (row_g >= 0 && !first) store_x(a.gx + (int64_t)pf * n_j + row_g, kEmpty);
+        sweep(ct, a.rg, a.cg, hf, k);
+        __syncthreads();
         double grown = -INFINITY;
-        if (has_g) {
-            if (row_g >= 0 && !first) store_x(a.gx + (int64_t)pf * n_j + row_g, kEmpty);
-            sweep(ct, a.rg, a.cg, hf, k);
-            __syncthreads();
-            if (row_g >= 0) {
-                sh.gp[tid] = sh.g[tid];
-                sh.vp[tid] = sh.v[tid];
-                const double g = potential(a.rp.misc[0], a.log_ni, al2, eps);
-                sh.g[tid] = g;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                store_x(a.gx + (int64_t)p * n_j + row_g, pack(g));
-                grown = (g - sh.v[tid]) * inv_eps;
-            }
+        if (row_g >= 0) {
+            sh.gp[tid] = sh.g[tid];
+            sh.vp[tid] = sh.v[tid];
+            const double g = potential(a.rp.misc[0], a.log_ni, al2, eps);
+            sh.g[tid] = g;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            store_x(a.gx + (int64_t)p * n_j + row_g, pack(g));
+            grown = (g - sh.v[tid]) * inv_eps;
         }
         if (checks) {
             if (row_f >= 0) grown = fmax(grown, (sh.f[tid] - sh.u[tid]) * inv_eps);
@@ -593,8 +588,8 @@ __global__ __launch_bounds__(kT) void resident_kernel(Args a, Segments seg) {
             if (so.row_g >= 0) sh.v[tid] = a.rp.v[so.row_g];
         }
     }
-    so.has_f = wg * kTeams < n_i;
-    so.has_g = wg * kTeams < n_j;
+    so.need_g = wg * kTeams < n_i ? n_j : 0;
+    so.need_f = wg * kTeams < n_j ? n_i : 0;
     so.pf = 1;
     so.pt = 2;
     so.pc = 2;
