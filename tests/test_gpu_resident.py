@@ -294,21 +294,24 @@ def test_route_beside_another_solve():
 
 
 def test_routes_of_several_threads():
-    """Wide and tall pairs from four threads: resident or by sweeps, never given up."""
+    """Wide and tall pairs from four threads, by whichever route: the same bits, and resident attempts are
+    not given up as a rule (one may be, where others' sweeps keep its CUs for 0.1 s)."""
     import threading
     import torch
     import wot_amd.ot as ot
     from wot_amd import _native
     shapes = [(300, 400), (1000, 260), (2000, 2500), (30, 20)]
     costs = [ot.DeviceCost.from_coordinates(*_pair(i, j, 2)[:2]) for i, j in shapes]
+    refs = [_gap(c, _pair(*s, 2)[2], _workspace(*s))[:2] for c, s in zip(costs, shapes)]
     torch.cuda.synchronize()
-    routes = [[] for _ in shapes]
+    routes, same = [[] for _ in shapes], [True] * len(shapes)
 
     def work(k):
         with torch.cuda.stream(torch.cuda.Stream()):
             ws = _workspace(*shapes[k])
             for _ in range(4):
-                _gap(costs[k], _pair(*shapes[k], 2)[2], ws)
+                f, h, _ = _gap(costs[k], _pair(*shapes[k], 2)[2], ws)
+                same[k] = same[k] and torch.equal(f, refs[k][0]) and torch.equal(h, refs[k][1])
                 routes[k].append(_route(ws, *shapes[k])[0])
 
     ts = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
@@ -316,7 +319,8 @@ def test_routes_of_several_threads():
         t.start()
     for t in ts:
         t.join()
-    assert all(r in (_native.ROUTE_RESIDENT, _native.ROUTE_SWEEPS) for rs in routes for r in rs)
+    assert all(same)
+    assert sum(r == _native.ROUTE_GAVE_UP for rs in routes for r in rs) <= 2
 
 
 @pytest.mark.parametrize('n_i,n_j', [(30, 20), (300, 400), (2049, 2047)])
