@@ -1218,12 +1218,12 @@ def bench_validation(args):
 
 def bench_sweeps(args):
     """Short, fixed workload for counter and trace runs of the stored-cost
-    solver: the 15,000 x 15,000 pair's cost (``--cost-reps`` extra builds in
-    each cost mode first), ``--iters`` fixed-iteration Sinkhorn iterations (2
-    row log-sum-exp sweeps each, one over C and one over C^T, 4*n*n algorithmic
-    bytes per sweep) with the given ``--tile``, then one plain device copy of
-    n*n float32 (n*n*4 bytes read and written) that calibrates the FETCH_SIZE
-    and WRITE_SIZE counters."""
+    solver's launched sweeps: the 15,000 x 15,000 pair's cost (``--cost-reps``
+    extra builds in each cost mode first), ``--iters`` fixed-iteration Sinkhorn
+    iterations (2 row log-sum-exp sweeps each, one over C and one over C^T,
+    4*n*n algorithmic bytes per sweep) with the given ``--tile``, then one plain
+    device copy of n*n float32 (n*n*4 bytes read and written) that calibrates the
+    FETCH_SIZE and WRITE_SIZE counters."""
     import torch
     import wot_amd.ot as ot
     from wot_amd.synthetic import day_pair
@@ -1238,16 +1238,14 @@ def bench_sweeps(args):
         for mode in ('f64', 'bf16x3', 'bf16x6'):
             ot.DeviceCost.from_coordinates(dp.x, dp.y, mode=mode)
     cost = ot.DeviceCost.from_coordinates(dp.x, dp.y)
-    st = {}
-    ot.transport_stablev2(cost, G=dp.growth, lambda1=1.0, lambda2=50.0, epsilon=0.05, scaling_iter=iters, tau=1e4,
-                          epsilon0=1.0, extra_iter=0, inner_iter_max=50, device_out=True, stats=st)
+    sweep_us = tune.row_sweep_us(cost, dp.growth, epsilon0=1.0, iters=iters)
     src = torch.empty((n, n), dtype=torch.float32, device='cuda').fill_(1.0)
     dst = torch.empty_like(src)
     torch.cuda.synchronize()
     dst.copy_(src)
     torch.cuda.synchronize()
     return {'workload': 'row sweeps of one %d x %d pair' % (n, n), 'iterations': iters, 'tile': args.tile,
-            'avg_sweep_us': 1000.0 * st['sweep_ms'] / max(st['sweeps'], 1), 'copy_bytes': src.numel() * 4}
+            'avg_sweep_us': sweep_us, 'copy_bytes': src.numel() * 4}
 
 
 def main():

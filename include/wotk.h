@@ -159,7 +159,7 @@ int wotk_transport_duality_gap(const float *C, int64_t ldc, const float *CT, int
  * I x J pair on `workspace` ran (no counterpart in the reference): *route
  * (HOST) is one of WOTK_ROUTE_*; *launches (HOST) the persistent launches of
  * the resident solver.  The routes differ in time, and the resident one has
- * the sweeps' bits.  Waits for the stream. */
+ * the sweeps' bits at their default tile.  Waits for the stream. */
 #define WOTK_ROUTE_SWEEPS 0    /* two launched sweeps per iteration                          */
 #define WOTK_ROUTE_ONE_READ 1  /* the iteration over one read of C                           */
 #define WOTK_ROUTE_RESIDENT 2  /* persistent launches                                        */
@@ -523,6 +523,15 @@ int wotk_probe_stablev2_coords_limits(const double *X, const double *Y, int64_t 
                                       int64_t inner_iter_max, int32_t terms, double *f_out, double *g_out,
                                       double *row_sums, double *median_out, void *workspace,
                                       size_t workspace_bytes, wotk_stats *stats, void *stream, int32_t polls);
+/* wotk_transport_stablev2 by two launched sweeps per iteration, whatever route
+ * pairs of this shape take (no counterpart in the reference): to time and check
+ * the sweeps' tiles (wotk_set_tile).  wotk_solver_route does not tell of it. */
+int wotk_probe_stablev2_sweeps(const float *C, int64_t ldc, const float *CT, int64_t ldct, int64_t I, int64_t J,
+                               const double *G, double lambda1, double lambda2, double epsilon,
+                               int64_t scaling_iter, double tau, double epsilon0, int64_t extra_iter,
+                               int64_t inner_iter_max, double *plan, int64_t ldp, double *row_sums, double *f_out,
+                               double *g_out, void *workspace, size_t workspace_bytes, wotk_stats *stats,
+                               void *stream);
 
 #ifdef __cplusplus
 }

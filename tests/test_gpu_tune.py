@@ -136,3 +136,65 @@ def test_every_shared_variant_repairs_fallback_tiles(tune):
             err = np.linalg.norm(R - Rref) / np.linalg.norm(Rref)
             assert err <= 1e-5, (tile, e, err)
     tune.reset()
+
+
+def _sweeps(cost, G, **kw):
+    """FP64 plan by launched sweeps, whatever route a solve of the pair takes."""
+    import ctypes
+    import torch
+    from wot_amd import _native
+    from wot_amd.ot import device as dev
+    n_i, n_j = cost.shape
+    L = _native.lib()
+    Gd = torch.from_numpy(np.ascontiguousarray(G)).cuda()
+    plan = torch.empty((n_i, n_j), dtype=torch.float64, device='cuda')
+    ws = dev.workspace(torch, L.wotk_solver_workspace_size(n_i, n_j), 'cuda')
+    st = _native.Stats()
+    _native.check(L.wotk_probe_stablev2_sweeps(
+        dev._ptr(cost.C), cost.ldc, dev._ptr(cost.CT), cost.ldct, n_i, n_j, dev._ptr(Gd), 1.0, 50.0, 0.05,
+        kw['scaling_iter'], kw['tau'], 1.0, kw['extra_iter'], kw['inner_iter_max'], dev._ptr(plan), n_j, None, None,
+        None, dev._ptr(ws), ws.numel(), ctypes.byref(st), dev._stream(torch)))
+    assert st.sweeps == 2 * (kw['scaling_iter'] + kw['extra_iter']) and st.sweep_ms > 0
+    return plan.cpu().numpy()
+
+
+# a pair that a solve takes in persistent launches (the bounds of the test of every variant above)
+def test_every_launched_sweep_variant_matches_oracle(tune):
+    import wot_amd.ot as ot
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(333, 517, dim=12, n_components=4, seed=21)
+    C = O.default_cost_matrix(dp.x, dp.y)
+    Rref = O.transport_stablev2(C, 1.0, 50.0, 0.05, G=dp.growth, epsilon0=1.0, **SCHED)
+    cost = ot.DeviceCost.from_coordinates(dp.x, dp.y)
+    base = None
+    for tile in tune.variants(tune.ROW_SWEEP):
+        tune.set_tile(tune.ROW_SWEEP, -1, tile)
+        R = _sweeps(cost, dp.growth, **SCHED)
+        base = R if base is None else base
+        err = np.linalg.norm(R - Rref) / np.linalg.norm(Rref)
+        assert err <= 1e-5 and np.linalg.norm(R - base) / np.linalg.norm(base) <= 1e-6, (tile, err)
+    tune.reset()
+
+
+# one pair of each route that a solve takes: persistent launches, one read per iteration, sweeps
+@pytest.mark.parametrize('n_i,n_j', [(300, 400), (2900, 2900), (40, 9000)])
+def test_trials_are_launched_sweeps(tune, monkeypatch, n_i, n_j):
+    import wot_amd.ot as ot
+    from wot_amd import _native
+    from wot_amd.synthetic import day_pair
+    dp = day_pair(n_i, n_j, dim=10, n_components=4, seed=3)
+    cost = ot.DeviceCost.from_coordinates(dp.x, dp.y)
+    real, calls = _native.lib(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(real, name)
+
+    monkeypatch.setattr(_native, 'lib', lambda: Spy())
+    r = tune.autotune_row_sweep(cost, iters=20, repeats=1)
+    monkeypatch.undo()
+    tune.reset()
+    assert all(v > 0 for v in r.timings.values())
+    assert calls.count('wotk_probe_stablev2_sweeps') == 2 * len(r.timings)
+    assert 'wotk_transport_stablev2' not in calls

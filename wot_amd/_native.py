@@ -142,7 +142,8 @@ SIGNATURES = {
     'wotk_set_tile': (ctypes.c_int, [_I32, _I32, ctypes.POINTER(Tile)]),
     'wotk_get_tile': (ctypes.c_int, [_I32, _I32, ctypes.POINTER(Tile)]),
 }
-for _probe, _of, _limits in (('wotk_probe_stablev2_limits', 'wotk_transport_stablev2', [_I32, _I64]),
+for _probe, _of, _limits in (('wotk_probe_stablev2_sweeps', 'wotk_transport_stablev2', []),
+                             ('wotk_probe_stablev2_limits', 'wotk_transport_stablev2', [_I32, _I64]),
                              ('wotk_probe_duality_gap_limits', 'wotk_transport_duality_gap', [_I32, _I64]),
                              ('wotk_probe_stablev2_coords_limits', 'wotk_transport_stablev2_coords', [_I32])):
     SIGNATURES[_probe] = (ctypes.c_int, SIGNATURES[_of][1] + _limits)

@@ -1073,11 +1073,11 @@ static int stablev2_call(const float *C, int64_t ldc, const float *CT, int64_t l
                          const double *G, double lambda1, double lambda2, double epsilon, int64_t scaling_iter,
                          double epsilon0, int64_t extra_iter, int64_t inner_iter_max, double *plan, int64_t ldp,
                          double *row_sums, double *f_out, double *g_out, void *workspace, size_t workspace_bytes,
-                         const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
+                         Buffers buffers, const ResidentLimits &lim, wotk_stats *stats, hipStream_t s) {
     const UnderWay here;
     Problem pb;
     Work w;
-    int rc = setup(C, ldc, CT, ldct, I, J, G, Buffers::kRoutes, workspace, workspace_bytes, &pb, &w, s);
+    int rc = setup(C, ldc, CT, ldct, I, J, G, buffers, workspace, workspace_bytes, &pb, &w, s);
     if (rc) return rc;
     rc = resident_or_not(pb, w, here, scaling_iter + extra_iter, s);
     if (rc) return rc;
@@ -1096,7 +1096,7 @@ extern "C" int wotk_transport_stablev2(const float *C, int64_t ldc, const float 
     (void)tau;  // absorption is exact in the log domain; tau only changes the FP64 reference's rounding
     return stablev2_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
                          inner_iter_max, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
-                         ResidentLimits{}, stats, (hipStream_t)stream);
+                         Buffers::kRoutes, ResidentLimits{}, stats, (hipStream_t)stream);
 }
 
 // limits of a probe: waits that end at their first look, launches of so many iterations (0: as ever)
@@ -1122,7 +1122,21 @@ extern "C" int wotk_probe_stablev2_limits(const float *C, int64_t ldc, const flo
     (void)tau;
     return stablev2_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
                          inner_iter_max, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
-                         probe_limits(give_up, launch_iters), stats, (hipStream_t)stream);
+                         Buffers::kRoutes, probe_limits(give_up, launch_iters), stats, (hipStream_t)stream);
+}
+
+extern "C" int wotk_probe_stablev2_sweeps(const float *C, int64_t ldc, const float *CT, int64_t ldct,
+                                          int64_t I, int64_t J, const double *G, double lambda1,
+                                          double lambda2, double epsilon, int64_t scaling_iter,
+                                          double tau, double epsilon0, int64_t extra_iter,
+                                          int64_t inner_iter_max, double *plan, int64_t ldp,
+                                          double *row_sums, double *f_out, double *g_out,
+                                          void *workspace, size_t workspace_bytes, wotk_stats *stats,
+                                          void *stream) {
+    (void)tau;
+    return stablev2_call(C, ldc, CT, ldct, I, J, G, lambda1, lambda2, epsilon, scaling_iter, epsilon0, extra_iter,
+                         inner_iter_max, plan, ldp, row_sums, f_out, g_out, workspace, workspace_bytes,
+                         Buffers::kSweeps, ResidentLimits{}, stats, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------

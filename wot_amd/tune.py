@@ -9,7 +9,7 @@ device-side sweep timer (hipEvents around the sweep loop), stores the fastest
 in the library and persists it per device and bucket in a JSON file, which
 later processes load before their first solve.
 
-    tune.autotune_row_sweep(cost)          # one stored-cost day pair
+    tune.autotune_row_sweep(cost)          # launched sweeps of a stored-cost day pair
     tune.autotune_time_course(tc, eps, l1) # the batched time course
 
 The cache file is ``$WOTK_TILE_CACHE`` (default ``~/.cache/wot_amd/tiles.json``);
@@ -171,26 +171,37 @@ def _pick(kernel, buckets, measure, repeats, persist):
     return TuneResult(kernel, buckets, best, timings)
 
 
-def autotune_row_sweep(cost, G=None, epsilon=0.05, lambda1=1.0, lambda2=50.0, iters=20, repeats=3, persist=True):
-    """Tune the stored-cost sweep on ``cost`` (an ``ot.device.DeviceCost``):
-    each variant runs ``iters`` fixed-epsilon Sinkhorn iterations (2 sweeps
-    each) and is timed by the library's sweep timer.  Both sweep shapes of the
-    pair (C and C^T) get the winning tile."""
+def row_sweep_us(cost, G=None, epsilon=0.05, lambda1=1.0, lambda2=50.0, epsilon0=None, iters=20):
+    """Time of one launched sweep over ``cost`` (an ``ot.device.DeviceCost``) with
+    the tiles as they are set, from ``iters`` iterations of two sweeps each.  A
+    solve itself may take a route without such sweeps (``wotk_solver_route``)."""
     import torch
     from .ot import device as dev
+    apply_persisted()
     n_i, n_j = cost.shape
-    if G is None:
-        G = torch.ones(n_i, dtype=torch.float64, device=cost.device)
-    params = dict(lambda1=lambda1, lambda2=lambda2, epsilon=epsilon, scaling_iter=int(iters), tau=1e4,
-                  epsilon0=epsilon, extra_iter=0, inner_iter_max=int(iters))
+    G = torch.ones(n_i, dtype=torch.float64, device=cost.device) if G is None else dev.as_device_f64(
+        torch, G, cost.device).view(-1)
+    if G.numel() != n_i:
+        raise ValueError('G has %d entries for %d source cells' % (G.numel(), n_i))
+    L = _native.lib()
+    ws = dev.workspace(torch, L.wotk_solver_workspace_size(n_i, n_j), cost.device)
+    st = _native.Stats()
+    _native.check(L.wotk_probe_stablev2_sweeps(
+        dev._ptr(cost.C), cost.ldc, dev._ptr(cost.CT), cost.ldct, n_i, n_j, dev._ptr(G), float(lambda1),
+        float(lambda2), float(epsilon), int(iters), 1e4, float(epsilon if epsilon0 is None else epsilon0), 0,
+        int(iters), None, n_j, None, None, None, dev._ptr(ws), ws.numel(), ctypes.byref(st), dev._stream(torch)))
+    return 1e3 * st.sweep_ms / max(1, st.sweeps)
+
+
+def autotune_row_sweep(cost, G=None, epsilon=0.05, lambda1=1.0, lambda2=50.0, iters=20, repeats=3, persist=True):
+    """Tune the launched sweeps of a stored cost on ``cost`` (an
+    ``ot.device.DeviceCost``): each variant runs ``iters`` fixed-epsilon Sinkhorn
+    iterations (2 sweeps each) and is timed by the library's sweep timer.  Both
+    sweep shapes of the pair (C and C^T) get the winning tile."""
+    n_i, n_j = cost.shape
     buckets = sorted({bucket(ROW_SWEEP, n_i, n_j), bucket(ROW_SWEEP, n_j, n_i)})
-
-    def measure():
-        out = dev.solve(cost, G, 'fixed_iters', params, want_plan=False)
-        st = out['stats']
-        return 1e3 * st['sweep_ms'] / max(1, st['sweeps'])
-
-    return _pick(ROW_SWEEP, buckets, measure, repeats, persist)
+    return _pick(ROW_SWEEP, buckets, lambda: row_sweep_us(cost, G, epsilon, lambda1, lambda2, iters=iters), repeats,
+                 persist)
 
 
 def autotune_time_course(tc, epsilons, lambda1s, lambda2=50.0, iters=20, repeats=2, share_exp=True, persist=True):
