@@ -33,7 +33,7 @@ SOLVER = dict(epsilon=0.05, lambda1=1.0, lambda2=50.0, epsilon0=1.0, tau=1e4, sc
               inner_iter_max=50, extra_iter=1000, growth_iters=3)
 
 
-def _traffic(name='lse_rows_kernel_15000x15000'):
+def _traffic(name):
     """HBM bytes per launch of a kernel from the calibrated PMC runs kept in profiles/."""
     path = os.path.join(ROOT, 'profiles', name + '.traffic.json')
     try:
@@ -419,12 +419,19 @@ def _secondary_pair(torch):
     want = q * CFG['n_source'] * torch.exp(-res['g'] / SOLVER['lambda2'])
     colsum = res['plan'].sum(0) * CFG['n_target']
     marg = float((colsum - want).abs().max() / want.abs().max())
-    avg = sweep_ms / 1000.0 / sweeps
-    alg = 4.0 * CFG['n_source'] * CFG['n_target']
     return {'workload': 'one day pair 15000x15000, d=30, fixed_iters, growth_iters=3, 6-term split-BF16 cost',
             'maps_per_s': 1.0 / el, 'ms_per_map': 1000.0 * el, 'marginal_identity_rel_err': marg,
-            'roofline': {'bound': 'hbm', 'kernel': 'lse_rows_kernel', 'avg_launch_us': avg * 1e6,
-                         'achieved': alg / avg / 1e9, 'peak': HBM_PEAK_GBS, 'frac': alg / avg / 1e9 / HBM_PEAK_GBS}}
+            'roofline': pair_roofline(sweep_ms, sweeps)}
+
+
+def pair_roofline(sweep_ms, sweeps):
+    """Roofline of the stored pair's iteration (two half sweeps in the solver's count): pairs of this size
+    read C once per iteration, 4 * I * J bytes in a row launch and the column launch behind it."""
+    iter_s = 2.0 * sweep_ms / 1000.0 / max(sweeps, 1)
+    alg = 4.0 * CFG['n_source'] * CFG['n_target']
+    return {'bound': 'hbm', 'kernel': 'one_pass_rows_kernel + one_pass_cols_kernel', 'avg_launch_us': iter_s * 1e6,
+            'achieved': alg / iter_s / 1e9, 'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
+            'frac': alg / iter_s / 1e9 / HBM_PEAK_GBS, 'alg_bytes_per_launch': alg}
 
 
 def _parse_tile(text):
@@ -1348,12 +1355,7 @@ def main():
     maps_per_s = args.steps / elapsed
     iters_per_map = SOLVER['growth_iters'] * (SOLVER['scaling_iter'] + SOLVER['extra_iter'])
 
-    # roofline of the dominant kernel (row LSE sweep): algorithmic bytes per
-    # launch = 4 * I * J (one FP32 cost row stream), launches alternate C / C^T
     n_i, n_j = CFG['n_source'], CFG['n_target']
-    avg_sweep_s = (sweep_ms / 1000.0) / max(sweeps, 1)
-    alg_bytes = 4.0 * n_i * n_j
-    achieved = alg_bytes / avg_sweep_s / 1e9
 
     # size-independent property at full size: column sums of the un-normalised
     # plan equal q * I * exp(-g / lambda2) after the last (b-update) half iteration
@@ -1380,10 +1382,7 @@ def main():
                    'tiles': tiles},
         'sinkhorn_iters_per_s': maps_per_s * iters_per_map,
         'marginal_identity_rel_err': marg_err,
-        'roofline': {'bound': 'hbm', 'achieved': achieved, 'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
-                     'frac': achieved / HBM_PEAK_GBS, 'traffic': _traffic(),
-                     'kernel': 'lse_rows_kernel', 'avg_launch_us': avg_sweep_s * 1e6,
-                     'alg_bytes_per_launch': alg_bytes},
+        'roofline': dict(pair_roofline(sweep_ms, sweeps), traffic=None),
     }
     del colsum, want, res
     if not args.no_baselines:
